@@ -96,6 +96,13 @@ namespace {
 #define WR_W2DN 1
 #endif
 
+// Geom of the batched kernels: hp and Ip are the row lengths of the workspace's
+// x terms, partial sums (hp) and act (Ip).  Aligned layers have hp = h, Ip = I;
+// ragged ones (k_rag_gu) round both up to whole K steps.
+struct GeomB : Geom {
+  int hp, Ip;
+};
+
 constexpr int kBlk = 256;       // 4 waves
 constexpr int kBK = 128;        // the base K step (columns); every step width is a multiple
 constexpr int kBM = 64;         // rows per block: 4 waves x 16
@@ -383,13 +390,21 @@ constexpr int kc_wide() {
   return std::is_same<WT, fp4x2>::value ? 256 : 256 * 8 / wbits<WT>();
 }
 
+// Third terms of a token tile (ragged layers only; rows as TokTile's).
+template <int TOK, int PIECES, bool L2>
+struct TokTileL2 {
+  H8 l2[TOK][PIECES];
+};
+template <int TOK, int PIECES>
+struct TokTileL2<TOK, PIECES, false> {};
+
 // Token tiles in LDS: hi holds the hi terms, lo the lo terms; row n is token
 // n of the pass, piece c covers columns [8 c, 8 c + 8) of the K step.  TOK
 // tokens per pass (16, 32 or 64): a launch whose experts have at most 16 (32)
 // tokens each takes the smaller tile, whose LDS and registers leave room for
 // more blocks per CU.
-template <int TOK, int KC>
-struct TokTile {
+template <int TOK, int KC, bool L2 = false>
+struct TokTile : TokTileL2<TOK, KC / 8 + (TOK == 64 ? 0 : 2), L2> {
   static constexpr int kP = KC / 8;  // 16-byte pieces per token row
   // The MFMA B-fragment reads (ds_read_b128, lane l at row l % 16, piece
   // 4 j + l / 16) are free of bank conflicts with rows padded by two pieces,
@@ -446,6 +461,16 @@ __device__ __forceinline__ void gu_tile_load(H8 (&hi)[TP], H8 (&lo)[TP],
       hi[q] = *reinterpret_cast<const H8*>(x_hi + off[q] + kb);
       if (with_lo) lo[q] = *reinterpret_cast<const H8*>(x_lo + off[q] + kb);
     }
+  }
+}
+// One term alone (the third terms of ragged layers).
+template <int TP>
+__device__ __forceinline__ void gu_term_load(H8 (&t)[TP], const f16* __restrict__ x,
+                                             const int64_t (&off)[TP], int kb) {
+#pragma unroll
+  for (int q = 0; q < TP; ++q) {
+    t[q] = h8zero();
+    if (off[q] >= 0) t[q] = *reinterpret_cast<const H8*>(x + off[q] + kb);
   }
 }
 
@@ -515,8 +540,8 @@ __device__ __forceinline__ void dn_tile_load_split(H8 (&hi)[TP], H8 (&lo)[TP],
   }
 }
 
-template <int TOK, int KC, int TP>
-__device__ __forceinline__ void tile_store(TokTile<TOK, KC>& xs, const H8 (&hi)[TP],
+template <int TOK, int KC, bool L2, int TP>
+__device__ __forceinline__ void tile_store(TokTile<TOK, KC, L2>& xs, const H8 (&hi)[TP],
                                            const H8 (&lo)[TP], bool with_lo) {
   static_assert(TP == tile_pieces<TOK, KC>(), "tile shares");
 #pragma unroll
@@ -526,6 +551,37 @@ __device__ __forceinline__ void tile_store(TokTile<TOK, KC>& xs, const H8 (&hi)[
     xs.hi[n][tslot<TOK, KC>(n, c)] = hi[q];
     if (with_lo) xs.lo[n][tslot<TOK, KC>(n, c)] = lo[q];
   }
+}
+template <int TOK, int KC, int TP>
+__device__ __forceinline__ void tile_store_l2(TokTile<TOK, KC, true>& xs, const H8 (&l2)[TP]) {
+#pragma unroll
+  for (int q = 0; q < TP; ++q) {
+    const int i = threadIdx.x + kBlk * q;
+    const int n = i / (KC / 8), c = i % (KC / 8);
+    xs.l2[n][tslot<TOK, KC>(n, c)] = l2[q];
+  }
+}
+// The third terms of a raw act piece: what hi and lo (dn_tile_split) leave of
+// it, in their type.  Both subtractions are exact.
+template <bool BF, int TP>
+__device__ __forceinline__ void dn_tile_split_l2(H8 (&l2)[TP], const ActRaw<TP>& t,
+                                                 const int (&sx)[TP]) {
+#pragma unroll
+  for (int q = 0; q < TP; ++q)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const float r = t.v[q][i / 4][i % 4];
+      float v = BF ? r : ldexpf(r, sx[q]);
+      if constexpr (BF) {
+        v -= (float)(__bf16)v;
+        v -= (float)(__bf16)v;
+        l2[q][i] = __builtin_bit_cast(f16, (__bf16)v);
+      } else {
+        v -= (float)(f16)v;
+        v -= (float)(f16)v;
+        l2[q][i] = (f16)v;
+      }
+    }
 }
 
 // Weight tiles.  A wave's rows are loaded 16 bytes per lane, KC columns of a
@@ -610,6 +666,49 @@ __device__ __forceinline__ void w_load(WRegs<WT, ROWS, KC>& r,
   }
 }
 
+// Ragged rows (K = the row length, any number from one piece up; rows start at
+// any address).  Lane l's piece of the step at kb starts at column
+// c = kb + E (l % LR).  It is loaded as 16 bytes at column min(c, K - E) of its
+// row, at whatever alignment that is (global loads take any on this target), so
+// every load is in bounds and unconditional; the step that holds the row's end
+// then shifts the piece's own columns down and zeroes those past K (w_rag_fix).
+// Bases are row starts here, without the lane's piece.
+template <typename WT, int KC>
+__device__ __forceinline__ int rag_piece_col(int lane, int kb) {
+  typedef WGeo<WT, KC> G;
+  return kb + (lane % G::kLaneRow) * G::kElems;
+}
+template <typename WT, int ROWS, int KC>
+__device__ __forceinline__ void w_load_rag(WRegs<WT, ROWS, KC>& r,
+                                           const WT* const (&base)[WRegs<WT, ROWS, KC>::N],
+                                           const uint8_t* const (&sc)[WRegs<WT, ROWS, KC>::N],
+                                           int kb, int K, int lane) {
+  const int c = min(rag_piece_col<WT, KC>(lane, kb), K - WGeo<WT, KC>::kElems);
+#pragma unroll
+  for (int i = 0; i < WRegs<WT, ROWS, KC>::N; ++i) {
+    r.v[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4u*>(base[i] + eoff<WT>(c)));
+    if constexpr (std::is_same<WT, fp4x2>::value) r.e[i] = sc[i][c / 32];
+  }
+}
+template <typename WT, int ROWS, int KC>
+__device__ __forceinline__ void w_rag_fix(WRegs<WT, ROWS, KC>& r, int kb, int K, int lane) {
+  if (kb + KC <= K) return;  // uniform
+  constexpr int E = WGeo<WT, KC>::kElems;
+  const int d = rag_piece_col<WT, KC>(lane, kb) - (K - E);  // columns loaded ahead of the piece's own
+#pragma unroll
+  for (int i = 0; i < WRegs<WT, ROWS, KC>::N; ++i) {
+    if (d > 0) {
+      if constexpr (std::is_same<WT, fp4x2>::value) {  // rows are whole pieces
+        r.v[i] = u32x4{0u, 0u, 0u, 0u};
+        r.e[i] = 127;
+      } else {
+        const unsigned __int128 v = __builtin_bit_cast(unsigned __int128, r.v[i]);
+        r.v[i] = d < E ? __builtin_bit_cast(u32x4, v >> (d * wbits<WT>())) : u32x4{0u, 0u, 0u, 0u};
+      }
+    }
+  }
+}
+
 __device__ __forceinline__ H8 fp8x8_to_h8(uint32_t a, uint32_t b) {
   typedef f16 h2 __attribute__((ext_vector_type(2)));
   const h2 p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(a, 1.0f, false);
@@ -680,28 +779,53 @@ struct GuScale {
   unsigned* s_amax;
 };
 
+// Ragged layers sum each K step apart and add it to a running sum, whose
+// length the step count then sets, instead of one chain through all MFMAs:
+// their error stays that of the per-token kernels' 64 lane sums (one chain,
+// h = 1500: 2.0 times it).
+template <int NT>
+__device__ __forceinline__ void ksum_open(f32x4 (&t)[NT], f32x4 (&a)[NT]) {
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    t[n] = a[n];
+    a[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  }
+}
+template <int NT>
+__device__ __forceinline__ void ksum_close(const f32x4 (&t)[NT], f32x4 (&a)[NT]) {
+#pragma unroll
+  for (int n = 0; n < NT; ++n) a[n] = t[n] + a[n];
+}
+
 // WK: the weight K step, KC (the token step) or a multiple of it: each weight
 // tile then serves WK / KC token steps (MXFP4 64-token tiles: 8 rows x 128
 // bytes per weight load instruction, with the 128-column token tile).
-template <typename WT, bool LO, int NT, int TOK, int KC, int WK = KC>
-__device__ __forceinline__ void gu_pass(TokTile<TOK, KC>& xs, WTile<WT, 32, WK>& wt,
+//
+// RAG (ragged layers): ragged weight rows; x and act rows of g.hp and g.Ip
+// columns, zero past h and I.  L2: x in three terms (fp32 x of ragged layers).
+template <typename WT, bool LO, int NT, int TOK, int KC, int WK = KC, bool RAG = false,
+          bool L2 = false>
+__device__ __forceinline__ void gu_pass(TokTile<TOK, KC, L2>& xs,
+                                        WTile<WT, 32, WK>& wt,
                                         const WT* const (&wbase)[WRegs<WT, 32, WK>::N],
                                         const uint8_t* const (&wsc)[WRegs<WT, 32, WK>::N],
                                         const f16* __restrict__ x_hi,
-                                        const f16* __restrict__ x_lo, const BatchRoute& r,
+                                        const f16* __restrict__ x_lo,
+                                        const f16* __restrict__ x_l2, const BatchRoute& r,
                                         int p0, int mt, float* __restrict__ act, int row0,
                                         const float* __restrict__ sc, const GuScale& xsc,
-                                        const Geom& g, int lane) {
+                                        const GeomB& g, int lane) {
   static_assert(WK % KC == 0 && (WK == KC || std::is_same<WT, fp4x2>::value),
                 "a weight step of whole token steps (MXFP4 only)");
+  static_assert(!RAG || WK == KC, "ragged rows take plain steps");
   constexpr int R = WK / KC;  // token steps per weight step; h % WK == 0
   f32x4 ag[NT], au[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) ag[n] = au[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   constexpr int TP = tile_pieces<TOK, KC>();
   int64_t off[TP];
-  tile_rows<KC>(off, r.pair_tok + p0, 0, mt, g.h);
-  const int ns = g.h / KC;
+  tile_rows<KC>(off, r.pair_tok + p0, 0, mt, RAG ? g.hp : g.h);
+  const int ns = (RAG ? g.hp : g.h) / KC;
   // fp16 operands: the epilogue tokens' x exponents, loaded here so that the
   // loads are in flight with the first K step's.
   constexpr bool SC = !bf16_ops<WT>();
@@ -716,21 +840,31 @@ __device__ __forceinline__ void gu_pass(TokTile<TOK, KC>& xs, WTile<WT, 32, WK>&
   // first token step of a weight step the next weight step's loads, are
   // issued before step s's MFMAs.
   WRegs<WT, 32, WK> wr;
-  H8 th[TP], tl[TP];
-  w_load<WT, 32, WK>(wr, wbase, wsc, 0);
+  H8 th[TP], tl[TP], t2[L2 ? TP : 1];
+  if constexpr (RAG)
+    w_load_rag<WT, 32, WK>(wr, wbase, wsc, 0, g.h, lane);
+  else
+    w_load<WT, 32, WK>(wr, wbase, wsc, 0);
   gu_tile_load(th, tl, x_hi, x_lo, off, 0, LO);
+  if constexpr (L2) gu_term_load(t2, x_l2, off, 0);
   for (int s0 = 0; s0 < ns; s0 += R) {
 #pragma unroll
     for (int hs = 0; hs < R; ++hs) {
       const int s = s0 + hs;
       __syncthreads();  // every wave is done reading the previous tiles
       tile_store(xs, th, tl, LO);
+      if constexpr (L2) tile_store_l2<TOK, KC>(xs, t2);
+      if constexpr (RAG) w_rag_fix<WT, 32, WK>(wr, s * KC, g.h, lane);
       if (hs == 0) w_store<WT, 32, WK>(wt, wr, lane);
       __syncthreads();
       if constexpr (R == 1) {
         if (s + 1 < ns) {
-          w_load<WT, 32, WK>(wr, wbase, wsc, (s + 1) * KC);
+          if constexpr (RAG)
+            w_load_rag<WT, 32, WK>(wr, wbase, wsc, (s + 1) * KC, g.h, lane);
+          else
+            w_load<WT, 32, WK>(wr, wbase, wsc, (s + 1) * KC);
           gu_tile_load(th, tl, x_hi, x_lo, off, (s + 1) * KC, LO);
+          if constexpr (L2) gu_term_load(t2, x_l2, off, (s + 1) * KC);
         }
       } else {
         // The next token step's loads first: the load counter is in order,
@@ -742,6 +876,11 @@ __device__ __forceinline__ void gu_pass(TokTile<TOK, KC>& xs, WTile<WT, 32, WK>&
       // scheduler sank them below the MFMAs at 32 and 64 tokens, so each
       // step's loads were awaited with no MFMA work in flight).
       if constexpr (std::is_same<WT, fp4x2>::value) __builtin_amdgcn_sched_barrier(0);
+      f32x4 tg[RAG ? NT : 1], tu[RAG ? NT : 1];  // RAG: the step's own sums (ksum_open)
+      if constexpr (RAG) {
+        ksum_open(tg, ag);
+        ksum_open(tu, au);
+      }
 #pragma unroll
       for (int j = 0; j < KC / 32; ++j) {
         const int c = 4 * j + (lane >> 4);
@@ -760,7 +899,16 @@ __device__ __forceinline__ void gu_pass(TokTile<TOK, KC>& xs, WTile<WT, 32, WK>&
             ag[n] = mfma<BF>(ga, bl, ag[n]);
             au[n] = mfma<BF>(ua, bl, au[n]);
           }
+          if constexpr (L2) {
+            const H8 b2 = xs.l2[tn][tslot<TOK, KC>(tn, c)];
+            ag[n] = mfma<BF>(ga, b2, ag[n]);
+            au[n] = mfma<BF>(ua, b2, au[n]);
+          }
         }
+      }
+      if constexpr (RAG) {
+        ksum_close(tg, ag);
+        ksum_close(tu, au);
       }
     }
   }
@@ -771,7 +919,14 @@ __device__ __forceinline__ void gu_pass(TokTile<TOK, KC>& xs, WTile<WT, 32, WK>&
   // exactly (a power of two).
   const int rq = row0 + (lane >> 4) * 4;
   f32x4 sg, su;
-  if constexpr (std::is_same<WT, fp8w>::value) {
+  if constexpr (std::is_same<WT, fp8w>::value && RAG) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int row = min(rq + i, g.I - 1);
+      sg[i] = sc[row];
+      su[i] = sc[g.I + row];
+    }
+  } else if constexpr (std::is_same<WT, fp8w>::value) {
     sg = *reinterpret_cast<const f32x4*>(sc + rq);
     su = *reinterpret_cast<const f32x4*>(sc + g.I + rq);
   }
@@ -791,9 +946,10 @@ __device__ __forceinline__ void gu_pass(TokTile<TOK, KC>& xs, WTile<WT, 32, WK>&
           v[i] = w * (silu(gs * sg[i]) * (us * su[i]));
         else
           v[i] = w * (silu(gs) * us);
+        if (RAG && rq + i >= g.I) v[i] = 0.0f;  // a clamped row
         m = fmaxf(m, fabsf(v[i]));
       }
-      *reinterpret_cast<f32x4*>(act + (int64_t)p * g.I + rq) = v;
+      *reinterpret_cast<f32x4*>(act + (int64_t)p * (RAG ? g.Ip : g.I) + rq) = v;
     }
     if constexpr (SC) {
       // max over the 16 rows of this wave's tile (lanes l, l^16, l^32, l^48
@@ -844,17 +1000,18 @@ constexpr int gu_min_blocks() {
 
 // ROUTE: the block routes the batch itself (route_small) instead of reading
 // k_route's output; block (0, 0) publishes the routing for the later kernels.
-template <typename WT, bool LO, int TOK, bool ROUTE, int KC, int WK = KC>
-__global__ __launch_bounds__(kBlk, (gu_min_blocks<WT, LO, TOK, KC, WK>())) void k_gu_mfma(const WT* __restrict__ wbuf,
-                                                  const f16* __restrict__ x_hi,
-                                                  const f16* __restrict__ x_lo,
-                                                  const int32_t* __restrict__ x_exp,
-                                                  unsigned* __restrict__ amax, BatchRoute r,
-                                                  float* __restrict__ act, Geom g,
-                                                  const float* __restrict__ logits,
-                                                  int32_t* __restrict__ ids_out,
-                                                  float* __restrict__ w_out) {
-  __shared__ TokTile<TOK, KC> xs;
+template <typename WT, bool LO, int TOK, bool ROUTE, int KC, int WK, bool RAG, bool L2>
+__device__ __forceinline__ void gu_block(const WT* __restrict__ wbuf,
+                                         const f16* __restrict__ x_hi,
+                                         const f16* __restrict__ x_lo,
+                                         const f16* __restrict__ x_l2,
+                                         const int32_t* __restrict__ x_exp,
+                                         unsigned* __restrict__ amax, BatchRoute r,
+                                         float* __restrict__ act, const GeomB& g,
+                                         const float* __restrict__ logits,
+                                         int32_t* __restrict__ ids_out,
+                                         float* __restrict__ w_out) {
+  __shared__ TokTile<TOK, KC, L2> xs;
   __shared__ WTile<WT, 32, WK> wts[kBlk / kWave];
   __shared__ GuRouteLds<ROUTE> rl;
   __shared__ unsigned s_amax[bf16_ops<WT>() ? 1 : TOK];
@@ -876,7 +1033,7 @@ __global__ __launch_bounds__(kBlk, (gu_min_blocks<WT, LO, TOK, KC, WK>())) void 
     (void)logits;
     (void)ids_out;
     (void)w_out;
-    const int sl = tile_slot<TOK>(r, slot);
+    const int sl = RAG ? (slot < r.n_active[0] ? slot : -1) : tile_slot<TOK>(r, slot);
     if (sl < 0) return;  // block-uniform
     e = r.active[sl];
     pbeg = r.off[e];
@@ -885,6 +1042,12 @@ __global__ __launch_bounds__(kBlk, (gu_min_blocks<WT, LO, TOK, KC, WK>())) void 
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int row0 = blockIdx.x * kBM + wave * 16;
+  if (RAG && (int)blockIdx.x * kBM >= g.I) {  // a block of act's padding columns: zeros
+    for (int i = threadIdx.x; i < M * (kBM / 4); i += kBlk)
+      *reinterpret_cast<f32x4*>(act + (int64_t)(pbeg + i / (kBM / 4)) * g.Ip + blockIdx.x * kBM +
+                                4 * (i % (kBM / 4))) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    return;
+  }
   const WT* blk = wbuf + (int64_t)e * g.stride;
   const WT* G = w_lane_base<WT, WK>(blk, row0, g.h, lane);
   // Tile rows 0-15: gate rows row0 ..; rows 16-31: the same up rows.
@@ -895,6 +1058,12 @@ __global__ __launch_bounds__(kBlk, (gu_min_blocks<WT, LO, TOK, KC, WK>())) void 
   const uint8_t* mxs = reinterpret_cast<const uint8_t*>(blk) + g.off_scale;
 #pragma unroll
   for (int i = 0; i < N; ++i) {
+    if constexpr (RAG) {  // row starts; rows past the last repeat it
+      const int row = min(row0 + lane / WGeo<WT, WK>::kLaneRow + RP * (i % (N / 2)), g.I - 1);
+      wbase[i] = blk + (i < N / 2 ? 0 : g.off_up) + eoff<WT>((int64_t)row * g.h);
+      wsc[i] = mxs + (i < N / 2 ? 0 : (int64_t)g.I * g.h / 32) + (int64_t)row * (g.h / 32);
+      continue;
+    }
     wbase[i] = G + (i < N / 2 ? 0 : g.off_up) + eoff<WT>((int64_t)(RP * (i % (N / 2))) * g.h);
     wsc[i] = w_lane_scale<WT, WK>(mxs + (i < N / 2 ? 0 : (int64_t)g.I * g.h / 32), row0, g.h,
                                   lane) +
@@ -907,21 +1076,43 @@ __global__ __launch_bounds__(kBlk, (gu_min_blocks<WT, LO, TOK, KC, WK>())) void 
     const int mt = min(TOK, M - m0);
     const int p0 = pbeg + m0;
     if constexpr (TOK == 16) {
-      gu_pass<WT, LO, 1, TOK, KC, WK>(xs, wt, wbase, wsc, x_hi, x_lo, r, p0, mt, act, row0, sc, xsc, g, lane);
+      gu_pass<WT, LO, 1, TOK, KC, WK, RAG, L2>(xs, wt, wbase, wsc, x_hi, x_lo, x_l2, r, p0, mt, act, row0, sc, xsc, g, lane);
     } else if constexpr (TOK == 32) {
       if (mt <= 16)
-        gu_pass<WT, LO, 1, TOK, KC, WK>(xs, wt, wbase, wsc, x_hi, x_lo, r, p0, mt, act, row0, sc, xsc, g, lane);
+        gu_pass<WT, LO, 1, TOK, KC, WK, RAG, L2>(xs, wt, wbase, wsc, x_hi, x_lo, x_l2, r, p0, mt, act, row0, sc, xsc, g, lane);
       else
-        gu_pass<WT, LO, 2, TOK, KC, WK>(xs, wt, wbase, wsc, x_hi, x_lo, r, p0, mt, act, row0, sc, xsc, g, lane);
+        gu_pass<WT, LO, 2, TOK, KC, WK, RAG, L2>(xs, wt, wbase, wsc, x_hi, x_lo, x_l2, r, p0, mt, act, row0, sc, xsc, g, lane);
     } else {
       switch ((mt + 15) / 16) {
-        case 1: gu_pass<WT, LO, 1, TOK, KC, WK>(xs, wt, wbase, wsc, x_hi, x_lo, r, p0, mt, act, row0, sc, xsc, g, lane); break;
-        case 2: gu_pass<WT, LO, 2, TOK, KC, WK>(xs, wt, wbase, wsc, x_hi, x_lo, r, p0, mt, act, row0, sc, xsc, g, lane); break;
-        case 3: gu_pass<WT, LO, 3, TOK, KC, WK>(xs, wt, wbase, wsc, x_hi, x_lo, r, p0, mt, act, row0, sc, xsc, g, lane); break;
-        default: gu_pass<WT, LO, 4, TOK, KC, WK>(xs, wt, wbase, wsc, x_hi, x_lo, r, p0, mt, act, row0, sc, xsc, g, lane); break;
+        case 1: gu_pass<WT, LO, 1, TOK, KC, WK, RAG, L2>(xs, wt, wbase, wsc, x_hi, x_lo, x_l2, r, p0, mt, act, row0, sc, xsc, g, lane); break;
+        case 2: gu_pass<WT, LO, 2, TOK, KC, WK, RAG, L2>(xs, wt, wbase, wsc, x_hi, x_lo, x_l2, r, p0, mt, act, row0, sc, xsc, g, lane); break;
+        case 3: gu_pass<WT, LO, 3, TOK, KC, WK, RAG, L2>(xs, wt, wbase, wsc, x_hi, x_lo, x_l2, r, p0, mt, act, row0, sc, xsc, g, lane); break;
+        default: gu_pass<WT, LO, 4, TOK, KC, WK, RAG, L2>(xs, wt, wbase, wsc, x_hi, x_lo, x_l2, r, p0, mt, act, row0, sc, xsc, g, lane); break;
       }
     }
   }
+}
+
+template <typename WT, bool LO, int TOK, bool ROUTE, int KC, int WK = KC>
+__global__ __launch_bounds__(kBlk, (gu_min_blocks<WT, LO, TOK, KC, WK>())) void k_gu_mfma(
+    const WT* __restrict__ wbuf, const f16* __restrict__ x_hi, const f16* __restrict__ x_lo,
+    const int32_t* __restrict__ x_exp, unsigned* __restrict__ amax, BatchRoute r,
+    float* __restrict__ act, GeomB g, const float* __restrict__ logits,
+    int32_t* __restrict__ ids_out, float* __restrict__ w_out) {
+  gu_block<WT, LO, TOK, ROUTE, KC, WK, false, false>(wbuf, x_hi, x_lo, nullptr, x_exp, amax, r,
+                                                     act, g, logits, ids_out, w_out);
+}
+
+// Ragged layers: any h and I of at least one 16-byte piece of weights, any
+// alignment of the pointers.
+template <typename WT, bool LO, bool L2, int TOK, bool ROUTE>
+__global__ __launch_bounds__(kBlk) void k_rag_gu(
+    const WT* __restrict__ wbuf, const f16* __restrict__ x_hi, const f16* __restrict__ x_lo,
+    const f16* __restrict__ x_l2, const int32_t* __restrict__ x_exp, unsigned* __restrict__ amax,
+    BatchRoute r, float* __restrict__ act, GeomB g, const float* __restrict__ logits,
+    int32_t* __restrict__ ids_out, float* __restrict__ w_out) {
+  gu_block<WT, LO, TOK, ROUTE, kBK, kBK, true, L2>(wbuf, x_hi, x_lo, x_l2, x_exp, amax, r, act, g,
+                                                   logits, ids_out, w_out);
 }
 
 // ---------------------------------------------------------------------------
@@ -943,17 +1134,20 @@ __device__ __forceinline__ int pair_exp(const unsigned* __restrict__ amax, int p
 
 // WK as in gu_pass: a weight step of WK / KC token steps (MXFP4 64-token
 // tiles, act split ahead); sb and se are then multiples of WK / KC.
-template <typename WT, int NT, int TOK, int KC, bool PRE, int WK = KC>
-__device__ __forceinline__ void dn_pass(TokTile<TOK, KC>& xs, WTile<WT, 16, WK>& wt,
+// RAG as in gu_pass (act split here, in three terms).
+template <typename WT, int NT, int TOK, int KC, bool PRE, int WK = KC, bool RAG = false>
+__device__ __forceinline__ void dn_pass(TokTile<TOK, KC, RAG>& xs,
+                                        WTile<WT, 16, WK>& wt,
                                         const WT* const (&wbase)[WRegs<WT, 16, WK>::N],
                                         const uint8_t* const (&wsc)[WRegs<WT, 16, WK>::N],
                                         const float* __restrict__ act,
                                         const unsigned* __restrict__ amax, int p0, int mt,
                                         int sb, int se, float* __restrict__ y, int row0,
-                                        const float* __restrict__ sdown, const Geom& g,
+                                        const float* __restrict__ sdown, const GeomB& g,
                                         int lane) {
   static_assert(WK % KC == 0 && (WK == KC || (std::is_same<WT, fp4x2>::value && PRE)),
                 "a weight step of whole token steps (MXFP4, act split ahead)");
+  static_assert(!RAG || (WK == KC && !PRE), "ragged rows take plain steps");
   constexpr int R = WK / KC;
   f32x4 acc[NT];
 #pragma unroll
@@ -968,7 +1162,7 @@ __device__ __forceinline__ void dn_pass(TokTile<TOK, KC>& xs, WTile<WT, 16, WK>&
   if (sb < se) {
     constexpr int TP = tile_pieces<TOK, KC>();
     int64_t off[TP];
-    tile_rows<KC>(off, nullptr, p0, mt, g.I);
+    tile_rows<KC>(off, nullptr, p0, mt, RAG ? g.Ip : g.I);
     int sx[TP];  // each staged piece's pair exponent (act split here)
 #pragma unroll
     for (int q = 0; q < TP; ++q) {
@@ -978,7 +1172,10 @@ __device__ __forceinline__ void dn_pass(TokTile<TOK, KC>& xs, WTile<WT, 16, WK>&
     WRegs<WT, 16, WK> wr;
     ActRaw<PRE ? 1 : TP> ar;  // act split here: raw pieces
     H8 ph[TP], pl[TP];        // act split ahead: the two terms
-    w_load<WT, 16, WK>(wr, wbase, wsc, sb * KC);
+    if constexpr (RAG)
+      w_load_rag<WT, 16, WK>(wr, wbase, wsc, sb * KC, g.I, lane);
+    else
+      w_load<WT, 16, WK>(wr, wbase, wsc, sb * KC);
     if constexpr (PRE)
       dn_tile_load_split(ph, pl, act, off, sb * KC);
     else
@@ -994,12 +1191,21 @@ __device__ __forceinline__ void dn_pass(TokTile<TOK, KC>& xs, WTile<WT, 16, WK>&
           H8 th[TP], tl[TP];
           dn_tile_split<bf16_ops<WT>()>(th, tl, ar, sx);
           tile_store(xs, th, tl, true);
+          if constexpr (RAG) {
+            H8 t2[TP];
+            dn_tile_split_l2<bf16_ops<WT>()>(t2, ar, sx);
+            tile_store_l2<TOK, KC>(xs, t2);
+          }
         }
+        if constexpr (RAG) w_rag_fix<WT, 16, WK>(wr, s * KC, g.I, lane);
         if (hs == 0) w_store<WT, 16, WK>(wt, wr, lane);
         __syncthreads();
         if constexpr (R == 1) {
           if (s + 1 < se) {
-            w_load<WT, 16, WK>(wr, wbase, wsc, (s + 1) * KC);
+            if constexpr (RAG)
+              w_load_rag<WT, 16, WK>(wr, wbase, wsc, (s + 1) * KC, g.I, lane);
+            else
+              w_load<WT, 16, WK>(wr, wbase, wsc, (s + 1) * KC);
             if constexpr (PRE)
               dn_tile_load_split(ph, pl, act, off, (s + 1) * KC);
             else
@@ -1013,6 +1219,8 @@ __device__ __forceinline__ void dn_pass(TokTile<TOK, KC>& xs, WTile<WT, 16, WK>&
         }
         if constexpr (std::is_same<WT, fp4x2>::value)
           __builtin_amdgcn_sched_barrier(0);  // loads ahead of the MFMAs, as in gu_pass
+        f32x4 ta[RAG ? NT : 1];
+        if constexpr (RAG) ksum_open(ta, acc);
 #pragma unroll
         for (int j = 0; j < KC / 32; ++j) {
           const int c = 4 * j + (lane >> 4);
@@ -1022,8 +1230,11 @@ __device__ __forceinline__ void dn_pass(TokTile<TOK, KC>& xs, WTile<WT, 16, WK>&
             const int tn = n * 16 + (lane & 15);
             acc[n] = mfma<bf16_ops<WT>()>(da, xs.hi[tn][tslot<TOK, KC>(tn, c)], acc[n]);
             acc[n] = mfma<bf16_ops<WT>()>(da, xs.lo[tn][tslot<TOK, KC>(tn, c)], acc[n]);
+            if constexpr (RAG)
+              acc[n] = mfma<bf16_ops<WT>()>(da, xs.l2[tn][tslot<TOK, KC>(tn, c)], acc[n]);
           }
         }
+        if constexpr (RAG) ksum_close(ta, acc);
       }
     }
   }
@@ -1031,7 +1242,12 @@ __device__ __forceinline__ void dn_pass(TokTile<TOK, KC>& xs, WTile<WT, 16, WK>&
   // exactly.  fp8: rows row0 + 4 (lane / 16) .. + 4 times their scales.
   const int rq = row0 + (lane >> 4) * 4;
   f32x4 sd;
-  if constexpr (std::is_same<WT, fp8w>::value) sd = *reinterpret_cast<const f32x4*>(sdown + rq);
+  if constexpr (std::is_same<WT, fp8w>::value && RAG) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sd[i] = sdown[min(rq + i, g.h - 1)];
+  } else if constexpr (std::is_same<WT, fp8w>::value) {
+    sd = *reinterpret_cast<const f32x4*>(sdown + rq);
+  }
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
     const int tn = n * 16 + (lane & 15);
@@ -1045,21 +1261,22 @@ __device__ __forceinline__ void dn_pass(TokTile<TOK, KC>& xs, WTile<WT, 16, WK>&
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] *= sd[i];
       }
-      *reinterpret_cast<f32x4*>(y + (int64_t)(p0 + tn) * g.h + rq) = v;
+      *reinterpret_cast<f32x4*>(y + (int64_t)(p0 + tn) * (RAG ? g.hp : g.h) + rq) = v;
     }
   }
 }
 
 // PRE: act was split into its two terms by k_act_split.  WK: the weight K
 // step (dn_pass); the K slices are then whole weight steps.
-template <typename WT, int TOK, int KC, bool PRE = false, int WK = KC>
-__global__ __launch_bounds__(kBlk) void k_dn_mfma(const WT* __restrict__ wbuf, BatchRoute r,
-                                                  const float* __restrict__ act,
-                                                  const unsigned* __restrict__ amax,
-                                                  float* __restrict__ ypart, Geom g, int P) {
-  __shared__ TokTile<TOK, KC> xs;
+template <typename WT, int TOK, int KC, bool PRE, int WK, bool RAG>
+__device__ __forceinline__ void dn_block(const WT* __restrict__ wbuf, const BatchRoute& r,
+                                         const float* __restrict__ act,
+                                         const unsigned* __restrict__ amax,
+                                         float* __restrict__ ypart, const GeomB& g, int P) {
+  __shared__ TokTile<TOK, KC, RAG> xs;
   __shared__ WTile<WT, 16, WK> wts[kBlk / kWave];
-  const int slot = tile_slot<TOK>(r, blockIdx.z);
+  const int slot = RAG ? ((int)blockIdx.z < r.n_active[0] ? (int)blockIdx.z : -1)
+                       : tile_slot<TOK>(r, blockIdx.z);
   if (slot < 0) return;
   const int e = r.active[slot];
   const int pbeg = r.off[e], M = r.off[e + 1] - pbeg;
@@ -1081,7 +1298,7 @@ __global__ __launch_bounds__(kBlk) void k_dn_mfma(const WT* __restrict__ wbuf, B
   }
   const int row0 = bx * kBM + wave * 16;
   constexpr int R = WK / KC;  // token steps per weight step (I % WK == 0)
-  const int nsteps = g.I / WK;
+  const int nsteps = (RAG ? g.Ip : g.I) / WK;
   const int sb = nsteps * ks / BatchWs::kKSplit * R;
   const int se = nsteps * (ks + 1) / BatchWs::kKSplit * R;
   const WT* blk = wbuf + (int64_t)e * g.stride;
@@ -1096,30 +1313,53 @@ __global__ __launch_bounds__(kBlk) void k_dn_mfma(const WT* __restrict__ wbuf, B
       reinterpret_cast<const uint8_t*>(blk) + g.off_scale + 2 * ((int64_t)g.I * g.h / 32);
 #pragma unroll
   for (int i = 0; i < N; ++i) {
+    if constexpr (RAG) {
+      const int row = min(row0 + lane / WGeo<WT, WK>::kLaneRow + WGeo<WT, WK>::kRowsPer * i, g.h - 1);
+      wbase[i] = blk + g.off_down + eoff<WT>((int64_t)row * g.I);
+      wsc[i] = mxs + (int64_t)row * (g.I / 32);
+      continue;
+    }
     wbase[i] = D + eoff<WT>((int64_t)(WGeo<WT, WK>::kRowsPer * i) * g.I);
     wsc[i] = w_lane_scale<WT, WK>(mxs, row0, g.I, lane) +
              (int64_t)(WGeo<WT, WK>::kRowsPer * i) * (g.I / 32);
   }
-  float* y = ypart + (int64_t)ks * P * g.h;
+  float* y = ypart + (int64_t)ks * P * (RAG ? g.hp : g.h);
   WTile<WT, 16, WK>& wt = wts[wave];
   for (int m0 = 0; m0 < M; m0 += TOK) {
     const int mt = min(TOK, M - m0);
     if constexpr (TOK == 16) {
-      dn_pass<WT, 1, TOK, KC, PRE, WK>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane);
+      dn_pass<WT, 1, TOK, KC, PRE, WK, RAG>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane);
     } else if constexpr (TOK == 32) {
       if (mt <= 16)
-        dn_pass<WT, 1, TOK, KC, PRE, WK>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane);
+        dn_pass<WT, 1, TOK, KC, PRE, WK, RAG>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane);
       else
-        dn_pass<WT, 2, TOK, KC, PRE, WK>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane);
+        dn_pass<WT, 2, TOK, KC, PRE, WK, RAG>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane);
     } else {
       switch ((mt + 15) / 16) {
-        case 1: dn_pass<WT, 1, TOK, KC, PRE, WK>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane); break;
-        case 2: dn_pass<WT, 2, TOK, KC, PRE, WK>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane); break;
-        case 3: dn_pass<WT, 3, TOK, KC, PRE, WK>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane); break;
-        default: dn_pass<WT, 4, TOK, KC, PRE, WK>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane); break;
+        case 1: dn_pass<WT, 1, TOK, KC, PRE, WK, RAG>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane); break;
+        case 2: dn_pass<WT, 2, TOK, KC, PRE, WK, RAG>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane); break;
+        case 3: dn_pass<WT, 3, TOK, KC, PRE, WK, RAG>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane); break;
+        default: dn_pass<WT, 4, TOK, KC, PRE, WK, RAG>(xs, wt, wbase, wsc, act, amax, pbeg + m0, mt, sb, se, y, row0, sdown, g, lane); break;
       }
     }
   }
+}
+
+template <typename WT, int TOK, int KC, bool PRE = false, int WK = KC>
+__global__ __launch_bounds__(kBlk) void k_dn_mfma(const WT* __restrict__ wbuf, BatchRoute r,
+                                                  const float* __restrict__ act,
+                                                  const unsigned* __restrict__ amax,
+                                                  float* __restrict__ ypart, GeomB g, int P) {
+  dn_block<WT, TOK, KC, PRE, WK, false>(wbuf, r, act, amax, ypart, g, P);
+}
+
+// Ragged layers, as k_rag_gu.
+template <typename WT, int TOK>
+__global__ __launch_bounds__(kBlk) void k_rag_dn(const WT* __restrict__ wbuf, BatchRoute r,
+                                                 const float* __restrict__ act,
+                                                 const unsigned* __restrict__ amax,
+                                                 float* __restrict__ ypart, GeomB g, int P) {
+  dn_block<WT, TOK, kBK, false, kBK, true>(wbuf, r, act, amax, ypart, g, P);
 }
 
 // act [P][I] (fp32, I a multiple of 8) split into its two 16-bit terms once,
@@ -1250,6 +1490,29 @@ __device__ __forceinline__ void f32_w_load(WRegsF<ROWS>& r, const float* const (
   for (int i = 0; i < ROWS / 4; ++i)
     r.v[i] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(base[i] + kb));
 }
+// Ragged rows, as w_load_rag and w_rag_fix: bases are row starts.
+template <int ROWS>
+__device__ __forceinline__ void f32_w_load_rag(WRegsF<ROWS>& r,
+                                               const float* const (&base)[ROWS / 4], int kb, int K,
+                                               int lane) {
+  const int c = min(kb + 4 * (lane % 16), K - 4);
+#pragma unroll
+  for (int i = 0; i < ROWS / 4; ++i)
+    r.v[i] = __builtin_bit_cast(
+        f32x4, __builtin_nontemporal_load(reinterpret_cast<const u32x4u*>(base[i] + c)));
+}
+template <int ROWS>
+__device__ __forceinline__ void f32_w_rag_fix(WRegsF<ROWS>& r, int kb, int K, int lane) {
+  if (kb + kBKF <= K) return;  // uniform
+  const int d = kb + 4 * (lane % 16) - (K - 4);
+#pragma unroll
+  for (int i = 0; i < ROWS / 4; ++i) {
+    const f32x4 v = r.v[i];
+    if (d > 0)
+      r.v[i] = f32x4{d == 1 ? v[1] : d == 2 ? v[2] : d == 3 ? v[3] : 0.0f,
+                     d == 1 ? v[2] : d == 2 ? v[3] : 0.0f, d == 1 ? v[3] : 0.0f, 0.0f};
+  }
+}
 template <int ROWS>
 __device__ __forceinline__ void f32_w_store(TileF<ROWS>& t, const WRegsF<ROWS>& r, int lane) {
 #pragma unroll
@@ -1259,33 +1522,45 @@ __device__ __forceinline__ void f32_w_store(TileF<ROWS>& t, const WRegsF<ROWS>& 
 
 // Gate/up pass over up to TOK tokens (NT tiles of 16) of one expert, rows
 // row0 .. + 16 of its gate and up matrices (tile rows 0-15 and 16-31).
-template <typename XT, int NT, int TOK>
+template <typename XT, int NT, int TOK, bool RAG>
 __device__ __forceinline__ void gu_pass_f32(TileF<TOK>& xs, TileF<32>& wt,
                                             const float* const (&wbase)[8],
                                             const XT* __restrict__ x, const BatchRoute& r,
                                             int p0, int mt, float* __restrict__ act, int row0,
-                                            const Geom& g, int lane) {
+                                            const GeomB& g, int lane) {
   f32x4 ag[NT], au[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) ag[n] = au[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   constexpr int TP = f32_tile_pieces<TOK>();
   int64_t off[TP];
-  f32_tile_rows(off, r.pair_tok + p0, 0, mt, g.h);
-  const int ns = g.h / kBKF;
+  f32_tile_rows(off, r.pair_tok + p0, 0, mt, RAG ? g.hp : g.h);
+  const int ns = (RAG ? g.hp : g.h) / kBKF;
   const int q = lane >> 4, rl = lane & 15;
   WRegsF<32> wr;
   typename RawX4<XT>::type tv[TP];
-  f32_w_load<32>(wr, wbase, 0);
+  if constexpr (RAG)
+    f32_w_load_rag<32>(wr, wbase, 0, g.h, lane);
+  else
+    f32_w_load<32>(wr, wbase, 0);
   f32_tile_load(tv, x, off, 0);
   for (int s = 0; s < ns; ++s) {
     __syncthreads();  // every wave is done reading the previous tiles
     f32_tile_store(xs, tv);
+    if constexpr (RAG) f32_w_rag_fix<32>(wr, s * kBKF, g.h, lane);
     f32_w_store<32>(wt, wr, lane);
     __syncthreads();
     if (s + 1 < ns) {
-      f32_w_load<32>(wr, wbase, (s + 1) * kBKF);
+      if constexpr (RAG)
+        f32_w_load_rag<32>(wr, wbase, (s + 1) * kBKF, g.h, lane);
+      else
+        f32_w_load<32>(wr, wbase, (s + 1) * kBKF);
       f32_tile_load(tv, x, off, (s + 1) * kBKF);
     }
+    f32x4 tg[RAG ? NT : 1], tu[RAG ? NT : 1];
+    if constexpr (RAG) {
+        ksum_open(tg, ag);
+        ksum_open(tu, au);
+      }
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const f32x4 ga = wt.v[rl][fslot(rl, 4 * j + q)];
@@ -1300,6 +1575,10 @@ __device__ __forceinline__ void gu_pass_f32(TileF<TOK>& xs, TileF<32>& wt,
         }
       }
     }
+    if constexpr (RAG) {
+        ksum_close(tg, ag);
+        ksum_close(tu, au);
+      }
   }
   // D layout: lane holds token n*16 + (lane % 16), rows 4 (lane / 16) .. +4.
   const int rq = row0 + q * 4;
@@ -1311,21 +1590,22 @@ __device__ __forceinline__ void gu_pass_f32(TileF<TOK>& xs, TileF<32>& wt,
       const float w = r.pair_w[p];
       f32x4 v;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = w * (silu(ag[n][i]) * au[n][i]);
-      *reinterpret_cast<f32x4*>(act + (int64_t)p * g.I + rq) = v;
+      for (int i = 0; i < 4; ++i)
+        v[i] = RAG && rq + i >= g.I ? 0.0f : w * (silu(ag[n][i]) * au[n][i]);
+      *reinterpret_cast<f32x4*>(act + (int64_t)p * (RAG ? g.Ip : g.I) + rq) = v;
     }
   }
 }
 
 // grid (I / 64, expert slots); as k_gu_mfma, with x read as it is (fp32 or
 // fp16) and no scaling.
-template <typename XT, int TOK, bool ROUTE>
-__global__ __launch_bounds__(kBlk) void k_gu_f32(const float* __restrict__ wbuf,
-                                                 const XT* __restrict__ x, BatchRoute r,
-                                                 float* __restrict__ act, Geom g,
-                                                 const float* __restrict__ logits,
-                                                 int32_t* __restrict__ ids_out,
-                                                 float* __restrict__ w_out) {
+template <typename XT, int TOK, bool ROUTE, bool RAG>
+__device__ __forceinline__ void gu_block_f32(const float* __restrict__ wbuf,
+                                             const XT* __restrict__ x, BatchRoute r,
+                                             float* __restrict__ act, const GeomB& g,
+                                             const float* __restrict__ logits,
+                                             int32_t* __restrict__ ids_out,
+                                             float* __restrict__ w_out) {
   __shared__ TileF<TOK> xs;
   __shared__ TileF<32> wts[kBlk / kWave];
   __shared__ GuRouteLds<ROUTE> rl;
@@ -1353,41 +1633,71 @@ __global__ __launch_bounds__(kBlk) void k_gu_f32(const float* __restrict__ wbuf,
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int row0 = blockIdx.x * kBM + wave * 16;
+  if (RAG && (int)blockIdx.x * kBM >= g.I) {  // a block of act's padding columns: zeros
+    for (int i = threadIdx.x; i < M * (kBM / 4); i += kBlk)
+      *reinterpret_cast<f32x4*>(act + (int64_t)(pbeg + i / (kBM / 4)) * g.Ip + blockIdx.x * kBM +
+                                4 * (i % (kBM / 4))) = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    return;
+  }
   const float* blk = wbuf + (int64_t)e * g.stride;
   const float* G = blk + (int64_t)(row0 + lane / 16) * g.h + 4 * (lane % 16);
   const float* wbase[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) wbase[i] = G + (i < 4 ? 0 : g.off_up) + (int64_t)(4 * (i % 4)) * g.h;
+  for (int i = 0; i < 8; ++i)
+    wbase[i] = RAG ? blk + (i < 4 ? 0 : g.off_up) +
+                         (int64_t)min(row0 + lane / 16 + 4 * (i % 4), g.I - 1) * g.h
+                   : G + (i < 4 ? 0 : g.off_up) + (int64_t)(4 * (i % 4)) * g.h;
   TileF<32>& wt = wts[wave];
   for (int m0 = 0; m0 < M; m0 += TOK) {
     const int mt = min(TOK, M - m0);
     const int p0 = pbeg + m0;
     if constexpr (TOK == 16) {
-      gu_pass_f32<XT, 1, TOK>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane);
+      gu_pass_f32<XT, 1, TOK, RAG>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane);
     } else if constexpr (TOK == 32) {
       if (mt <= 16)
-        gu_pass_f32<XT, 1, TOK>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane);
+        gu_pass_f32<XT, 1, TOK, RAG>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane);
       else
-        gu_pass_f32<XT, 2, TOK>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane);
+        gu_pass_f32<XT, 2, TOK, RAG>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane);
     } else {
       switch ((mt + 15) / 16) {
-        case 1: gu_pass_f32<XT, 1, TOK>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane); break;
-        case 2: gu_pass_f32<XT, 2, TOK>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane); break;
-        case 3: gu_pass_f32<XT, 3, TOK>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane); break;
-        default: gu_pass_f32<XT, 4, TOK>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane); break;
+        case 1: gu_pass_f32<XT, 1, TOK, RAG>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane); break;
+        case 2: gu_pass_f32<XT, 2, TOK, RAG>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane); break;
+        case 3: gu_pass_f32<XT, 3, TOK, RAG>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane); break;
+        default: gu_pass_f32<XT, 4, TOK, RAG>(xs, wt, wbase, x, r, p0, mt, act, row0, g, lane); break;
       }
     }
   }
 }
 
+template <typename XT, int TOK, bool ROUTE>
+__global__ __launch_bounds__(kBlk) void k_gu_f32(const float* __restrict__ wbuf,
+                                                 const XT* __restrict__ x, BatchRoute r,
+                                                 float* __restrict__ act, GeomB g,
+                                                 const float* __restrict__ logits,
+                                                 int32_t* __restrict__ ids_out,
+                                                 float* __restrict__ w_out) {
+  gu_block_f32<XT, TOK, ROUTE, false>(wbuf, x, r, act, g, logits, ids_out, w_out);
+}
+
+// Ragged layers, as k_rag_gu; x is the workspace's padded fp32 copy.
+template <int TOK, bool ROUTE>
+__global__ __launch_bounds__(kBlk) void k_rag_gu_f32(const float* __restrict__ wbuf,
+                                                     const float* __restrict__ x, BatchRoute r,
+                                                     float* __restrict__ act, GeomB g,
+                                                     const float* __restrict__ logits,
+                                                     int32_t* __restrict__ ids_out,
+                                                     float* __restrict__ w_out) {
+  gu_block_f32<float, TOK, ROUTE, true>(wbuf, x, r, act, g, logits, ids_out, w_out);
+}
+
 // Down pass: K steps [sb, se) of 64 columns, rows row0 .. + 16 of the down
 // matrix against the pass's act rows (fp32, as written by the gate/up pass).
-template <int NT, int TOK>
+template <int NT, int TOK, bool RAG>
 __device__ __forceinline__ void dn_pass_f32(TileF<TOK>& xs, TileF<16>& wt,
                                             const float* const (&wbase)[4],
                                             const float* __restrict__ act, int p0, int mt,
                                             int sb, int se, float* __restrict__ y, int row0,
-                                            const Geom& g, int lane) {
+                                            const GeomB& g, int lane) {
   f32x4 acc[NT];
 #pragma unroll
   for (int n = 0; n < NT; ++n) acc[n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1395,20 +1705,29 @@ __device__ __forceinline__ void dn_pass_f32(TileF<TOK>& xs, TileF<16>& wt,
   if (sb < se) {
     constexpr int TP = f32_tile_pieces<TOK>();
     int64_t off[TP];
-    f32_tile_rows(off, nullptr, p0, mt, g.I);
+    f32_tile_rows(off, nullptr, p0, mt, RAG ? g.Ip : g.I);
     WRegsF<16> wr;
     f32x4 tv[TP];
-    f32_w_load<16>(wr, wbase, sb * kBKF);
+    if constexpr (RAG)
+      f32_w_load_rag<16>(wr, wbase, sb * kBKF, g.I, lane);
+    else
+      f32_w_load<16>(wr, wbase, sb * kBKF);
     f32_tile_load(tv, act, off, sb * kBKF);
     for (int s = sb; s < se; ++s) {
       __syncthreads();
       f32_tile_store(xs, tv);
+      if constexpr (RAG) f32_w_rag_fix<16>(wr, s * kBKF, g.I, lane);
       f32_w_store<16>(wt, wr, lane);
       __syncthreads();
       if (s + 1 < se) {
-        f32_w_load<16>(wr, wbase, (s + 1) * kBKF);
+        if constexpr (RAG)
+          f32_w_load_rag<16>(wr, wbase, (s + 1) * kBKF, g.I, lane);
+        else
+          f32_w_load<16>(wr, wbase, (s + 1) * kBKF);
         f32_tile_load(tv, act, off, (s + 1) * kBKF);
       }
+      f32x4 ta[RAG ? NT : 1];
+      if constexpr (RAG) ksum_open(ta, acc);
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const f32x4 da = wt.v[rl][fslot(rl, 4 * j + q)];
@@ -1419,22 +1738,24 @@ __device__ __forceinline__ void dn_pass_f32(TileF<TOK>& xs, TileF<16>& wt,
           for (int m = 0; m < 4; ++m) acc[n] = mfma_f32(da[m], b[m], acc[n]);
         }
       }
+      if constexpr (RAG) ksum_close(ta, acc);
     }
   }
   const int rq = row0 + q * 4;
 #pragma unroll
   for (int n = 0; n < NT; ++n) {
     const int tn = n * 16 + rl;
-    if (tn < mt) *reinterpret_cast<f32x4*>(y + (int64_t)(p0 + tn) * g.h + rq) = acc[n];
+    if (tn < mt)
+      *reinterpret_cast<f32x4*>(y + (int64_t)(p0 + tn) * (RAG ? g.hp : g.h) + rq) = acc[n];
   }
 }
 
 // grid (h / 64, kKSplit, expert slots); K slice ks covers steps
 // [nsteps ks / kKSplit, nsteps (ks + 1) / kKSplit) of I / 64.
-template <int TOK>
-__global__ __launch_bounds__(kBlk) void k_dn_f32(const float* __restrict__ wbuf, BatchRoute r,
-                                                 const float* __restrict__ act,
-                                                 float* __restrict__ ypart, Geom g, int P) {
+template <int TOK, bool RAG>
+__device__ __forceinline__ void dn_block_f32(const float* __restrict__ wbuf, const BatchRoute& r,
+                                             const float* __restrict__ act,
+                                             float* __restrict__ ypart, const GeomB& g, int P) {
   __shared__ TileF<TOK> xs;
   __shared__ TileF<16> wts[kBlk / kWave];
   const int slot = blockIdx.z;
@@ -1445,34 +1766,51 @@ __global__ __launch_bounds__(kBlk) void k_dn_f32(const float* __restrict__ wbuf,
   const int wave = threadIdx.x / kWave;
   const int row0 = blockIdx.x * kBM + wave * 16;
   const int ks = blockIdx.y;
-  const int nsteps = g.I / kBKF;
+  const int nsteps = (RAG ? g.Ip : g.I) / kBKF;
   const int sb = nsteps * ks / BatchWs::kKSplit;
   const int se = nsteps * (ks + 1) / BatchWs::kKSplit;
   const float* D = wbuf + (int64_t)e * g.stride + g.off_down +
                    (int64_t)(row0 + lane / 16) * g.I + 4 * (lane % 16);
   const float* wbase[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) wbase[i] = D + (int64_t)(4 * i) * g.I;
-  float* y = ypart + (int64_t)ks * P * g.h;
+  for (int i = 0; i < 4; ++i)
+    wbase[i] = RAG ? wbuf + (int64_t)e * g.stride + g.off_down +
+                         (int64_t)min(row0 + lane / 16 + 4 * i, g.h - 1) * g.I
+                   : D + (int64_t)(4 * i) * g.I;
+  float* y = ypart + (int64_t)ks * P * (RAG ? g.hp : g.h);
   TileF<16>& wt = wts[wave];
   for (int m0 = 0; m0 < M; m0 += TOK) {
     const int mt = min(TOK, M - m0);
     if constexpr (TOK == 16) {
-      dn_pass_f32<1, TOK>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane);
+      dn_pass_f32<1, TOK, RAG>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane);
     } else if constexpr (TOK == 32) {
       if (mt <= 16)
-        dn_pass_f32<1, TOK>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane);
+        dn_pass_f32<1, TOK, RAG>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane);
       else
-        dn_pass_f32<2, TOK>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane);
+        dn_pass_f32<2, TOK, RAG>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane);
     } else {
       switch ((mt + 15) / 16) {
-        case 1: dn_pass_f32<1, TOK>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane); break;
-        case 2: dn_pass_f32<2, TOK>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane); break;
-        case 3: dn_pass_f32<3, TOK>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane); break;
-        default: dn_pass_f32<4, TOK>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane); break;
+        case 1: dn_pass_f32<1, TOK, RAG>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane); break;
+        case 2: dn_pass_f32<2, TOK, RAG>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane); break;
+        case 3: dn_pass_f32<3, TOK, RAG>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane); break;
+        default: dn_pass_f32<4, TOK, RAG>(xs, wt, wbase, act, pbeg + m0, mt, sb, se, y, row0, g, lane); break;
       }
     }
   }
+}
+
+template <int TOK>
+__global__ __launch_bounds__(kBlk) void k_dn_f32(const float* __restrict__ wbuf, BatchRoute r,
+                                                 const float* __restrict__ act,
+                                                 float* __restrict__ ypart, GeomB g, int P) {
+  dn_block_f32<TOK, false>(wbuf, r, act, ypart, g, P);
+}
+
+template <int TOK>
+__global__ __launch_bounds__(kBlk) void k_rag_dn_f32(const float* __restrict__ wbuf, BatchRoute r,
+                                                     const float* __restrict__ act,
+                                                     float* __restrict__ ypart, GeomB g, int P) {
+  dn_block_f32<TOK, true>(wbuf, r, act, ypart, g, P);
 }
 
 // out[t][row]: grid (ceil(h / 256), B); K = k, so that every loop is exact.
@@ -1481,7 +1819,7 @@ __global__ __launch_bounds__(kBlk) void k_dn_f32(const float* __restrict__ wbuf,
 // selection order, K slices ascending).
 template <typename OT, int K>
 __global__ __launch_bounds__(kBlk) void k_combine(const float* __restrict__ ypart, BatchRoute r,
-                                                  OT* __restrict__ out, int h, int P) {
+                                                  OT* __restrict__ out, int h, int hp, int P) {
   const int t = blockIdx.y;
   const int row = blockIdx.x * kBlk + threadIdx.x;
   if (row >= h) return;
@@ -1493,7 +1831,7 @@ __global__ __launch_bounds__(kBlk) void k_combine(const float* __restrict__ ypar
   for (int kk = 0; kk < K; ++kk)
 #pragma unroll
     for (int ks = 0; ks < BatchWs::kKSplit; ++ks)
-      v[kk][ks] = ypart[((int64_t)ks * P + p[kk]) * h + row];
+      v[kk][ks] = ypart[((int64_t)ks * P + p[kk]) * hp + row];
   float s = 0.0f;
 #pragma unroll
   for (int kk = 0; kk < K; ++kk)
@@ -1503,16 +1841,29 @@ __global__ __launch_bounds__(kBlk) void k_combine(const float* __restrict__ ypar
 }
 
 template <typename OT, int K>
-hipError_t launch_combine(const BatchWs& w, const Problem& p, hipStream_t s) {
+hipError_t launch_combine(const BatchWs& w, const Problem& p, int hp, hipStream_t s) {
   hipLaunchKernelGGL((k_combine<OT, K>), dim3((p.h + kBlk - 1) / kBlk, p.B), dim3(kBlk), 0, s,
-                     w.ypart, w.route, static_cast<OT*>(p.out), p.h, p.B * K);
+                     w.ypart, w.route, static_cast<OT*>(p.out), p.h, hp, p.B * K);
   return hipGetLastError();
 }
 
-template <typename WT, typename XT>
-hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
-  constexpr int64_t es = sizeof(WT);  // bytes per storage unit (two MXFP4 codes per byte)
-  Geom g;
+template <typename OT>
+hipError_t launch_combine_k(const BatchWs& w, const Problem& p, int hp, hipStream_t s) {
+  static_assert(WR_MAX_TOPK == 6, "one combine instantiation per k");
+  switch (p.k) {
+    case 1: return launch_combine<OT, 1>(w, p, hp, s);
+    case 2: return launch_combine<OT, 2>(w, p, hp, s);
+    case 3: return launch_combine<OT, 3>(w, p, hp, s);
+    case 4: return launch_combine<OT, 4>(w, p, hp, s);
+    case 5: return launch_combine<OT, 5>(w, p, hp, s);
+    default: return launch_combine<OT, 6>(w, p, hp, s);
+  }
+}
+
+// es: bytes per storage unit (two MXFP4 codes per byte).  ragged: workspace
+// rows of whole K steps.
+GeomB make_geom_b(const Problem& p, int64_t es, bool ragged) {
+  GeomB g;
   g.E = p.E;
   g.h = p.h;
   g.I = p.I;
@@ -1523,6 +1874,82 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
   g.off_up = p.off_up_b / es;
   g.off_down = p.off_down_b / es;
   g.off_scale = p.off_scale_b;
+  g.hp = ragged ? BatchWs::padded(p.h) : p.h;
+  g.Ip = ragged ? BatchWs::padded(p.I) : p.I;
+  return g;
+}
+
+// Rows of whole, aligned 16-byte pieces and whole K steps.
+bool aligned_ok(const Problem& p) {
+  if (p.wdt == WR_F32)  // 64-column K steps, 16-byte rows
+    return p.vec == 4 && p.h % kBKF == 0 && p.I % kBKF == 0;
+  const bool wt = ((p.wdt == WR_F16 || p.wdt == WR_BF16) && p.vec == 8) ||
+                  (p.wdt == WR_FP8_E4M3 && p.vec == 16) || (p.wdt == WR_MXFP4 && p.vec == 32);
+  return wt && p.h % kBK == 0 && p.I % kBK == 0;
+}
+
+// Token tile of a ragged layer: 16 and 32 as the aligned layers', then 64
+// when the average expert gets more than 24 tokens (an expert with more
+// than the tile takes several passes).
+int rag_tile(const Problem& p) {
+  if (p.B <= WR_SMALL_TILE_MAX_B) return 16;
+  return p.B <= WR_MID_TILE_MAX_B || p.B * p.k <= 24 * p.E ? 32 : 64;
+}
+
+template <typename WT, typename XT>
+hipError_t ragged_t(const Problem& p, const BatchWs& w, hipStream_t s) {
+  const GeomB g = make_geom_b(p, sizeof(WT), true);
+  const int P = p.B * p.k, slots = std::min(p.E, P);
+  const WT* wb = static_cast<const WT*>(p.wbuf);
+  constexpr bool LO = std::is_same<XT, float>::value || bf16_ops<WT>();
+  const int tile = rag_tile(p);
+  hipError_t err = hipSuccess;
+  if (tile > 16) {
+    hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
+                       p.topk_ids, p.topk_w, w.route);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+  }
+  const dim3 gg(g.Ip / kBM, slots), gd((p.h + kBM - 1) / kBM, BatchWs::kKSplit, slots);
+  constexpr bool L2 = std::is_same<XT, float>::value;  // fp16 x: two terms hold all of it
+  auto gu = tile == 16   ? k_rag_gu<WT, LO, L2, 16, true>
+            : tile == 32 ? k_rag_gu<WT, LO, L2, 32, false>
+                         : k_rag_gu<WT, LO, L2, kMaxTok, false>;
+  auto dn = tile == 16 ? k_rag_dn<WT, 16> : (tile == 32 ? k_rag_dn<WT, 32> : k_rag_dn<WT, kMaxTok>);
+  hipLaunchKernelGGL(gu, gg, dim3(kBlk), 0, s, wb, w.x_hi, w.x_lo, w.x_l2(), w.x_exp, w.amax,
+                     w.route, w.act, g, w.logits, p.topk_ids, p.topk_w);
+  if ((err = hipGetLastError()) != hipSuccess) return err;
+  hipLaunchKernelGGL(dn, gd, dim3(kBlk), 0, s, wb, w.route, w.act, w.amax, w.ypart, g, P);
+  if ((err = hipGetLastError()) != hipSuccess) return err;
+  return launch_combine_k<XT>(w, p, g.hp, s);
+}
+
+template <typename OT>
+hipError_t ragged_f32(const Problem& p, const BatchWs& w, hipStream_t s) {
+  const GeomB g = make_geom_b(p, 4, true);
+  const int P = p.B * p.k, slots = std::min(p.E, P);
+  const float* wb = static_cast<const float*>(p.wbuf);
+  const int tile = rag_tile(p);
+  hipError_t err = hipSuccess;
+  if (tile > 16) {
+    hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
+                       p.topk_ids, p.topk_w, w.route);
+    if ((err = hipGetLastError()) != hipSuccess) return err;
+  }
+  const dim3 gg(g.Ip / kBM, slots), gd((p.h + kBM - 1) / kBM, BatchWs::kKSplit, slots);
+  auto gu = tile == 16 ? k_rag_gu_f32<16, true>
+                       : (tile == 32 ? k_rag_gu_f32<32, false> : k_rag_gu_f32<kMaxTok, false>);
+  auto dn = tile == 16 ? k_rag_dn_f32<16> : (tile == 32 ? k_rag_dn_f32<32> : k_rag_dn_f32<kMaxTok>);
+  hipLaunchKernelGGL(gu, gg, dim3(kBlk), 0, s, wb, w.x_f32(), w.route, w.act, g, w.logits,
+                     p.topk_ids, p.topk_w);
+  if ((err = hipGetLastError()) != hipSuccess) return err;
+  hipLaunchKernelGGL(dn, gd, dim3(kBlk), 0, s, wb, w.route, w.act, w.ypart, g, P);
+  if ((err = hipGetLastError()) != hipSuccess) return err;
+  return launch_combine_k<OT>(w, p, g.hp, s);
+}
+
+template <typename WT, typename XT>
+hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
+  const GeomB g = make_geom_b(p, sizeof(WT), false);
   const int P = p.B * p.k;
   const int slots = std::min(p.E, P);
   const WT* wb = static_cast<const WT*>(p.wbuf);
@@ -1638,30 +2065,12 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
     }
   }
   if ((err = hipGetLastError()) != hipSuccess) return err;
-  static_assert(WR_MAX_TOPK == 6, "one combine instantiation per k");
-  switch (p.k) {
-    case 1: return launch_combine<XT, 1>(w, p, s);
-    case 2: return launch_combine<XT, 2>(w, p, s);
-    case 3: return launch_combine<XT, 3>(w, p, s);
-    case 4: return launch_combine<XT, 4>(w, p, s);
-    case 5: return launch_combine<XT, 5>(w, p, s);
-    default: return launch_combine<XT, 6>(w, p, s);
-  }
+  return launch_combine_k<XT>(w, p, g.hp, s);
 }
 
 template <typename XT>
 hipError_t grouped_f32(const Problem& p, const BatchWs& w, hipStream_t s) {
-  Geom g;
-  g.E = p.E;
-  g.h = p.h;
-  g.I = p.I;
-  g.k = p.k;
-  g.renorm = p.renorm;
-  g.B = p.B;
-  g.stride = p.stride_b / 4;
-  g.off_up = p.off_up_b / 4;
-  g.off_down = p.off_down_b / 4;
-  g.off_scale = -1;
+  const GeomB g = make_geom_b(p, 4, false);
   const int P = p.B * p.k;
   const int slots = std::min(p.E, P);
   const float* wb = static_cast<const float*>(p.wbuf);
@@ -1692,29 +2101,47 @@ hipError_t grouped_f32(const Problem& p, const BatchWs& w, hipStream_t s) {
                        0, s, wb, w.route, w.act, w.ypart, g, P);
   }
   if ((err = hipGetLastError()) != hipSuccess) return err;
-  switch (p.k) {
-    case 1: return launch_combine<XT, 1>(w, p, s);
-    case 2: return launch_combine<XT, 2>(w, p, s);
-    case 3: return launch_combine<XT, 3>(w, p, s);
-    case 4: return launch_combine<XT, 4>(w, p, s);
-    case 5: return launch_combine<XT, 5>(w, p, s);
-    default: return launch_combine<XT, 6>(w, p, s);
-  }
+  return launch_combine_k<XT>(w, p, g.hp, s);
 }
 
 }  // namespace
 
+// Aligned layers always; ragged ones (rows of at least one 16-byte piece, which
+// MXFP4 rows always are) where tokens share experts and the layer is not tiny.
+// Measured, µs per call, per-token kernels against these:
+//   fewer than 1.5 pairs per expert: E 8, k 2, h 1000, I 1400, B = 4 fp16 22.1
+//   / 34.0, fp8 23.5 / 29.4; E 16, k 4, 1501 x 1003, B = 4 fp16 43.3 / 48.3,
+//   fp32 58.5 / 72.2; with more: B = 8 fp16 33.4 / 34.7 and 69.2 / 53.5, fp8
+//   37.9 / 30.1 and 73.0 / 42.9, fp32 53.3 / 50.9 and 105 / 80.0; B = 32 fp16
+//   72.0 / 39.3 and 211 / 60.6;
+//   few weight bytes over all pairs (four launches and their latency): 264 x
+//   520, fp16 B = 8 (13 MB) 17.9 / 21.7, B = 16 (26 MB) 23.1 / 21.8; fp32 B =
+//   16 (52 MB) 23.8 / 25.5; fp8 B = 8 (7 MB) 21.1 / 20.4; 101 x 37, fp16
+//   B = 32 (1 MB) 16.7 / 21.7.
 bool grouped_ok(const Problem& p) {
   if (p.B <= 1) return false;
-  if (p.wdt == WR_F32)  // 64-column K steps, 16-byte rows
-    return p.vec == 4 && p.h % kBKF == 0 && p.I % kBKF == 0;
-  const bool wt = ((p.wdt == WR_F16 || p.wdt == WR_BF16) && p.vec == 8) ||
-                  (p.wdt == WR_FP8_E4M3 && p.vec == 16) || (p.wdt == WR_MXFP4 && p.vec == 32);
-  return wt && p.h % kBK == 0 && p.I % kBK == 0;
+  if (aligned_ok(p)) return true;
+  const int piece = p.wdt == WR_F32          ? 4
+                    : p.wdt == WR_FP8_E4M3 ? 16
+                    : p.wdt == WR_MXFP4    ? 32
+                                           : 8;
+  if (p.h < piece || p.I < piece) return false;
+  const int64_t pairs = (int64_t)p.B * p.k;
+  const int64_t tiny = (int64_t)(p.wdt == WR_F32 ? 64 : piece == 8 ? 16 : 4) << 20;
+  return 2 * pairs >= 3 * p.E && pairs * p.stride_b > tiny;
 }
 
 hipError_t launch_grouped(const Problem& p, hipStream_t s) {
   const BatchWs w = BatchWs::carve(p.ws, p.E, p.h, p.I, p.k, p.B);
+  const bool ragged = !aligned_ok(p);
+  if (p.wdt == WR_F32 && ragged) {  // x in fp32 rows of whole K steps
+    XSplit xs = x_split(p);
+    xs.f32 = w.x_f32();
+    xs.ld = BatchWs::padded(p.h);
+    hipError_t err = launch_logits_split(p, w.logits, xs, s);
+    if (err != hipSuccess) return err;
+    return p.adt == WR_F16 ? ragged_f32<f16>(p, w, s) : ragged_f32<float>(p, w, s);
+  }
   if (p.wdt == WR_F32) {  // exact fp32 products: x as it is, logits only
     hipError_t err = launch_logits(p, w.logits, s);
     if (err != hipSuccess) return err;
@@ -1722,9 +2149,25 @@ hipError_t launch_grouped(const Problem& p, hipStream_t s) {
   }
   // bf16 operands (bf16 and MXFP4 weights): bf16 terms, no scaling.
   const bool bf = p.wdt == WR_BF16 || p.wdt == WR_MXFP4;
-  hipError_t err = launch_logits_split(p, w.logits, w.x_hi, w.x_lo, w.x_exp,
-                                       bf ? nullptr : w.amax, bf ? 1 : 0, s);
+  XSplit xs = x_split(p);
+  xs.hi = w.x_hi;
+  xs.lo = w.x_lo;
+  xs.l2 = ragged && p.adt == WR_F32 ? w.x_l2() : nullptr;
+  xs.exp = w.x_exp;
+  xs.amax = bf ? nullptr : w.amax;
+  xs.bf16 = bf ? 1 : 0;
+  xs.ld = ragged ? BatchWs::padded(p.h) : p.h;
+  hipError_t err = launch_logits_split(p, w.logits, xs, s);
   if (err != hipSuccess) return err;
+  if (ragged) {
+    if (p.wdt == WR_FP8_E4M3)
+      return p.adt == WR_F16 ? ragged_t<fp8w, f16>(p, w, s) : ragged_t<fp8w, float>(p, w, s);
+    if (p.wdt == WR_BF16)
+      return p.adt == WR_F16 ? ragged_t<bf16w, f16>(p, w, s) : ragged_t<bf16w, float>(p, w, s);
+    if (p.wdt == WR_MXFP4)
+      return p.adt == WR_F16 ? ragged_t<fp4x2, f16>(p, w, s) : ragged_t<fp4x2, float>(p, w, s);
+    return p.adt == WR_F16 ? ragged_t<f16, f16>(p, w, s) : ragged_t<f16, float>(p, w, s);
+  }
   if (p.wdt == WR_FP8_E4M3)
     return p.adt == WR_F16 ? grouped_t<fp8w, f16>(p, w, s) : grouped_t<fp8w, float>(p, w, s);
   if (p.wdt == WR_BF16)

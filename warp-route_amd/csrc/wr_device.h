@@ -431,6 +431,20 @@ __device__ __forceinline__ typename WVec<T, VEC>::type load_wq(const T* p, const
   }
 }
 
+// 16 bytes at any address (global loads take any alignment on this target).
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(1)));
+// load_wq at any address.
+template <typename T, int VEC>
+__device__ __forceinline__ typename WVec<T, VEC>::type load_wq_u(const T* p, const uint8_t* sc) {
+  const u32x4 q = __builtin_nontemporal_load(reinterpret_cast<const u32x4u*>(p));
+  if constexpr (std::is_same<T, fp4x2>::value) {
+    return fp4v32{q, *sc};
+  } else {
+    (void)sc;
+    return __builtin_bit_cast(typename WVec<T, VEC>::type, q);
+  }
+}
+
 template <typename V>
 __device__ __forceinline__ float velem(const V& v, int i) {
   if constexpr (std::is_same<V, f16>::value || std::is_same<V, float>::value) {
@@ -534,6 +548,22 @@ __device__ __forceinline__ void load_x(const XT* __restrict__ p, float (&v)[VEC]
   } else {
 #pragma unroll
     for (int i = 0; i < VEC; ++i) v[i] = (float)p[i];
+  }
+}
+
+// load_x at any address; VEC elements are whole 16-byte pieces (fp32), or one
+// or more 8-byte ones (fp16).
+template <typename XT, int VEC>
+__device__ __forceinline__ void load_x_u(const XT* __restrict__ p, float (&v)[VEC]) {
+  constexpr int N = VEC * (int)sizeof(XT) / 16 > 0 ? 16 / (int)sizeof(XT) : VEC;
+  typedef XT xv __attribute__((ext_vector_type(N)));
+  typedef XT xu __attribute__((ext_vector_type(N), aligned(1)));
+  static_assert(VEC % N == 0, "whole pieces");
+#pragma unroll
+  for (int q = 0; q < VEC / N; ++q) {
+    const xv t = *reinterpret_cast<const xu*>(p + N * q);
+#pragma unroll
+    for (int i = 0; i < N; ++i) v[N * q + i] = (float)t[i];
   }
 }
 

@@ -139,6 +139,14 @@ struct BatchWs {
   BatchRoute route;
   float* act;    // [P][I], grouped pair order, scaled by the gate weight
   float* ypart;  // [kKSplit][P][h]: down partial sums
+  // Row lengths of ragged layers (h or I not whole K steps): x and act rows are
+  // zero past h and I, the partial sums' tails unused.
+  static constexpr int padded(int n) { return (n + 127) / 128 * 128; }
+  // Ragged layers: third bf16 terms of x, in the partial sums' bytes (which the
+  // down kernel writes after the gate/up kernel has read them); x in fp32, in
+  // the two terms' bytes (adjacent: padded rows are whole 256-byte units).
+  _Float16* x_l2() const { return reinterpret_cast<_Float16*>(ypart); }
+  float* x_f32() const { return reinterpret_cast<float*>(x_hi); }
   static size_t bytes(int E, int h, int I, int k, int B) {
     size_t n = 0;
     carve_into(nullptr, &n, E, h, I, k, B);
@@ -158,6 +166,8 @@ struct BatchWs {
       return p;
     };
     const size_t P = (size_t)B * k;
+    h = padded(h);
+    I = padded(I);
     w.logits = reinterpret_cast<float*>(take((size_t)B * WR_MAX_EXPERTS * 4));
     w.x_hi = reinterpret_cast<_Float16*>(take((size_t)B * h * 2));
     w.x_lo = reinterpret_cast<_Float16*>(take((size_t)B * h * 2));
@@ -205,12 +215,31 @@ struct NaiveWs {
 // Launchers (wr_kernels.hip, wr_naive.hip).  Each returns the first HIP
 // error it meets.
 hipError_t launch_logits(const Problem& p, float* logits, hipStream_t s);
-// Logits, plus x split into two 16-bit terms for the grouped batched path:
-// bf16 terms x = hi + lo when split_bf16, else fp16 terms
-// x 2^x_exp[b] = hi + lo (lo = 0 for fp16 x); also zeroes amax (k words per
-// token, BatchWs::kAmaxStride apart) when it is not NULL.
-hipError_t launch_logits_split(const Problem& p, float* logits, _Float16* x_hi, _Float16* x_lo,
-                               int32_t* x_exp, unsigned* amax, int split_bf16, hipStream_t s);
+// What the router launch writes of x for the grouped batched path, rows ld
+// elements apart and zero from column h on.  hi set: x in 16-bit terms, bf16
+// terms x = hi + lo (+ l2, when set) with bf16, else fp16 terms
+// x 2^e = hi + lo, e = split_exp(max|x|), exp[b] = e (bf16 keeps fp32's
+// exponent range, so no scaling).  f32 set: x in fp32.  amax (when set) gets
+// its k words of token b zeroed, BatchWs::kAmaxStride apart.
+struct XSplit {
+  _Float16* hi;
+  _Float16* lo;
+  _Float16* l2;
+  float* f32;
+  int32_t* exp;
+  unsigned* amax;
+  int k;
+  int bf16;
+  int ld;
+};
+inline XSplit x_split(const Problem& p) {
+  XSplit xs{};
+  xs.k = p.k;
+  xs.ld = p.h;
+  return xs;
+}
+// Logits and, with them, x as xs asks.
+hipError_t launch_logits_split(const Problem& p, float* logits, const XSplit& xs, hipStream_t s);
 // Grouped batched path: usable when grouped_ok(p).
 bool grouped_ok(const Problem& p);
 hipError_t launch_grouped(const Problem& p, hipStream_t s);

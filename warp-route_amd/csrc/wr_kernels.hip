@@ -202,25 +202,11 @@ __device__ __forceinline__ float router_combine(const float* p) {
   return (p[0] + p[1]) + (p[2] + p[3]);
 }
 
-// x split into two 16-bit terms for the grouped batched path.  hi == NULL:
-// no split.  bf16: bf16 terms x = hi + lo (bf16 keeps fp32's exponent range,
-// so no scaling).  Otherwise fp16 terms of x 2^e, e = split_exp(max|x|), and
-// exp[b] = e; amax (when not NULL) gets its k words of token b zeroed, every
-// kAmaxStride words.
-struct XSplit {
-  f16* hi;
-  f16* lo;
-  int32_t* exp;
-  unsigned* amax;
-  int k;
-  int bf16;
-};
-
 // grid (E, B), block 256.  Token b's logits go to logits[b * 64 + e] (padded
 // so that consumers can read all 64 with scalar loads).  Block (0, 0) also
 // zeroes the 8-byte words at zero + i * zstride, i < nzero <= kBlock (the
 // single-token kernel's arrival words, timeout flag and claim counters),
-// which the next kernel on the stream reads.  With xs.hi != NULL,
+// which the next kernel on the stream reads.  With xs.hi or xs.f32 set,
 // block (e, b) also writes its 1/E
 // share of token b's split x (XSplit); every block of the token derives the
 // same exponent from the whole row.
@@ -246,25 +232,32 @@ __global__ __launch_bounds__(kBlock) void k_router_logits(const float* __restric
     *reinterpret_cast<uint64_t*>(zero + (int64_t)threadIdx.x * zstride) = 0ull;
   __syncthreads();
   if (threadIdx.x == 0) logits[(int64_t)b * WR_MAX_EXPERTS + e] = router_combine(part);
-  if (xs.hi != nullptr) {
+  if (xs.hi != nullptr || xs.f32 != nullptr) {
     const XT* xb = x + (int64_t)b * h;
     const int ex = scaled ? split_exp(fmaxf(fmaxf(pmax[0], pmax[1]), fmaxf(pmax[2], pmax[3])),
                                       std::is_same<XT, f16>::value)
                           : 0;
-    const int cs = (h + E - 1) / E;
-    const int end = min(h, (e + 1) * cs);
+    const int cs = (xs.ld + E - 1) / E;
+    const int end = min(xs.ld, (e + 1) * cs);
     for (int i = e * cs + (int)threadIdx.x; i < end; i += kBlock) {
-      const float v = (float)xb[i];
+      const float v = i < h ? (float)xb[i] : 0.0f;
+      const int64_t o = (int64_t)b * xs.ld + i;
       if (xs.bf16) {
         const __bf16 bh = (__bf16)v;
         const __bf16 bl = (__bf16)(v - (float)bh);
-        xs.hi[(int64_t)b * h + i] = __builtin_bit_cast(f16, bh);
-        xs.lo[(int64_t)b * h + i] = __builtin_bit_cast(f16, bl);
+        xs.hi[o] = __builtin_bit_cast(f16, bh);
+        xs.lo[o] = __builtin_bit_cast(f16, bl);
+        if (xs.l2 != nullptr)
+          xs.l2[o] = __builtin_bit_cast(f16, (__bf16)(v - (float)bh - (float)bl));
+      } else if (xs.f32 != nullptr) {
+        xs.f32[o] = v;
       } else {
         const float vs = ldexpf(v, ex);
         const f16 vh = (f16)vs;
-        xs.hi[(int64_t)b * h + i] = vh;
-        xs.lo[(int64_t)b * h + i] = (f16)(vs - (float)vh);
+        const f16 vl = (f16)(vs - (float)vh);
+        xs.hi[o] = vh;
+        xs.lo[o] = vl;
+        if (xs.l2 != nullptr) xs.l2[o] = (f16)(vs - (float)vh - (float)vl);
       }
     }
     if (e == 0) {
@@ -331,6 +324,63 @@ __device__ __forceinline__ const uint8_t* mx_at(const uint8_t* row, int64_t c) {
   else return nullptr;
 }
 
+// Ragged rows (RAG; K = the row length, at least VEC; rows at any address): the
+// piece of lane l in the chunk at column c - l VEC is loaded from column
+// rag_col = min(c, K - VEC), unaligned and always in bounds, weights and
+// activations alike; in the chunk that holds the row's end, rag_mask keeps the
+// columns from c on (the others belong to lower lanes), and none for c >= K.
+template <int VEC>
+__device__ __forceinline__ int rag_col(int c, int K) {
+  return min(c, K - VEC);
+}
+template <int VEC>
+__device__ __forceinline__ bool rag_last(int c, int K, int lane) {  // wave-uniform
+  return c + (kWave - lane) * VEC > K;
+}
+template <int VEC>
+__device__ __forceinline__ u32x4 rag_mask(int c, int K) {
+  const int d = c - (K - VEC);  // columns of the piece that are not this lane's
+  typedef unsigned __int128 u128;
+  const u128 m = d >= VEC ? u128(0) : ~u128(0) << (max(d, 0) * (128 / VEC));
+  return __builtin_bit_cast(u32x4, m);
+}
+template <typename V>
+__device__ __forceinline__ void rag_keep(V& v, const u32x4& m) {
+  if constexpr (std::is_same<V, fp4v32>::value) {  // rows are whole pieces
+    v.q &= m;
+    if (m[0] == 0u) v.e = 127u;
+  } else {
+    v = __builtin_bit_cast(V, __builtin_bit_cast(u32x4, v) & m);
+  }
+}
+template <int VEC>
+__device__ __forceinline__ void rag_keep_x(float (&v)[VEC], int c, int K) {
+  const int d = c - (K - VEC);
+#pragma unroll
+  for (int i = 0; i < VEC; ++i) v[i] = i < d ? 0.0f : v[i];
+}
+// A weight piece at column c of the row at `row` (load_wq), ragged or not; sc
+// is the row's first block scale.
+template <typename WT, int VEC, bool RAG>
+__device__ __forceinline__ typename WVec<WT, VEC>::type load_row(const WT* row, const uint8_t* sc,
+                                                                 int c, int K) {
+  if constexpr (!RAG) {
+    return load_wq<WT, VEC>(row + eoff<WT>(c), mx_at<WT>(sc, c));
+  } else {
+    const int cc = rag_col<VEC>(c, K);
+    return load_wq_u<WT, VEC>(row + eoff<WT>(cc), mx_at<WT>(sc, cc));
+  }
+}
+// VEC activation values at column c of the row at p.
+template <typename XT, int VEC, bool RAG>
+__device__ __forceinline__ void load_x_row(const XT* __restrict__ p, int c, int K,
+                                           float (&v)[VEC]) {
+  if constexpr (!RAG)
+    load_x<XT, VEC>(p + c, v);
+  else
+    load_x_u<XT, VEC>(p + rag_col<VEC>(c, K), v);
+}
+
 // act for intermediate index r of the expert block at blk, from the gate and
 // up dot products gs and us and the gate weight wk:
 //   wk * silu(gs) * us                                  (unscaled types)
@@ -380,7 +430,7 @@ __device__ __forceinline__ float down_scale(const WT* wbuf, const Geom& g, const
 // share(k * ceil(I / RPW), w, nw); item it covers rows [r0, r0 + RPW) of
 // selected expert kk = it / ceil(I / RPW).
 // ---------------------------------------------------------------------------
-template <typename WT, typename XT, int VEC, int RPW, int U>
+template <typename WT, typename XT, int VEC, int RPW, int U, bool RAG>
 __global__ __launch_bounds__(kBlock) void k_gateup(const WT* __restrict__ wbuf,
                                                    const XT* __restrict__ x,
                                                    const float* __restrict__ logits,
@@ -435,18 +485,33 @@ __global__ __launch_bounds__(kBlock) void k_gateup(const WT* __restrict__ wbuf,
 #pragma unroll
         for (int j = 0; j < RPW; ++j) {
           const bool okj = ok && j < nrows;
-          wg[u][j] = okj ? load_wq<WT, VEC>(G + eoff<WT>((int64_t)j * g.h + c),
-                                            mx_at<WT>(mx_row(blk, g, 0, r0 + j), c))
+          wg[u][j] = okj ? load_row<WT, VEC, RAG>(G + eoff<WT>((int64_t)j * g.h),
+                                                  mx_row(blk, g, 0, r0 + j), c, g.h)
                          : vzero<V>();
-          wu[u][j] = okj ? load_wq<WT, VEC>(Up + eoff<WT>((int64_t)j * g.h + c),
-                                            mx_at<WT>(mx_row(blk, g, 1, r0 + j), c))
+          wu[u][j] = okj ? load_row<WT, VEC, RAG>(Up + eoff<WT>((int64_t)j * g.h),
+                                                  mx_row(blk, g, 1, r0 + j), c, g.h)
                          : vzero<V>();
         }
         if (ok) {
-          load_x<XT, VEC>(xb + c, xv[u]);
+          load_x_row<XT, VEC, RAG>(xb, c, g.h, xv[u]);
         } else {
 #pragma unroll
           for (int i = 0; i < VEC; ++i) xv[u][i] = 0.0f;
+        }
+      }
+      if constexpr (RAG) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int c = c0 + u * CH;
+          if (rag_last<VEC>(c, g.h, lane)) {
+            const u32x4 m = rag_mask<VEC>(c, g.h);
+            rag_keep_x<VEC>(xv[u], c, g.h);
+#pragma unroll
+            for (int j = 0; j < RPW; ++j) {
+              rag_keep(wg[u][j], m);
+              rag_keep(wu[u][j], m);
+            }
+          }
         }
       }
 #pragma unroll
@@ -476,7 +541,7 @@ __global__ __launch_bounds__(kBlock) void k_gateup(const WT* __restrict__ wbuf,
 // share(ceil(h / RPD), w, nw); for each it streams rows [r0, r0 + RPD) of
 // every selected down matrix against that expert's act vector.
 // ---------------------------------------------------------------------------
-template <typename WT, typename OT, int VEC, int RPD, int U>
+template <typename WT, typename OT, int VEC, int RPD, int U, bool RAG>
 __global__ __launch_bounds__(kBlock) void k_down(const WT* __restrict__ wbuf,
                                                  const float* __restrict__ logits,
                                                  const float* __restrict__ act,
@@ -521,14 +586,26 @@ __global__ __launch_bounds__(kBlock) void k_down(const WT* __restrict__ wbuf,
 #pragma unroll
           for (int j = 0; j < RPD; ++j)
             wv[u][j] = (ok && j < nrows)
-                           ? load_wq<WT, VEC>(D + eoff<WT>((int64_t)j * g.I + c),
-                                              mx_at<WT>(mx_row(blk, g, 2, r0 + j), c))
+                           ? load_row<WT, VEC, RAG>(D + eoff<WT>((int64_t)j * g.I),
+                                                    mx_row(blk, g, 2, r0 + j), c, g.I)
                            : vzero<V>();
           if (ok) {
-            load_x<float, VEC>(a + c, av[u]);
+            load_x_row<float, VEC, RAG>(a, c, g.I, av[u]);
           } else {
 #pragma unroll
             for (int i = 0; i < VEC; ++i) av[u][i] = 0.0f;
+          }
+        }
+        if constexpr (RAG) {
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            const int c = c0 + u * CH;
+            if (rag_last<VEC>(c, g.I, lane)) {
+              const u32x4 m = rag_mask<VEC>(c, g.I);
+              rag_keep_x<VEC>(av[u], c, g.I);
+#pragma unroll
+              for (int j = 0; j < RPD; ++j) rag_keep(wv[u][j], m);
+            }
           }
         }
 #pragma unroll
@@ -780,7 +857,7 @@ __host__ __device__ __forceinline__ int chunk_of_block(int b) {
 
 // Rows [r0, r0 + RPW) of selected expert kk's gate/up matrices; the results go
 // to a[0 .. RPW) with agent-scope stores.
-template <typename WT, typename XT, int VEC, int RPW, int U>
+template <typename WT, typename XT, int VEC, int RPW, int U, bool RAG>
 __device__ __forceinline__ void gateup_item(const WT* __restrict__ wbuf, const XT* __restrict__ xb,
                                             float* a, const Geom& g, const TopK& t, int kk,
                                             int r0, int lane, const Handoff* hsp = nullptr) {
@@ -806,18 +883,33 @@ __device__ __forceinline__ void gateup_item(const WT* __restrict__ wbuf, const X
 #pragma unroll
       for (int j = 0; j < RPW; ++j) {
         const bool okj = ok && j < nrows;
-        wg[u][j] = okj ? load_wq<WT, VEC>(G + eoff<WT>((int64_t)j * g.h + c),
-                                          mx_at<WT>(mx_row(blk, g, 0, r0 + j), c))
+        wg[u][j] = okj ? load_row<WT, VEC, RAG>(G + eoff<WT>((int64_t)j * g.h),
+                                                mx_row(blk, g, 0, r0 + j), c, g.h)
                        : vzero<V>();
-        wu[u][j] = okj ? load_wq<WT, VEC>(Up + eoff<WT>((int64_t)j * g.h + c),
-                                          mx_at<WT>(mx_row(blk, g, 1, r0 + j), c))
+        wu[u][j] = okj ? load_row<WT, VEC, RAG>(Up + eoff<WT>((int64_t)j * g.h),
+                                                mx_row(blk, g, 1, r0 + j), c, g.h)
                        : vzero<V>();
       }
       if (ok) {
-        load_x<XT, VEC>(xb + c, xv[u]);
+        load_x_row<XT, VEC, RAG>(xb, c, g.h, xv[u]);
       } else {
 #pragma unroll
         for (int i = 0; i < VEC; ++i) xv[u][i] = 0.0f;
+      }
+    }
+    if constexpr (RAG) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int c = c0 + u * CH;
+        if (rag_last<VEC>(c, g.h, lane)) {
+          const u32x4 m = rag_mask<VEC>(c, g.h);
+          rag_keep_x<VEC>(xv[u], c, g.h);
+#pragma unroll
+          for (int j = 0; j < RPW; ++j) {
+            rag_keep(wg[u][j], m);
+            rag_keep(wu[u][j], m);
+          }
+        }
       }
     }
 #pragma unroll
@@ -1068,7 +1160,7 @@ __device__ __forceinline__ void gateup_item_xl(const WT* __restrict__ wbuf,
 // Down tile of a fused down block: U column chunks q = q0 + 4 u (chunk q is
 // columns [(q mod nch) * 64 VEC, +64 VEC) of selected expert q / nch), RPD rows
 // from r0.
-template <typename WT, int VEC, int RPD, int U, bool STG = false>
+template <typename WT, int VEC, int RPD, int U, bool STG = false, bool RAG = false>
 __device__ __forceinline__ void down_tile_load(typename WVec<WT, VEC>::type (&wv)[U][RPD],
                                                const WT* __restrict__ wbuf, const Geom& g,
                                                const TopK& t, int r0, int nrows, int q0,
@@ -1083,6 +1175,15 @@ __device__ __forceinline__ void down_tile_load(typename WVec<WT, VEC>::type (&wv
     const int c = (q - kk * nch) * kWave * VEC + lane * VEC;
     const bool ok = okq && c < g.I;
     const WT* blk = wbuf + (int64_t)topk_id(t, kk) * g.stride;
+    if constexpr (RAG) {
+      const WT* row = blk + g.off_down + eoff<WT>((int64_t)r0 * g.I);
+#pragma unroll
+      for (int j = 0; j < RPD; ++j)
+        wv[u][j] = (ok && j < nrows) ? load_row<WT, VEC, true>(row + eoff<WT>((int64_t)j * g.I),
+                                                               mx_row(blk, g, 2, r0 + j), c, g.I)
+                                     : vzero<V>();
+      continue;
+    }
     const WT* D = blk + g.off_down + eoff<WT>((int64_t)r0 * g.I + c);
 #pragma unroll
     for (int j = 0; j < RPD; ++j)
@@ -1118,8 +1219,10 @@ __device__ __forceinline__ void down_tile_scales(typename WVec<WT, VEC>::type (&
 // acc[j] += tile row j . act over the tile's chunks (act of expert kk at
 // act + kk * act_row).  fp8: each chunk's products are summed apart and
 // added times the row scale of the chunk's expert, sdn[kk * RPD + j].
-template <typename WT, typename V, int VEC, int RPD, int U>
-__device__ __forceinline__ void down_tile_fma(float (&acc)[RPD], const V (&wv)[U][RPD],
+// RAG: the tile as loaded; the chunk that ends the row is masked here.
+template <typename WT, typename V, int VEC, int RPD, int U, bool RAG = false>
+__device__ __forceinline__ void down_tile_fma(float (&acc)[RPD],
+                                              std::conditional_t<RAG, V, const V> (&wv)[U][RPD],
                                               const float* act, const Geom& g,
                                               int64_t act_row, int q0, int nch, int lane,
                                               const float* sdn) {
@@ -1131,10 +1234,24 @@ __device__ __forceinline__ void down_tile_fma(float (&acc)[RPD], const V (&wv)[U
     const int kk = q / nch;
     const int c = (q - kk * nch) * kWave * VEC + lane * VEC;
     if (q < C && c < g.I) {
-      load_x<float, VEC>(act + kk * act_row + c, av[u]);
+      load_x_row<float, VEC, RAG>(act + kk * act_row, c, g.I, av[u]);
     } else {
 #pragma unroll
       for (int i = 0; i < VEC; ++i) av[u][i] = 0.0f;
+    }
+  }
+  if constexpr (RAG) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = q0 + u * kWavesPerBlock;
+      const int kk = q / nch;
+      const int c = (q - kk * nch) * kWave * VEC + lane * VEC;
+      if (q < C && rag_last<VEC>(c, g.I, lane)) {  // wave-uniform
+        const u32x4 m = rag_mask<VEC>(c, g.I);
+        rag_keep_x<VEC>(av[u], c, g.I);
+#pragma unroll
+        for (int j = 0; j < RPD; ++j) rag_keep(wv[u][j], m);
+      }
     }
   }
   if constexpr (std::is_same<WT, fp8w>::value) {
@@ -1178,6 +1295,19 @@ constexpr size_t fused_raw_bytes() {
   }
 }
 
+template <typename XT>
+struct Ragged {};
+template <typename XA>
+struct XArg {
+  typedef XA type;
+  static constexpr bool kRagged = false;
+};
+template <typename XT>
+struct XArg<Ragged<XT>> {
+  typedef XT type;
+  static constexpr bool kRagged = true;
+};
+
 // WR_TIMELINE builds hold the claiming variant to 4 blocks per CU, the
 // occupancy its default build has, so that the timeline shows the launch
 // configuration the default build runs.
@@ -1186,12 +1316,17 @@ constexpr size_t fused_raw_bytes() {
 #else
 #define WR_FUSED_BOUNDS __launch_bounds__(kBlock)
 #endif
-template <typename WT, typename XT, int VEC, int RPW, int U1, int RPD, int U2, bool XL,
+// XA: x's and out's type XT, or Ragged<XT> for rows that are not whole, aligned
+// VEC-element pieces (load_row; the plain register path only).
+template <typename WT, typename XA, int VEC, int RPW, int U1, int RPD, int U2, bool XL,
           bool STG, bool CLAIM = false, bool ROUTE = false>
 __global__ WR_FUSED_BOUNDS void k_fused_ffn(
-    const WT* __restrict__ wbuf, const XT* __restrict__ x, const float* __restrict__ logits,
-    float* act, XT* __restrict__ out, int32_t* __restrict__ ids_out, float* __restrict__ w_out,
-    Geom g, Handoff hs) {
+    const WT* __restrict__ wbuf, const typename XArg<XA>::type* __restrict__ x,
+    const float* __restrict__ logits, float* act, typename XArg<XA>::type* __restrict__ out,
+    int32_t* __restrict__ ids_out, float* __restrict__ w_out, Geom g, Handoff hs) {
+  typedef typename XArg<XA>::type XT;
+  constexpr bool RAG = XArg<XA>::kRagged;
+  static_assert(!RAG || !(XL || STG || CLAIM || ROUTE), "ragged rows take the plain register path");
   typedef typename WVec<WT, VEC>::type V;
   constexpr int COLS = kWavesPerBlock * RPW;  // act columns per gate/up block
   constexpr int LB = 32 / COLS;               // chunks per 128-byte act line
@@ -1262,8 +1397,8 @@ __global__ WR_FUSED_BOUNDS void k_fused_ffn(
         const int kk = G / bpk;
         const int it = (G - kk * bpk) * kWavesPerBlock + wave;
         if (it < items)
-          gateup_item<WT, XT, VEC, RPW, U1>(wbuf, x, act + kk * act_row + it * RPW, g, t, kk,
-                                            it * RPW, lane, &hs);
+          gateup_item<WT, XT, VEC, RPW, U1, RAG>(wbuf, x, act + kk * act_row + it * RPW, g, t, kk,
+                                                 it * RPW, lane, &hs);
       }
       __builtin_amdgcn_s_waitcnt(0);  // this wave's act stores have completed
       __syncthreads();
@@ -1313,13 +1448,13 @@ __global__ WR_FUSED_BOUNDS void k_fused_ffn(
                       lds_raw + (size_t)kk * RPD * ib, nrows * ib, lane);
   }
   V pre[U2][RPD];
-  down_tile_load<WT, VEC, RPD, U2, STG>(pre, wbuf, g, t, r0, nrows, wave, nch, lane);
+  down_tile_load<WT, VEC, RPD, U2, STG, RAG>(pre, wbuf, g, t, r0, nrows, wave, nch, lane);
   // The next PRE chunks of this wave (after the U2 in registers) go to LDS:
   // the tail after the hand-off then has one dependent load round fewer, and
   // those bytes stream during the end of the gate/up phase.  Slot (v, j)
   // holds row j of chunk wave + 4 (U2 + v), lane l's 16 bytes at 16 l.
   // Register-path kernels only: the x-in-LDS variant's copy takes the LDS.
-  constexpr int PRE = (!XL && sizeof(V) == 16) ? WR_DN_LDS_ROWCHUNKS / RPD : 0;
+  constexpr int PRE = (!XL && !RAG && sizeof(V) == 16) ? WR_DN_LDS_ROWCHUNKS / RPD : 0;
   constexpr int kPreBytes = kWavesPerBlock * PRE * RPD * kWave * 16;
   __shared__ __align__(16) unsigned char dpre[kPreBytes > 0 ? kPreBytes : 16];
   const int wu = __builtin_amdgcn_readfirstlane(wave);
@@ -1451,7 +1586,7 @@ __global__ WR_FUSED_BOUNDS void k_fused_ffn(
 #pragma unroll
   for (int j = 0; j < RPD; ++j) acc[j] = 0.0f;
   if constexpr (STG) down_tile_scales<WT, VEC, RPD, U2>(pre, lds_raw, g, nrows, wave, nch, lane);
-  down_tile_fma<WT, V, VEC, RPD, U2>(acc, pre, act, g, act_row, wave, nch, lane, sdn);
+  down_tile_fma<WT, V, VEC, RPD, U2, RAG>(acc, pre, act, g, act_row, wave, nch, lane, sdn);
   if constexpr (PRE > 0) {
     __builtin_amdgcn_s_waitcnt(0);  // this wave's global-to-LDS loads have landed
     asm volatile("" ::: "memory");
@@ -1492,9 +1627,9 @@ __global__ WR_FUSED_BOUNDS void k_fused_ffn(
   }
   for (int q0 = wave + kWavesPerBlock * (U2 + PRE + spre); q0 < C; q0 += kWavesPerBlock * U2) {
     V wv[U2][RPD];
-    down_tile_load<WT, VEC, RPD, U2, STG>(wv, wbuf, g, t, r0, nrows, q0, nch, lane);
+    down_tile_load<WT, VEC, RPD, U2, STG, RAG>(wv, wbuf, g, t, r0, nrows, q0, nch, lane);
     if constexpr (STG) down_tile_scales<WT, VEC, RPD, U2>(wv, lds_raw, g, nrows, q0, nch, lane);
-    down_tile_fma<WT, V, VEC, RPD, U2>(acc, wv, act, g, act_row, q0, nch, lane, sdn);
+    down_tile_fma<WT, V, VEC, RPD, U2, RAG>(acc, wv, act, g, act_row, q0, nch, lane, sdn);
   }
 #pragma unroll
   for (int j = 0; j < RPD; ++j) {
@@ -1567,7 +1702,7 @@ bool router_vec4(const Problem& p) {
 
 template <typename XT>
 hipError_t logits_t(const Problem& p, float* logits, unsigned* zero, int nzero, int zstride,
-                    hipStream_t s, XSplit xs = XSplit{nullptr, nullptr, nullptr, nullptr, 0, 0}) {
+                    hipStream_t s, XSplit xs = XSplit{}) {
   const dim3 grid(p.E, p.B);
   const XT* x = static_cast<const XT*>(p.x);
   if (router_vec4(p))
@@ -1586,11 +1721,11 @@ hipError_t logits_t(const Problem& p, float* logits, unsigned* zero, int nzero, 
 // instead of two dependent ones (DeepSeek's 4 KB rows: 31.3 -> 28.0 us).
 // fp8 rows always take 4: four chunks of 16 fp32 x values per lane would
 // cost 64 VGPRs and a wave per SIMD.
-int fused_rpw(const Problem& p) {
+int fused_rpw(const Problem& p, bool pieces) {
   const int64_t row_bytes = (int64_t)p.h * weight_es(p.wdt);
-  if (p.wdt == WR_FP8_E4M3) return p.vec > 1 ? WR_F8_RPW : 2;
-  if (p.wdt == WR_MXFP4) return p.vec == 32 ? 4 : 2;
-  return (p.vec > 1 && row_bytes <= 2048) ? 4 : 2;
+  if (p.wdt == WR_FP8_E4M3) return pieces ? WR_F8_RPW : 2;
+  if (p.wdt == WR_MXFP4) return 4;
+  return (pieces && row_bytes <= 2048) ? 4 : 2;
 }
 
 // act chunks of the single-token fused kernel, and its gate/up blocks (the
@@ -1672,7 +1807,7 @@ constexpr int kFoldSlotsPerCu = 2;
 // in the workspace.  Otherwise a request to compute the router rows inside
 // the kernel (one launch per layer): *fold tells whether this shape's variant
 // did, and if not nothing was launched.
-template <typename WT, typename XT, int VEC, int RPW, int U1>
+template <typename WT, typename XT, int VEC, int RPW, int U1, bool RAG>
 hipError_t fused_rpw_t(const Problem& p, const FusedWs& w, bool* fold, hipStream_t s) {
   const Geom g = make_geom(p);
   Handoff hs;
@@ -1702,6 +1837,18 @@ hipError_t fused_rpw_t(const Problem& p, const FusedWs& w, bool* fold, hipStream
   constexpr int RPD = kFp4 ? WR_F4_RPD : (kFp8 ? WR_F8_RPD : WR_FU_RPD);
   constexpr int U2 = kFp4 ? WR_F4_U2 : (kFp8 ? WR_F8_U2 : WR_FU_U);
   const int n2 = (p.h + RPD - 1) / RPD;
+  if constexpr (RAG) {
+    if (fold != nullptr) {  // ragged layers keep the router launch
+      *fold = false;
+      return hipSuccess;
+    }
+    hs.nb = hs.n1 + n2;
+    WR_TL_GRID(hs.nb);
+    hipLaunchKernelGGL((k_fused_ffn<WT, Ragged<XT>, VEC, RPW, U1, RPD, U2, false, false>), dim3(hs.nb), dim3(kBlock),
+                       0, s, static_cast<const WT*>(p.wbuf), static_cast<const XT*>(p.x), w.logits,
+                       w.act, static_cast<XT*>(p.out), p.topk_ids, p.topk_w, g, hs);
+    return hipGetLastError();
+  } else {
   // Gate/up blocks read x from an LDS copy for small enough h (and, except
   // for MXFP4, few enough gate/up blocks).
   constexpr int kXlMax = xl_max_h<WT>();
@@ -1807,6 +1954,7 @@ hipError_t fused_rpw_t(const Problem& p, const FusedWs& w, bool* fold, hipStream
                        p.topk_ids, p.topk_w, g, hs);
     return hipGetLastError();
   }
+  }
 }
 
 // Column chunks in flight per gate/up row: fp8 WR_F8_U1, MXFP4 one (32 x
@@ -1843,49 +1991,75 @@ bool f4_whole_rows(const Problem& p) {
   }
 }
 
-template <typename WT, typename XT, int VEC>
+template <typename WT, typename XT, int VEC, bool RAG>
 hipError_t fused_t(const Problem& p, const FusedWs& w, bool* fold, hipStream_t s) {
-  if (fused_rpw(p) == 4) {
-    if constexpr (std::is_same<WT, fp4x2>::value && VEC == 32) {
-      if (f4_whole_rows<WT, XT, VEC>(p)) return fused_rpw_t<WT, XT, VEC, 4, 2>(p, w, fold, s);
+  if constexpr (VEC > 1) {
+    if (fused_rpw(p, true) == 4) {
+      if constexpr (std::is_same<WT, fp4x2>::value && !RAG) {
+        if (f4_whole_rows<WT, XT, VEC>(p))
+          return fused_rpw_t<WT, XT, VEC, 4, 2, false>(p, w, fold, s);
+      }
+      return fused_rpw_t<WT, XT, VEC, 4, fused_u1<WT, 4>(), RAG>(p, w, fold, s);
     }
-    return fused_rpw_t<WT, XT, VEC, 4, fused_u1<WT, 4>()>(p, w, fold, s);
   }
-  return fused_rpw_t<WT, XT, VEC, 2, fused_u1<WT, 2>()>(p, w, fold, s);
+  if constexpr (std::is_same<WT, fp4x2>::value && RAG)
+    return hipErrorInvalidValue;  // MXFP4 rows always take 4 (fused_rpw)
+  else
+    return fused_rpw_t<WT, XT, VEC, 2, fused_u1<WT, 2>(), RAG>(p, w, fold, s);
 }
 
-template <typename WT, typename XT, int VEC>
-hipError_t ffn_t(const Problem& p, const FusedWs& w, bool* fold, hipStream_t s) {
+// Several tokens, one grid row each.
+template <typename WT, typename XT, int VEC, bool RAG>
+hipError_t per_token_t(const Problem& p, const FusedWs& w, hipStream_t s) {
   constexpr int RPW = WR_GU_RPW, RPD = WR_DN_RPD;
   // fp8: half the chunks in flight (16 fp32 x values per chunk and lane);
   // MXFP4: one chunk (32 values), and one chunk per down tile.
   constexpr bool kFp4 = std::is_same<WT, fp4x2>::value;
   constexpr int U1 = kFp4 ? 1 : (std::is_same<WT, fp8w>::value ? WR_GU_U / 2 : WR_GU_U);
   constexpr int UD = kFp4 ? 1 : WR_DN_U;
-  if (p.B == 1) return fused_t<WT, XT, VEC>(p, w, fold, s);
-  if (fold != nullptr) {  // several tokens: the router runs in its own launch
-    *fold = false;
-    return hipSuccess;
-  }
   const Geom g = make_geom(p);
   const WT* wb = static_cast<const WT*>(p.wbuf);
   const int nw1 = waves_for(p.k * ((p.I + RPW - 1) / RPW), p.B);
   const dim3 g1((nw1 + kWavesPerBlock - 1) / kWavesPerBlock, p.B);
-  hipLaunchKernelGGL((k_gateup<WT, XT, VEC, RPW, U1>), g1, dim3(kBlock), 0, s, wb,
+  hipLaunchKernelGGL((k_gateup<WT, XT, VEC, RPW, U1, RAG>), g1, dim3(kBlock), 0, s, wb,
                      static_cast<const XT*>(p.x), w.logits, w.act, p.topk_ids, p.topk_w, g, nw1);
   hipError_t err = hipGetLastError();
   if (err != hipSuccess) return err;
   const int nw2 = waves_for((p.h + RPD - 1) / RPD, p.B);
   const dim3 g2((nw2 + kWavesPerBlock - 1) / kWavesPerBlock, p.B);
-  hipLaunchKernelGGL((k_down<WT, XT, VEC, RPD, UD>), g2, dim3(kBlock), 0, s, wb, w.logits,
+  hipLaunchKernelGGL((k_down<WT, XT, VEC, RPD, UD, RAG>), g2, dim3(kBlock), 0, s, wb, w.logits,
                      w.act, static_cast<XT*>(p.out), g, nw2);
   return hipGetLastError();
 }
 
+template <typename WT, typename XT, int VEC, bool RAG>
+hipError_t ffn_t(const Problem& p, const FusedWs& w, bool* fold, hipStream_t s) {
+  if (p.B == 1) return fused_t<WT, XT, VEC, RAG>(p, w, fold, s);
+  if (fold != nullptr) {  // several tokens: the router runs in its own launch
+    *fold = false;
+    return hipSuccess;
+  }
+  return per_token_t<WT, XT, VEC, RAG>(p, w, s);
+}
+
+// Rows of whole, aligned 16-byte pieces; else ragged rows (at least one piece
+// long, which MXFP4 rows always are) long enough that half of a wave's lanes
+// have a piece of the average one; shorter ones take one element per lane and
+// access.  Measured, one token, us, one element / ragged pieces: fp16 257 x 259
+// 11.8 / 10.9, 513 x 515 14.7 / 11.5, 1500 x 2050 57.8 / 16.3; fp8 101 x 37 10.7
+// / 14.0, 385 x 387 11.8 / 12.4, 513 x 515 13.9 / 12.4, 1500 x 2050 26.2 / 14.7;
+// fp32 1500 x 2050 24.1 / 22.3.
 template <typename WT, typename XT>
 hipError_t ffn_w(const Problem& p, const FusedWs& w, bool* fold, hipStream_t s) {
-  constexpr int V = wvec_width<WT>(), V1 = wvec_scalar<WT>();
-  return p.vec == V ? ffn_t<WT, XT, V>(p, w, fold, s) : ffn_t<WT, XT, V1>(p, w, fold, s);
+  constexpr int V = wvec_width<WT>();
+  if (p.vec == V) return ffn_t<WT, XT, V, false>(p, w, fold, s);
+  if constexpr (std::is_same<WT, fp4x2>::value) {
+    return ffn_t<WT, XT, V, true>(p, w, fold, s);
+  } else {
+    if (p.h >= V && p.I >= V && p.h + p.I >= kWave * V)
+      return ffn_t<WT, XT, V, true>(p, w, fold, s);
+    return ffn_t<WT, XT, 1, false>(p, w, fold, s);
+  }
 }
 
 template <typename XT>
@@ -1961,9 +2135,7 @@ hipError_t launch_fused_route(const Problem& p, hipStream_t s) { return run_rout
 
 hipError_t launch_fused_ffn(const Problem& p, hipStream_t s) { return run_ffn_only(p, nullptr, s); }
 
-hipError_t launch_logits_split(const Problem& p, float* logits, f16* x_hi, f16* x_lo,
-                               int32_t* x_exp, unsigned* amax, int split_bf16, hipStream_t s) {
-  const XSplit xs{x_hi, x_lo, x_exp, amax, p.k, split_bf16};
+hipError_t launch_logits_split(const Problem& p, float* logits, const XSplit& xs, hipStream_t s) {
   return p.adt == WR_F16 ? logits_t<f16>(p, logits, nullptr, 0, 0, s, xs)
                          : logits_t<float>(p, logits, nullptr, 0, 0, s, xs);
 }
