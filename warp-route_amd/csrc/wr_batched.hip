@@ -109,19 +109,21 @@ constexpr int kBM = 64;         // rows per block: 4 waves x 16
 constexpr int kMaxTok = 64;     // tokens per pass, at most: 4 MFMA N tiles
 
 // The expert slot that z (the grid's slot index) runs in a TOK-token tile
-// launch, or -1.  n_active[1] (k_route) counts the experts with more than
-// WR_TILE_SPLIT_M pairs: with none, the 32-token launch takes every slot,
-// else the 64-token launch does.  The other launch's blocks leave after one
-// load.  16-token tiles run alone and take every slot.
+// launch, or -1.  n_active[1] (k_route) is the call's tile class: 0 when no
+// expert has more than WR_TILE_SPLIT_M pairs (the 32-token launch takes every
+// slot), 1 when none has more than kMaxTok (the 64-token launch), else 2 (the
+// many-token launch, TOK = kManyTok).  The other launches' blocks leave after
+// one load.  16-token tiles run alone and take every slot.
+constexpr int kManyTok = 2 * kMaxTok;  // marks the many-token launch
 template <int TOK>
 __device__ __forceinline__ int tile_slot(const BatchRoute& r, int z) {
-  static_assert(TOK == 16 || TOK == 32 || TOK == kMaxTok, "tile sizes");
+  static_assert(TOK == 16 || TOK == 32 || TOK == kMaxTok || TOK == kManyTok, "tile sizes");
   static_assert(WR_MID_TILE_MAX_B <= WR_TILE_SPLIT_M, "32-token batches lead with no 64-token class");
   if constexpr (TOK == 16) {
     return z < r.n_active[0] ? z : -1;
   } else {
-    const int n = r.n_active[0], nb = r.n_active[1];
-    const bool mine = TOK == kMaxTok ? nb > 0 : nb == 0;
+    const int n = r.n_active[0], cls = r.n_active[1];
+    const bool mine = cls == (TOK == 32 ? 0 : TOK == kMaxTok ? 1 : 2);
     return mine && z < n ? z : -1;
   }
 }
@@ -169,7 +171,7 @@ __device__ __forceinline__ void group_pairs(int P, int E, int k, const int* sel_
                                             const float* sel_w, int* cnt, int* off_s, int* off,
                                             int* active, int* na, int32_t* pair_tok,
                                             float* pair_w, int32_t* tok_pair,
-                                            int* nbig = nullptr) {
+                                            int* cls = nullptr, int max_cls = 2) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int nw = blockDim.x / kWave;
@@ -191,13 +193,14 @@ __device__ __forceinline__ void group_pairs(int P, int E, int k, const int* sel_
     }
     off_s[E] = o;
     off[E] = o;
-    int nb = 0;
+    int most = 0;
     for (int e = 0; e < E; ++e) {
       if (cnt[e] > 0) active[n++] = e;
-      nb += cnt[e] > WR_TILE_SPLIT_M;
+      most = max(most, cnt[e]);
     }
     *na = n;
-    if (nbig != nullptr) *nbig = nb;  // experts for 64-token tiles (tile_slot)
+    if (cls != nullptr)  // tile_slot
+      *cls = min(max_cls, (most > WR_TILE_SPLIT_M) + (most > kMaxTok));
   }
   __syncthreads();
   // Stable placement: expert e's pairs in token order.
@@ -220,7 +223,8 @@ __device__ __forceinline__ void group_pairs(int P, int E, int k, const int* sel_
 
 __global__ __launch_bounds__(1024) void k_route(const float* __restrict__ logits, int B, int E,
                                                 int k, int renorm, int32_t* __restrict__ ids_out,
-                                                float* __restrict__ w_out, BatchRoute r) {
+                                                float* __restrict__ w_out, BatchRoute r,
+                                                int max_cls) {
   __shared__ int s_cnt[WR_MAX_EXPERTS];
   __shared__ int s_off[WR_MAX_EXPERTS + 1];
   __shared__ int s_id[kRouteLds];
@@ -278,7 +282,7 @@ __global__ __launch_bounds__(1024) void k_route(const float* __restrict__ logits
   }
   __syncthreads();
   group_pairs(P, E, k, sel_id, sel_w, s_cnt, s_off, r.off, r.active, r.n_active, r.pair_tok,
-              r.pair_w, r.tok_pair, r.n_active + 1);
+              r.pair_w, r.tok_pair, r.n_active + 1, max_cls);
 }
 
 // In-block routing for small batches (B <= WR_SMALL_TILE_MAX_B): every
@@ -1266,6 +1270,21 @@ __device__ __forceinline__ void dn_pass(TokTile<TOK, KC, RAG>& xs,
   }
 }
 
+// Workgroups go to the 8 XCDs round-robin by linear id, so with the grid's own
+// (row tile, K slice) order every XCD ran all K slices and its L2 fetched the
+// whole act tensor.  Relabel: XCD pair q serves K slice q, and an XCD's L2
+// holds a quarter of act.  A bijection on (x, y) whenever gridDim.x is even;
+// the z plane keeps its XCD offset (x*y blocks, a multiple of 8).
+__device__ __forceinline__ void dn_relabel(int& bx, int& ks) {
+  constexpr int kXcd = 8, kPer = kXcd / BatchWs::kKSplit;
+  static_assert(kXcd % BatchWs::kKSplit == 0, "K slices per XCD pair");
+  if (gridDim.x % kPer == 0) {
+    const int l = blockIdx.x + gridDim.x * blockIdx.y;
+    ks = (l % kXcd) / kPer;
+    bx = l % kPer + kPer * (l / kXcd);
+  }
+}
+
 // PRE: act was split into its two terms by k_act_split.  WK: the weight K
 // step (dn_pass); the K slices are then whole weight steps.
 template <typename WT, int TOK, int KC, bool PRE, int WK, bool RAG>
@@ -1282,20 +1301,8 @@ __device__ __forceinline__ void dn_block(const WT* __restrict__ wbuf, const Batc
   const int pbeg = r.off[e], M = r.off[e + 1] - pbeg;
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
-  // Workgroups go to the 8 XCDs round-robin by linear id, so with the grid's
-  // own (row tile, K slice) order every XCD ran all K slices and its L2
-  // fetched the whole act tensor.  Relabel: XCD pair q serves K slice q, and
-  // an XCD's L2 holds a quarter of act.  A bijection on (x, y) whenever
-  // gridDim.x is even; the z plane keeps its XCD offset (x*y blocks, a
-  // multiple of 8).
-  constexpr int kXcd = 8, kPer = kXcd / BatchWs::kKSplit;
-  static_assert(kXcd % BatchWs::kKSplit == 0, "K slices per XCD pair");
   int bx = blockIdx.x, ks = blockIdx.y;
-  if (gridDim.x % kPer == 0) {
-    const int l = blockIdx.x + gridDim.x * blockIdx.y;
-    ks = (l % kXcd) / kPer;
-    bx = l % kPer + kPer * (l / kXcd);
-  }
+  dn_relabel(bx, ks);
   const int row0 = bx * kBM + wave * 16;
   constexpr int R = WK / KC;  // token steps per weight step (I % WK == 0)
   const int nsteps = (RAG ? g.Ip : g.I) / WK;
@@ -1393,6 +1400,471 @@ __global__ __launch_bounds__(kBlk) void k_act_split(float* __restrict__ act,
     dn_tile_split<BF>(hi, lo, t, sx);
     reinterpret_cast<H8*>(a)[0] = hi[0];
     reinterpret_cast<H8*>(a)[1] = lo[0];
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Many tokens per expert (B > 64 and an expert with more than 64 pairs): up to
+// kPassTok tokens of an expert in one pass, so that its weights stream once
+// (the 64-token kernels read them again for every 64 tokens), in the wave
+// layout that reads the least from LDS per MFMA: with 4 waves of 32 weight
+// rows, every wave reads every token fragment (10 KB per 16 MFMAs, more LDS
+// time than MFMA time); here the block's 128 weight rows x the pass's tokens
+// are split in 2 x 2 waves of 64 rows x half of the tokens (12 KB per 32
+// MFMAs).  A pass has NTW tiles of 16 tokens per wave.  Staging: token tiles of
+// 32 columns in two LDS buffers with two more in registers, weight rows 128
+// bytes at a time (MXFP4: 64) in two LDS buffers with one more in registers, so
+// that a sub-step of 32 columns has one barrier and its loads were issued two
+// sub-steps before they are stored.  Experts of at most 64 tokens run gu_pass /
+// dn_pass.
+// ---------------------------------------------------------------------------
+constexpr int kPassTok = 160;  // tokens per pass
+constexpr int kManyRows = 128;  // weight rows per block: 64 gate and 64 up, or 128 down
+constexpr int kManyP = 4;       // 16-byte pieces per token row and term of a sub-step
+
+// Columns of a weight step.
+template <typename WT>
+constexpr int many_kw() {
+  return wbits<WT>() == 16 ? 64 : 128;
+}
+// LDS of a many-token block: two token tiles (two terms each), two weight
+// steps, MXFP4's block scales of both; at least a 64-token pass's tiles.
+template <typename WT>
+struct ManyLds {
+  static constexpr int kX = 2 * kPassTok * kManyP * 16;  // bytes per buffer
+  static constexpr int kPW = many_kw<WT>() / WGeo<WT, many_kw<WT>()>::kElems;  // pieces per row
+  static constexpr int kW = kManyRows * kPW * 16;
+  static constexpr int kS = std::is_same<WT, fp4x2>::value ? kManyRows * kPW : 0;
+  static constexpr int kBig = 2 * (kX + kW + kS);
+  static constexpr int kSmall =
+      (int)(sizeof(TokTile<kMaxTok, kBK>) + kBlk / kWave * sizeof(WTile<WT, 32, kBK>));
+  static constexpr int kBytes = kBig > kSmall ? kBig : kSmall;
+};
+
+// Tokens per pass of an expert of M tokens: equal passes, in whole tiles of
+// both token halves.
+__device__ __forceinline__ int many_pass(int M) {
+  const int np = (M + kPassTok - 1) / kPassTok, per = (M + np - 1) / np;
+  return (per + 31) / 32 * 32;
+}
+
+// v, unknown to the compiler: what a pass derives from it is not computed ahead
+// of the pass loop, for every tile count at once (which spilled registers).
+__device__ __forceinline__ int opaque(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// Slot of 16-byte piece c of row n in rows of P pieces: 16 consecutive rows'
+// pieces c lie in 16 distinct 16-byte groups of the 64 banks.  The same slot
+// for n + 16.
+template <int P>
+__device__ __forceinline__ int many_slot(int n, int c) {
+  constexpr int L = 16 / P;  // rows that share 256 bytes
+  return c ^ ((n / L) & (P - 1));
+}
+
+// Token rows of a pass: x's two terms by pair (rows from LDS), or act rows
+// split ahead (k_act_split: 8 hi terms, then 8 lo terms).  Rows past the pass's
+// tokens repeat a valid one; their sums are not used.
+// at(n, c, t): bytes from base to piece c of term t of row n, 32 bits (the host
+// checks that x's two terms lie within 4 GiB); kCol: bytes per column.
+struct RowsX {
+  const char* base;  // the hi terms
+  uint32_t lo;       // bytes from a hi term to its lo term
+  const int* s_row;
+  int ld;
+  static constexpr int kCol = 2;
+  __device__ __forceinline__ uint32_t at(int n, int c, int t) const {
+    return ((uint32_t)s_row[n] * (uint32_t)ld + 8 * c) * 2 + (t ? lo : 0);
+  }
+};
+struct RowsAct {
+  const char* base;  // the pass's first row
+  int mt, ld;
+  static constexpr int kCol = 4;
+  __device__ __forceinline__ uint32_t at(int n, int c, int t) const {
+    return ((uint32_t)min(n, mt - 1) * (uint32_t)ld + 8 * c) * 4 + 16 * t;
+  }
+};
+
+// Weight rows of a wave's 32-row tile as wave-uniform addresses (in scalar
+// registers) and one 32-bit lane offset for all of them: pointers per row group
+// would take 16 of the registers that a pass's sums leave.  mat: tile row 0 at
+// column 0.  H = 2: 16 rows there and 16 more half elements on (gate and up
+// rows); H = 1: 32 consecutive rows.
+template <typename WT, int H, int KC>
+struct WSrc {
+  const WT* mat;
+  int64_t half, ld;
+  const uint8_t* sc;  // MXFP4: the same of the block scales, half_s bytes apart
+  int64_t half_s;
+  uint32_t lane_b, lane_s;  // bytes of the lane's row and piece within a row group
+  static constexpr int N = WRegs<WT, 32, KC>::N, RP = WGeo<WT, KC>::kRowsPer;
+  __device__ __forceinline__ WSrc(const WT* m, int64_t h, int64_t l, const uint8_t* s, int64_t hs,
+                                  int lane)
+      : mat(m), half(h), ld(l), sc(s), half_s(hs) {
+    typedef WGeo<WT, KC> G;
+    const int row = lane / G::kLaneRow, col = (lane % G::kLaneRow) * G::kElems;
+    lane_b = (uint32_t)(eoff<WT>((int64_t)row * ld + col) * sizeof(WT));
+    lane_s = (uint32_t)(row * (ld / 32) + col / 32);
+  }
+  __device__ __forceinline__ void load(WRegs<WT, 32, KC>& r, int kb) const {
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const int64_t row = RP * (i % (N / H));
+      const char* p = reinterpret_cast<const char*>(mat + (i < N / H ? 0 : half) +
+                                                    eoff<WT>(row * ld + kb));
+      r.v[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p + lane_b));
+      if constexpr (std::is_same<WT, fp4x2>::value)
+        r.e[i] = (sc + (i < N / H ? 0 : half_s) + row * (ld / 32) + kb / 32)[lane_s];
+    }
+  }
+};
+
+// acc[f][n] += weight rows 64 (wave % 2) + 16 f .. of the block's 128 x tokens
+// 16 (NTW (wave / 2) + n) .. of the pass, over columns [kb, ke) of K, whole
+// weight steps.  Each wave stages the 32 rows of src at rows 32 wave.
+template <typename WT, bool LO, int NTW, int H, typename Rows>
+__device__ __forceinline__ void many_mm(f32x4 (&acc)[4][NTW], unsigned char* raw,
+                                        const WSrc<WT, H, many_kw<WT>()>& src, const Rows& rows,
+                                        int kb, int ke, int lane, int wave) {
+  typedef ManyLds<WT> L;
+  constexpr int KW = many_kw<WT>(), R = KW / 32, P = kManyP, PW = L::kPW, TOK = 32 * NTW;
+  // A sub-step's pieces, hi terms then lo terms, kBlk per round: NTW per thread
+  // with both terms.
+  constexpr int NP = TOK * P * (LO ? 2 : 1), TP = (NP + kBlk - 1) / kBlk;
+  constexpr int NW = WRegs<WT, 32, KW>::N;
+  constexpr bool BF = bf16_ops<WT>(), F4 = std::is_same<WT, fp4x2>::value;
+  static_assert(R % 2 == 0 && TOK <= kPassTok, "buffers alternate within a weight step");
+  H8* const xb = reinterpret_cast<H8*>(raw);
+  H8* const wb = reinterpret_cast<H8*>(raw + 2 * L::kX);
+  uint8_t* const sb = raw + 2 * (L::kX + L::kW);
+  WRegs<WT, 32, KW> wr;
+  H8 tx[2][TP];
+  const int r15 = lane & 15, q4 = lane >> 4;
+  // Piece q of this thread: 64 wave + 256 q + lane, of one term for a whole
+  // wave (a wave past the last piece repeats the tile's last rows).  Token rows
+  // 16 apart have the same slots, so its place in a buffer is the thread's own
+  // plus a wave-uniform part.
+  uint32_t at[TP];
+  const int tid = kWave * wave + lane, trow = tid / P, tc = tid % P;
+  const int place = trow * P + many_slot<P>(trow, tc);
+  auto term = [&](int q) { return LO && kWave * wave + kBlk * q >= TOK * P ? 1 : 0; };
+  auto row0 = [&](int q) { return min(kBlk / P * q - TOK * term(q), TOK - (wave + 1) * kWave / P); };
+#pragma unroll
+  for (int q = 0; q < TP; ++q) at[q] = rows.at(trow + row0(q), tc, term(q));
+  // Every load is unconditional, columns past the end clamped (their tiles are
+  // never read): behind a branch the compiler waits for all loads in flight.
+  auto xload = [&](int set, int col) {
+    const char* b = rows.base + (int64_t)min(col, ke - 32) * Rows::kCol;
+#pragma unroll
+    for (int q = 0; q < TP; ++q) tx[set][q] = *reinterpret_cast<const H8*>(b + at[q]);
+  };
+  auto xstore = [&](int b) {  // sub-step of parity b: set b to buffer b
+    H8* x = xb + b * (L::kX / 16);
+#pragma unroll
+    for (int q = 0; q < TP; ++q) x[place + (term(q) * kPassTok + row0(q)) * P] = tx[b][q];
+  };
+  auto wstore = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+      const int row = 32 * wave + WGeo<WT, KW>::kRowsPer * i + lane / PW, c = lane % PW;
+      wb[b * (L::kW / 16) + row * PW + many_slot<PW>(row, c)] = __builtin_bit_cast(H8, wr.v[i]);
+      if constexpr (F4) sb[b * L::kS + row * PW + c] = wr.e[i];
+    }
+  };
+  // Fragment f of sub-step jj of the weight step in buffer b: the 8 weights of
+  // this lane's row at columns 32 jj + 8 q4, decoded (a_frag).
+  auto frag = [&](int b, int f, int jj) -> H8 {
+    const int row = 64 * (wave & 1) + 16 * f + r15;
+    const H8* w = wb + b * (L::kW / 16) + row * PW;
+    if constexpr (wbits<WT>() == 16) {
+      return w[many_slot<PW>(r15, 4 * jj + q4)];
+    } else if constexpr (wbits<WT>() == 8) {
+      const uint2 v =
+          reinterpret_cast<const uint2*>(&w[many_slot<PW>(r15, 2 * jj + (q4 >> 1))])[q4 & 1];
+      return fp8x8_to_h8(v.x, v.y);
+    } else {
+      const uint32_t v = reinterpret_cast<const uint32_t*>(&w[many_slot<PW>(r15, jj)])[q4];
+      return fp4x8_to_bf8(v, e8m0_value(sb[b * L::kS + row * PW + jj]));
+    }
+  };
+  // Prologue: sub-step 0 and weight step 0 in LDS, sub-steps 1 and 2 and weight
+  // step 1 on their way.
+  __syncthreads();  // the previous pass is done with the buffers
+  src.load(wr, kb);
+  xload(0, kb);
+  xload(1, kb + 32);
+  wstore(0);
+  xstore(0);
+  xload(0, kb + 64);
+  src.load(wr, min(kb + KW, ke - KW));
+  int wcur = 0;
+  for (int k0 = kb; k0 < ke; k0 += KW, wcur ^= 1) {
+#pragma unroll
+    for (int hs = 0; hs < R; ++hs) {
+      const int k = k0 + 32 * hs;
+      __syncthreads();  // this sub-step's tiles are visible, the last one's are free
+      xstore((hs + 1) & 1);
+      xload((hs + 1) & 1, k + 96);
+      if (hs == R - 1) {
+        wstore(wcur ^ 1);
+        src.load(wr, min(k0 + 2 * KW, ke - KW));
+      }
+      __builtin_amdgcn_sched_barrier(0);  // loads ahead of the MFMAs
+      H8 a[4];
+#pragma unroll
+      for (int f = 0; f < 4; ++f) a[f] = frag(wcur, f, hs);
+      const H8* bx = xb + (hs & 1) * (L::kX / 16) + (16 * NTW * (wave >> 1) + r15) * P +
+                     many_slot<P>(r15, q4);
+#pragma unroll
+      for (int n = 0; n < NTW; ++n) {
+        const H8 bh = bx[16 * P * n];
+#pragma unroll
+        for (int f = 0; f < 4; ++f) acc[f][n] = mfma<BF>(a[f], bh, acc[f][n]);
+        if constexpr (LO) {
+          const H8 bl = bx[16 * P * n + kPassTok * P];
+#pragma unroll
+          for (int f = 0; f < 4; ++f) acc[f][n] = mfma<BF>(a[f], bl, acc[f][n]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+}
+
+template <typename WT, bool LO, int NTW>
+__device__ __forceinline__ void gu_pass_many(unsigned char* raw,
+                                             const WSrc<WT, 2, many_kw<WT>()>& src,
+                                             const RowsX& rows,
+                                             const BatchRoute& r, int p0, int mt,
+                                             float* __restrict__ act, int row0,
+                                             const float* __restrict__ sc, const GuScale& xsc,
+                                             const GeomB& g, int lane, int wave) {
+  constexpr bool SC = !bf16_ops<WT>();
+  f32x4 acc[4][NTW];
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int n = 0; n < NTW; ++n) acc[f][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  many_mm<WT, LO, NTW, 2>(acc, raw, src, rows, 0, g.h, lane, wave);
+  // Fragments 2 t and 2 t + 1: gate and up rows rq ..+4 (D layout as in gu_pass).
+#pragma unroll
+  for (int n = 0; n < NTW; ++n) {
+    const int tn = (NTW * (wave >> 1) + n) * 16 + (lane & 15);
+    float mx = 0.0f;
+    if (tn < mt) {
+      const int p = p0 + tn;
+      const float w = r.pair_w[p];
+      const int xe = SC ? xsc.x_exp[rows.s_row[tn]] : 0;
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const int rq = row0 + (2 * (wave & 1) + t) * 16 + (lane >> 4) * 4;
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float gs = SC ? ldexpf(acc[2 * t][n][i], -xe) : acc[2 * t][n][i];
+          const float us = SC ? ldexpf(acc[2 * t + 1][n][i], -xe) : acc[2 * t + 1][n][i];
+          if constexpr (std::is_same<WT, fp8w>::value)
+            v[i] = w * (silu(gs * sc[rq + i]) * (us * sc[g.I + rq + i]));
+          else
+            v[i] = w * (silu(gs) * us);
+          mx = fmaxf(mx, fabsf(v[i]));
+        }
+        *reinterpret_cast<f32x4*>(act + (int64_t)p * g.I + rq) = v;
+      }
+    }
+    if constexpr (SC) {
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      if (lane < 16 && tn < mt) atomicMax(xsc.s_amax + tn, __float_as_uint(mx));
+    }
+  }
+  if constexpr (SC) {  // as in gu_pass
+    __syncthreads();
+    if ((int)threadIdx.x < mt) {
+      const unsigned v = xsc.s_amax[threadIdx.x];
+      xsc.s_amax[threadIdx.x] = 0u;
+      __hip_atomic_fetch_max(xsc.amax + (int64_t)(p0 + threadIdx.x) * BatchWs::kAmaxStride, v,
+                             __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  }
+}
+
+// grid (I / 64, expert slots).  Two blocks per CU: 256 VGPRs.
+template <typename WT, bool LO, int WK = kBK>
+__global__ __launch_bounds__(kBlk, 2) void k_many_gu(
+    const WT* __restrict__ wbuf, const f16* __restrict__ x_hi, const f16* __restrict__ x_lo,
+    const int32_t* __restrict__ x_exp, unsigned* __restrict__ amax, BatchRoute r,
+    float* __restrict__ act, GeomB g) {
+  static_assert(kPassTok <= kBlk, "a thread per token of a pass");
+  __shared__ __align__(16) unsigned char raw[ManyLds<WT>::kBytes];
+  __shared__ unsigned s_amax[bf16_ops<WT>() ? 1 : kPassTok];
+  __shared__ int s_row[kPassTok];
+  const int slot = tile_slot<kManyTok>(r, blockIdx.y);
+  if (slot < 0) return;  // block-uniform
+  const int e = r.active[slot];
+  const int pbeg = r.off[e], M = r.off[e + 1] - pbeg;
+  if (!bf16_ops<WT>() && threadIdx.x < kPassTok) s_amax[threadIdx.x] = 0u;
+  const GuScale xsc{x_exp, amax, s_amax};
+  const int lane0 = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const int row0 = blockIdx.x * kBM;
+  const WT* blk = wbuf + (int64_t)e * g.stride;
+  const uint8_t* mxs = reinterpret_cast<const uint8_t*>(blk) + g.off_scale;
+  const float* sc = nullptr;
+  if constexpr (std::is_same<WT, fp8w>::value) sc = wscales(blk, g.off_scale);
+  const int wrow = row0 + wave * 16;  // this wave's staged rows (gate; the same up rows)
+  if (M <= kMaxTok) {
+    const int lane = lane0;
+    const WT* G = w_lane_base<WT, WK>(blk, wrow, g.h, lane);
+    constexpr int N = WRegs<WT, 32, WK>::N, RP = WGeo<WT, WK>::kRowsPer;
+    const WT* wbase[N];
+    const uint8_t* wsc[N];
+#pragma unroll
+    for (int i = 0; i < N; ++i) {  // as in gu_block
+      wbase[i] = G + (i < N / 2 ? 0 : g.off_up) + eoff<WT>((int64_t)(RP * (i % (N / 2))) * g.h);
+      wsc[i] = w_lane_scale<WT, WK>(mxs + (i < N / 2 ? 0 : (int64_t)g.I * g.h / 32), wrow, g.h,
+                                    lane) +
+               (int64_t)(RP * (i % (N / 2))) * (g.h / 32);
+    }
+    auto& xs = *reinterpret_cast<TokTile<kMaxTok, kBK>*>(raw);
+    auto& wt = reinterpret_cast<WTile<WT, 32, WK>*>(raw + sizeof(xs))[wave];
+    switch ((M + 15) / 16) {
+      case 1: gu_pass<WT, LO, 1, kMaxTok, kBK, WK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
+      case 2: gu_pass<WT, LO, 2, kMaxTok, kBK, WK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
+      case 3: gu_pass<WT, LO, 3, kMaxTok, kBK, WK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
+      default: gu_pass<WT, LO, 4, kMaxTok, kBK, WK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
+    }
+    return;
+  }
+  const WSrc<WT, 2, many_kw<WT>()> src(blk + eoff<WT>((int64_t)wrow * g.h), g.off_up, g.h,
+                            mxs + (int64_t)wrow * (g.h / 32), (int64_t)g.I * g.h / 32, lane0);
+  const RowsX rows{reinterpret_cast<const char*>(x_hi),
+                   (uint32_t)(reinterpret_cast<const char*>(x_lo) -
+                              reinterpret_cast<const char*>(x_hi)),
+                   s_row, g.h};
+  const int per = many_pass(M);
+  for (int m0 = 0; m0 < M; m0 += per) {
+    const int mt = min(per, M - m0);
+    const int p0 = pbeg + m0;
+    __syncthreads();  // the previous pass is done with s_row
+    if (threadIdx.x < kPassTok)
+      s_row[threadIdx.x] = r.pair_tok[p0 + min((int)threadIdx.x, mt - 1)];
+    __syncthreads();
+    const int lane = opaque(lane0);
+    switch ((mt + 31) / 32) {
+      case 1: case 2: case 3: gu_pass_many<WT, LO, 3>(raw, src, rows, r, p0, mt, act, row0, sc, xsc, g, lane, wave); break;
+      case 4: gu_pass_many<WT, LO, 4>(raw, src, rows, r, p0, mt, act, row0, sc, xsc, g, lane, wave); break;
+      default: gu_pass_many<WT, LO, 5>(raw, src, rows, r, p0, mt, act, row0, sc, xsc, g, lane, wave); break;
+    }
+  }
+}
+
+template <typename WT, int NTW>
+__device__ __forceinline__ void dn_pass_many(unsigned char* raw,
+                                             const WSrc<WT, 1, many_kw<WT>()>& src,
+                                             const float* __restrict__ act,
+                                             const unsigned* __restrict__ amax, int p0, int mt,
+                                             int kb, int ke, float* __restrict__ y, int row0,
+                                             const float* __restrict__ sdown, const GeomB& g,
+                                             int lane, int wave) {
+  f32x4 acc[4][NTW];
+#pragma unroll
+  for (int f = 0; f < 4; ++f)
+#pragma unroll
+    for (int n = 0; n < NTW; ++n) acc[f][n] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  const RowsAct rows{reinterpret_cast<const char*>(act + (int64_t)p0 * g.I), mt, g.I};
+  if (kb < ke) many_mm<WT, true, NTW, 1>(acc, raw, src, rows, kb, ke, lane, wave);
+#pragma unroll
+  for (int n = 0; n < NTW; ++n) {
+    const int tn = (NTW * (wave >> 1) + n) * 16 + (lane & 15);
+    if (tn < mt) {
+      const int ae = pair_exp<WT>(amax, p0 + tn);
+#pragma unroll
+      for (int f = 0; f < 4; ++f) {
+        const int rq = row0 + 64 * (wave & 1) + f * 16 + (lane >> 4) * 4;
+        f32x4 v = acc[f][n];
+        if constexpr (!bf16_ops<WT>()) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] = ldexpf(v[i], -ae);
+        }
+        if constexpr (std::is_same<WT, fp8w>::value) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) v[i] *= sdown[rq + i];
+        }
+        *reinterpret_cast<f32x4*>(y + (int64_t)(p0 + tn) * g.h + rq) = v;
+      }
+    }
+  }
+}
+
+// grid (h / 128, kKSplit, expert slots), act split ahead; K slices of whole WK
+// steps, as k_dn_mfma's.
+template <typename WT, int WK = kBK>
+__global__ __launch_bounds__(kBlk, 2) void k_many_dn(const WT* __restrict__ wbuf, BatchRoute r,
+                                                     const float* __restrict__ act,
+                                                     const unsigned* __restrict__ amax,
+                                                     float* __restrict__ ypart, GeomB g, int P) {
+  __shared__ __align__(16) unsigned char raw[ManyLds<WT>::kBytes];
+  const int slot = tile_slot<kManyTok>(r, blockIdx.z);
+  if (slot < 0) return;
+  const int e = r.active[slot];
+  const int pbeg = r.off[e], M = r.off[e + 1] - pbeg;
+  const int lane0 = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  int bx = blockIdx.x, ks = blockIdx.y;
+  dn_relabel(bx, ks);
+  const int row0 = bx * kManyRows;
+  const int nsteps = g.I / WK;
+  const int kb = nsteps * ks / BatchWs::kKSplit * WK;
+  const int ke = nsteps * (ks + 1) / BatchWs::kKSplit * WK;
+  const WT* blk = wbuf + (int64_t)e * g.stride;
+  const float* sdown = nullptr;
+  if constexpr (std::is_same<WT, fp8w>::value) sdown = wscales(blk, g.off_scale) + 2 * g.I;
+  const uint8_t* mxs =
+      reinterpret_cast<const uint8_t*>(blk) + g.off_scale + 2 * ((int64_t)g.I * g.h / 32);
+  float* y = ypart + (int64_t)ks * P * g.h;
+  if (M <= kMaxTok) {  // the block's rows in two halves of 4 x 16
+    const int lane = lane0;
+    auto& xs = *reinterpret_cast<TokTile<kMaxTok, kBK>*>(raw);
+    auto& wt = reinterpret_cast<WTile<WT, 16, WK>*>(raw + sizeof(xs))[wave];
+    constexpr int N = WRegs<WT, 16, WK>::N;
+    for (int half = 0; half < 2; ++half) {
+      const int wrow = row0 + half * kBM + wave * 16;
+      const WT* D = w_lane_base<WT, WK>(blk + g.off_down, wrow, g.I, lane);
+      const WT* wbase[N];
+      const uint8_t* wsc[N];
+#pragma unroll
+      for (int i = 0; i < N; ++i) {  // as in dn_block
+        wbase[i] = D + eoff<WT>((int64_t)(WGeo<WT, WK>::kRowsPer * i) * g.I);
+        wsc[i] = w_lane_scale<WT, WK>(mxs, wrow, g.I, lane) +
+                 (int64_t)(WGeo<WT, WK>::kRowsPer * i) * (g.I / 32);
+      }
+      const int sb = kb / kBK, se = ke / kBK;
+      switch ((M + 15) / 16) {
+        case 1: dn_pass<WT, 1, kMaxTok, kBK, true, WK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
+        case 2: dn_pass<WT, 2, kMaxTok, kBK, true, WK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
+        case 3: dn_pass<WT, 3, kMaxTok, kBK, true, WK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
+        default: dn_pass<WT, 4, kMaxTok, kBK, true, WK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
+      }
+    }
+    return;
+  }
+  const int wrow = row0 + wave * 32;
+  const WSrc<WT, 1, many_kw<WT>()> src(blk + g.off_down + eoff<WT>((int64_t)wrow * g.I), 0, g.I,
+                            mxs + (int64_t)wrow * (g.I / 32), 0, lane0);
+  const int per = many_pass(M);
+  for (int m0 = 0; m0 < M; m0 += per) {
+    const int mt = min(per, M - m0);
+    const int p0 = pbeg + m0;
+    const int lane = opaque(lane0);
+    switch ((mt + 31) / 32) {
+      case 1: case 2: case 3: dn_pass_many<WT, 3>(raw, src, act, amax, p0, mt, kb, ke, y, row0, sdown, g, lane, wave); break;
+      case 4: dn_pass_many<WT, 4>(raw, src, act, amax, p0, mt, kb, ke, y, row0, sdown, g, lane, wave); break;
+      default: dn_pass_many<WT, 5>(raw, src, act, amax, p0, mt, kb, ke, y, row0, sdown, g, lane, wave); break;
+    }
   }
 }
 
@@ -1906,7 +2378,7 @@ hipError_t ragged_t(const Problem& p, const BatchWs& w, hipStream_t s) {
   hipError_t err = hipSuccess;
   if (tile > 16) {
     hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
-                       p.topk_ids, p.topk_w, w.route);
+                       p.topk_ids, p.topk_w, w.route, 0);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
   const dim3 gg(g.Ip / kBM, slots), gd((p.h + kBM - 1) / kBM, BatchWs::kKSplit, slots);
@@ -1932,7 +2404,7 @@ hipError_t ragged_f32(const Problem& p, const BatchWs& w, hipStream_t s) {
   hipError_t err = hipSuccess;
   if (tile > 16) {
     hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
-                       p.topk_ids, p.topk_w, w.route);
+                       p.topk_ids, p.topk_w, w.route, 0);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
   const dim3 gg(g.Ip / kBM, slots), gd((p.h + kBM - 1) / kBM, BatchWs::kKSplit, slots);
@@ -1955,10 +2427,12 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
   const WT* wb = static_cast<const WT*>(p.wbuf);
 
   hipError_t err = hipSuccess;
+  // The many-token kernels address x's two terms with 32-bit offsets.
+  const bool many = p.B > kMaxTok && (int64_t)p.B * p.h * 4 < (int64_t{1} << 32);
   // Small batches route inside the gate/up kernel (one launch fewer).
   if (p.B > WR_SMALL_TILE_MAX_B) {
     hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
-                       p.topk_ids, p.topk_w, w.route);
+                       p.topk_ids, p.topk_w, w.route, many ? 2 : 1);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
   // The lo term of x: fp32 x, or any x against bf16 (8-bit mantissa) terms.
@@ -1992,38 +2466,42 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
     // 168 us and bf16 161 -> 165 us (the launch costs more than the repeated
     // splits of 32-token tiles).
     constexpr bool kPre32 = wbits<WT>() < 16;
+    // The classes (tile_slot) that the call can be of: an expert has at most B
+    // tokens, and with more than n pairs per expert on average one has more
+    // than n.  One of the launches made runs.
     const bool mid = p.B <= WR_MID_TILE_MAX_B;
+    const bool run32 = P <= WR_TILE_SPLIT_M * p.E;
+    const bool run64 = !mid && (!many || P <= kMaxTok * p.E);
+    const dim3 gg(p.I / kBM, slots), gd(p.h / kBM, BatchWs::kKSplit, slots);
     // MXFP4 32-token tiles: the wide step where it divides h (gate/up) or I
     // (down); its 128-column step loads 16 rows x 64 bytes per instruction.
     // B = 24 / 32: 115.1 / 119.6 -> 102.8 / 103.5 us per call (gate/up 176
     // VGPRs, 2 blocks per CU; a 3-block bound, 144 VGPRs, measured slower).
     constexpr int KM = (WR_MID_WIDE && std::is_same<WT, fp4x2>::value) ? kc_wide<WT>() : kBK;
-    // Beyond WR_MID_TILE_MAX_B both tile launches are made and one of them
-    // runs (tile_slot).
-    if (KM != kBK && p.h % KM == 0)
-      hipLaunchKernelGGL((k_gu_mfma<WT, LO, 32, false, KM>), dim3(p.I / kBM, slots), dim3(kBlk),
-                         0, s, wb, w.x_hi, w.x_lo, w.x_exp, w.amax, w.route, w.act, g, nullptr,
-                         nullptr, nullptr);
-    else
-      hipLaunchKernelGGL((k_gu_mfma<WT, LO, 32, false, kBK>), dim3(p.I / kBM, slots), dim3(kBlk),
-                         0, s, wb, w.x_hi, w.x_lo, w.x_exp, w.amax, w.route, w.act, g, nullptr,
-                         nullptr, nullptr);
-    if ((err = hipGetLastError()) != hipSuccess) return err;
-    if (!mid) {
-      bool wide = false;
-      if constexpr (WR_W2 && std::is_same<WT, fp4x2>::value) {
-        wide = p.h % kc_wide<WT>() == 0;
-        if (wide)
-          hipLaunchKernelGGL((k_gu_mfma<WT, LO, kMaxTok, false, kBK, kc_wide<WT>()>),
-                             dim3(p.I / kBM, slots), dim3(kBlk), 0, s, wb, w.x_hi, w.x_lo,
-                             w.x_exp, w.amax, w.route, w.act, g, nullptr, nullptr, nullptr);
-      }
-      if (!wide)
-        hipLaunchKernelGGL((k_gu_mfma<WT, LO, kMaxTok, false, kBK>), dim3(p.I / kBM, slots),
-                           dim3(kBlk), 0, s, wb, w.x_hi, w.x_lo, w.x_exp, w.amax, w.route, w.act,
-                           g, nullptr, nullptr, nullptr);
+    // The weight step of 64-token and many-token tiles.
+    constexpr int KG = (WR_W2 && std::is_same<WT, fp4x2>::value) ? kc_wide<WT>() : kBK;
+    constexpr int KD = (WR_W2DN && std::is_same<WT, fp4x2>::value) ? kc_wide<WT>() : kBK;
+    if (run32) {
+      auto k = KM != kBK && p.h % KM == 0 ? k_gu_mfma<WT, LO, 32, false, KM>
+                                          : k_gu_mfma<WT, LO, 32, false, kBK>;
+      hipLaunchKernelGGL(k, gg, dim3(kBlk), 0, s, wb, w.x_hi, w.x_lo, w.x_exp, w.amax, w.route,
+                         w.act, g, nullptr, nullptr, nullptr);
+      if ((err = hipGetLastError()) != hipSuccess) return err;
+    }
+    if (many) {
+      hipLaunchKernelGGL((k_many_gu<WT, LO>), gg, dim3(kBlk), 0, s, wb, w.x_hi, w.x_lo, w.x_exp,
+                         w.amax, w.route, w.act, g);
+      if ((err = hipGetLastError()) != hipSuccess) return err;
+    }
+    if (run64) {
+      auto k = KG != kBK && p.h % KG == 0 ? k_gu_mfma<WT, LO, kMaxTok, false, kBK, KG>
+                                          : k_gu_mfma<WT, LO, kMaxTok, false, kBK>;
+      hipLaunchKernelGGL(k, gg, dim3(kBlk), 0, s, wb, w.x_hi, w.x_lo, w.x_exp, w.amax, w.route,
+                         w.act, g, nullptr, nullptr, nullptr);
     }
     if ((err = hipGetLastError()) != hipSuccess) return err;
+    // act is split when the 64-token or many-token launch runs, and for 8- and
+    // 4-bit weights always.
     if (!mid || kPre32) {
       const int64_t pieces = (int64_t)P * (p.I / 8);
       const int split_blocks = (int)std::min<int64_t>((pieces + kBlk - 1) / kBlk, 4096);
@@ -2032,36 +2510,21 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
                          kPre32 ? nullptr : static_cast<const int32_t*>(w.route.n_active + 1));
       if ((err = hipGetLastError()) != hipSuccess) return err;
     }
-    if (mid && KM != kBK && p.I % KM == 0)
-      hipLaunchKernelGGL((k_dn_mfma<WT, 32, KM, kPre32>), dim3(p.h / kBM, BatchWs::kKSplit, slots),
-                         dim3(kBlk), 0, s, wb, w.route, w.act, w.amax, w.ypart, g, P);
-    else if (mid)
-      hipLaunchKernelGGL((k_dn_mfma<WT, 32, kBK, kPre32>), dim3(p.h / kBM, BatchWs::kKSplit, slots),
-                         dim3(kBlk), 0, s, wb, w.route, w.act, w.amax, w.ypart, g, P);
-    else {
-      // act is split when the 64-token launch runs, and for 8- and 4-bit
-      // weights always
-      if (KM != kBK && p.I % KM == 0)
-        hipLaunchKernelGGL((k_dn_mfma<WT, 32, KM, kPre32>),
-                           dim3(p.h / kBM, BatchWs::kKSplit, slots), dim3(kBlk), 0, s, wb,
-                           w.route, w.act, w.amax, w.ypart, g, P);
-      else
-        hipLaunchKernelGGL((k_dn_mfma<WT, 32, kBK, kPre32>),
-                           dim3(p.h / kBM, BatchWs::kKSplit, slots), dim3(kBlk), 0, s, wb,
-                           w.route, w.act, w.amax, w.ypart, g, P);
+    if (run32) {
+      auto k = KM != kBK && p.I % KM == 0 ? k_dn_mfma<WT, 32, KM, kPre32>
+                                          : k_dn_mfma<WT, 32, kBK, kPre32>;
+      hipLaunchKernelGGL(k, gd, dim3(kBlk), 0, s, wb, w.route, w.act, w.amax, w.ypart, g, P);
       if ((err = hipGetLastError()) != hipSuccess) return err;
-      bool wide = false;
-      if constexpr (WR_W2DN && std::is_same<WT, fp4x2>::value) {
-        wide = p.I % kc_wide<WT>() == 0;
-        if (wide)
-          hipLaunchKernelGGL((k_dn_mfma<WT, kMaxTok, kBK, true, kc_wide<WT>()>),
-                             dim3(p.h / kBM, BatchWs::kKSplit, slots), dim3(kBlk), 0, s, wb,
-                             w.route, w.act, w.amax, w.ypart, g, P);
-      }
-      if (!wide)
-        hipLaunchKernelGGL((k_dn_mfma<WT, kMaxTok, kBK, true>),
-                           dim3(p.h / kBM, BatchWs::kKSplit, slots), dim3(kBlk), 0, s, wb,
-                           w.route, w.act, w.amax, w.ypart, g, P);
+    }
+    if (many) {
+      hipLaunchKernelGGL((k_many_dn<WT>), dim3(p.h / kManyRows, BatchWs::kKSplit, slots),
+                         dim3(kBlk), 0, s, wb, w.route, w.act, w.amax, w.ypart, g, P);
+      if ((err = hipGetLastError()) != hipSuccess) return err;
+    }
+    if (run64) {
+      auto k = KD != kBK && p.I % KD == 0 ? k_dn_mfma<WT, kMaxTok, kBK, true, KD>
+                                          : k_dn_mfma<WT, kMaxTok, kBK, true>;
+      hipLaunchKernelGGL(k, gd, dim3(kBlk), 0, s, wb, w.route, w.act, w.amax, w.ypart, g, P);
     }
   }
   if ((err = hipGetLastError()) != hipSuccess) return err;
@@ -2078,7 +2541,7 @@ hipError_t grouped_f32(const Problem& p, const BatchWs& w, hipStream_t s) {
   hipError_t err = hipSuccess;
   if (p.B > WR_SMALL_TILE_MAX_B) {
     hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
-                       p.topk_ids, p.topk_w, w.route);
+                       p.topk_ids, p.topk_w, w.route, 0);
     if ((err = hipGetLastError()) != hipSuccess) return err;
   }
   if (p.B <= WR_SMALL_TILE_MAX_B) {

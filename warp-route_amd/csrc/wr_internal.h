@@ -117,7 +117,7 @@ struct BatchRoute {
   int32_t* tok_pair;  // [P] by q: p
   int32_t* off;       // [E + 1]: expert e's pairs are [off[e], off[e + 1])
   int32_t* active;    // [E]: experts with pairs, ascending
-  int32_t* n_active;  // [2]: experts with pairs; how many have more than 32 (k_route)
+  int32_t* n_active;  // [2]: experts with pairs; the call's tile class (k_route)
 };
 
 struct BatchWs {
