@@ -4,25 +4,26 @@
 //
 // The reference's batched kernel runs one warp per token and re-reads every
 // selected expert's weights for every token (src/fused_moe_batched.cu:66-184).
-// Here a call with B tokens is five launches:
-//   1. k_router_logits (wr_kernels.hip): logits[B][64]; it also splits x into
-//      two 16-bit terms.  fp16 terms are of x 2^e_b, with a power of two e_b
-//      per token that puts max|x 2^e_b| in [2^14, 2^15): hi stays finite and
-//      |x 2^e_b - (hi + lo)| <= 2^-22 |x 2^e_b| + 2^-25 (split_exp).
-//   2. k_route: one block selects every token's top-K (the same
-//      wave_select_topk as every other path, so ids and weights are
-//      bit-identical to the single-token op) and groups the (token, expert)
-//      pairs by expert, tokens ascending, with ballot prefix sums
-//      (deterministic, no atomics).  For B <= WR_SMALL_TILE_MAX_B there is
-//      no k_route launch: every gate/up block of step 3 does the same
-//      routing in LDS (route_small), and block (0, 0) publishes it.
+// Here a call with B tokens is these launches:
+//   1. The router, which also splits x into two 16-bit terms (fp16 terms are of
+//      x 2^e_b, with a power of two e_b per token that puts max|x 2^e_b| in
+//      [2^14, 2^15): hi stays finite and |x 2^e_b - (hi + lo)| <= 2^-22
+//      |x 2^e_b| + 2^-25 (split_exp)): k_router_topk (wr_kernels.hip), which
+//      selects every token's top-K as well; for B <= WR_SMALL_TILE_MAX_B
+//      k_router_logits, logits[B][64].
+//   2. k_group: one block groups the (token, expert) pairs by expert, tokens
+//      ascending, with ballot prefix sums (deterministic, no global atomics).
+//      For B <= WR_SMALL_TILE_MAX_B there is no such launch: every gate/up block
+//      of step 3 selects (the same wave_select_topk as every other path, so ids
+//      and weights are bit-identical to the single-token op) and groups in LDS
+//      (route_small), and block (0, 0) publishes it.
 //   3. k_gu_mfma: block (row tile, expert slot): 4 waves x 16 gate rows and
 //      the same 16 up rows each, all of the expert's tokens (up to 64 per
 //      pass); the token tile is staged in LDS and shared by the 4 waves.
-//      Tiles of 16 tokens for B <= 16 and 32 for B <= 32; beyond that both
-//      the 32- and the 64-token kernels are launched and one of them runs,
-//      as k_route's count of experts with more than 32 pairs says
-//      (tile_slot).
+//      Tiles of 16 tokens for B <= 16 and 32 for B <= 32; beyond that the 32-
+//      and 64-token kernels and, for B > 64, the many-token kernels (k_many_gu)
+//      are launched where the pair counts allow them, and one of them runs, as
+//      k_group's largest count says (tile_slot).
 //      v_mfma_f32_16x16x32_f16 with A = weight rows (fp16, or fp8 E4M3 codes
 //      staged as they are and converted exactly to fp16 per fragment) and
 //      B = the hi and lo terms of x; products are exact and accumulate in
@@ -48,10 +49,10 @@
 // is padded to 16 tokens per tile; at 2 MFMAs per product term it stays far
 // below the time the weight stream takes (the path is HBM-bound).
 //
-// Requirements (else the per-token kernels in wr_kernels.hip run): fp16,
-// bf16, fp8 or MXFP4 weights with 16-byte aligned rows, and h and I
-// multiples of 128.  The power-of-two scaling leaves no range condition on x
-// or act beyond fp32's own.
+// Requirements: 16-byte aligned weight rows, and h and I multiples of 128 (fp32
+// weights: 64).  Other layers take the ragged variants (k_rag_gu, k_rag_dn), or
+// the per-token kernels in wr_kernels.hip (grouped_ok).  The power-of-two
+// scaling leaves no range condition on x or act beyond fp32's own.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -69,9 +70,9 @@ namespace {
 #ifndef WR_MID_TILE_MAX_B
 #define WR_MID_TILE_MAX_B 32    // and up to this size 32-token tiles
 #endif
-// Larger batches launch both the 32- and the 64-token tile kernels, and one
-// of them runs (tile_slot): the 32-token one when no expert has more than
-// this many pairs, else the 64-token one, for every expert.  Mixtral, B = 64,
+// Larger batches launch both the 32- and the 64-token tile kernels (and the
+// many-token ones), and one of them runs (tile_slot): the 32-token one when no
+// expert has more than this many pairs, for every expert.  Mixtral, B = 64,
 // per call, in 32-token tiles against 64-token tiles: random routing (26
 // pairs per expert at most) fp16 486 against 527 us, fp8 316 against 346,
 // MXFP4 241 against 290; clustered routing (64 pairs on the pair's experts)
@@ -109,7 +110,7 @@ constexpr int kBM = 64;         // rows per block: 4 waves x 16
 constexpr int kMaxTok = 64;     // tokens per pass, at most: 4 MFMA N tiles
 
 // The expert slot that z (the grid's slot index) runs in a TOK-token tile
-// launch, or -1.  n_active[1] (k_route) is the call's tile class: 0 when no
+// launch, or -1.  n_active[1] (k_group) is the call's tile class: 0 when no
 // expert has more than WR_TILE_SPLIT_M pairs (the 32-token launch takes every
 // slot), 1 when none has more than kMaxTok (the 64-token launch), else 2 (the
 // many-token launch, TOK = kManyTok).  The other launches' blocks leave after
@@ -155,11 +156,8 @@ __device__ __forceinline__ H8 h8zero() {
 }
 
 // ---------------------------------------------------------------------------
-// Routing: one block of 16 waves.  The per-pair selection lives in LDS when it
-// fits (kRouteLds pairs), else in the workspace.
+// Routing
 // ---------------------------------------------------------------------------
-constexpr int kRouteLds = 4096;
-
 // Groups the P = B k selections (sel_id / sel_w, index q = t k + kk) by
 // expert: off[E + 1], active (experts with pairs, ascending), *na, and for
 // pair p (expert-major, tokens ascending within an expert) pair_tok[p] and
@@ -170,8 +168,7 @@ constexpr int kRouteLds = 4096;
 __device__ __forceinline__ void group_pairs(int P, int E, int k, const int* sel_id,
                                             const float* sel_w, int* cnt, int* off_s, int* off,
                                             int* active, int* na, int32_t* pair_tok,
-                                            float* pair_w, int32_t* tok_pair,
-                                            int* cls = nullptr, int max_cls = 2) {
+                                            float* pair_w, int32_t* tok_pair) {
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int nw = blockDim.x / kWave;
@@ -193,14 +190,9 @@ __device__ __forceinline__ void group_pairs(int P, int E, int k, const int* sel_
     }
     off_s[E] = o;
     off[E] = o;
-    int most = 0;
-    for (int e = 0; e < E; ++e) {
+    for (int e = 0; e < E; ++e)
       if (cnt[e] > 0) active[n++] = e;
-      most = max(most, cnt[e]);
-    }
     *na = n;
-    if (cls != nullptr)  // tile_slot
-      *cls = min(max_cls, (most > WR_TILE_SPLIT_M) + (most > kMaxTok));
   }
   __syncthreads();
   // Stable placement: expert e's pairs in token order.
@@ -221,27 +213,41 @@ __device__ __forceinline__ void group_pairs(int P, int E, int k, const int* sel_
   }
 }
 
-__global__ __launch_bounds__(1024) void k_route(const float* __restrict__ logits, int B, int E,
-                                                int k, int renorm, int32_t* __restrict__ ids_out,
-                                                float* __restrict__ w_out, BatchRoute r,
-                                                int max_cls) {
-  __shared__ int s_cnt[WR_MAX_EXPERTS];
-  __shared__ int s_off[WR_MAX_EXPERTS + 1];
-  __shared__ int s_id[kRouteLds];
-  __shared__ float s_w[kRouteLds];
-  const int lane = threadIdx.x & (kWave - 1);
-  const int wave = threadIdx.x / kWave;
-  const int nw = blockDim.x / kWave;
-  const int P = B * k;
-  int* sel_id = P <= kRouteLds ? s_id : r.sel_id;
-  float* sel_w = P <= kRouteLds ? s_w : r.sel_w;
-
-  // Selection.  E <= 16: four tokens per wave at once, one per 16-lane row
-  // (row_select_topk).  Else lane e holds logit e, and a wave's next 4 tokens
-  // are loaded at once.
-  if (E <= 16) {
-    const int row = lane >> 4, li = lane & 15;
-    for (int t0 = 4 * wave; t0 < B; t0 += 4 * nw) {  // wave-uniform bound
+// Groups the P selections that k_router_topk left in r.sel_id / r.sel_w by
+// expert, as group_pairs does, and names the call's tile class (tile_slot).
+// One block of 16 waves, each with an equal run of 64-pair chunks in order.  A
+// lane finds the lanes of its chunk with its expert from one ballot per id bit,
+// so a chunk costs the same for any number of experts (one ballot per expert
+// and chunk before: B = 256, E = 64, k = 6 about 5 us).
+//
+// logits set (E <= 16): the block first selects from them, four tokens per wave
+// at once, one per 16-lane row (row_select_topk), also to ids_out / w_out when
+// set.
+__global__ __launch_bounds__(1024) void k_group(int P, int E, int k, BatchRoute r, int max_cls,
+                                                const float* __restrict__ logits, int renorm,
+                                                int32_t* __restrict__ ids_out,
+                                                float* __restrict__ w_out) {
+  constexpr int NW = 1024 / kWave;
+  __shared__ int base[NW][WR_MAX_EXPERTS];  // counts, then next positions, per wave
+  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+  const int chunks = (P + kWave - 1) / kWave, per = (chunks + NW - 1) / NW;
+  const int c0 = wave * per, c1 = min(chunks, c0 + per);
+  volatile int* mine = base[wave];
+  mine[lane] = 0;
+  // The lanes with this lane's id (valid lanes only).
+  auto same = [&](int id, bool valid) {
+    uint64_t m = __ballot(valid);
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+      const uint64_t s = __ballot((id >> b) & 1);
+      m &= (id >> b) & 1 ? s : ~s;
+    }
+    return m;
+  };
+  static_assert(WR_MAX_EXPERTS <= 64, "six id bits");
+  if (logits != nullptr) {
+    const int row = lane >> 4, li = lane & 15, B = P / k;
+    for (int t0 = 4 * wave; t0 < B; t0 += 4 * NW) {  // wave-uniform bound
       const int t = t0 + row;
       const float l = t < B ? logits[(int64_t)t * WR_MAX_EXPERTS + li] : 0.0f;
       int sid;
@@ -249,45 +255,83 @@ __global__ __launch_bounds__(1024) void k_route(const float* __restrict__ logits
       row_select_topk(l, E, k, renorm, sid, sw);
       if (t < B && li < k) {
         const int q = t * k + li;
-        sel_id[q] = sid;
-        sel_w[q] = sw;
+        r.sel_id[q] = sid;
+        r.sel_w[q] = sw;
         if (ids_out != nullptr) ids_out[q] = sid;
         if (w_out != nullptr) w_out[q] = sw;
       }
     }
-  } else {
-    for (int t0 = wave; t0 < B; t0 += 4 * nw) {
-      float l[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = t0 + i * nw;
-        l[i] = t < B ? logits[(int64_t)t * WR_MAX_EXPERTS + lane] : 0.0f;
+    __syncthreads();
+  }
+  const uint64_t below = (1ull << lane) - 1ull;
+  for (int c = c0; c < c1; ++c) {
+    const int q = c * kWave + lane;
+    const bool valid = q < P;
+    const int id = valid ? r.sel_id[q] : 0;
+    const uint64_t m = same(id, valid);
+    if (valid && (m & below) == 0) mine[id] = mine[id] + __popcll(m);
+  }
+  __syncthreads();
+  if (wave == 0) {
+    int tot = 0;
+    if (lane < E) {
+      for (int w = 0; w < NW; ++w) {
+        const int v = base[w][lane];
+        base[w][lane] = tot;
+        tot += v;
       }
+    }
+    int incl = tot;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int t = t0 + i * nw;
-        if (t < B) {  // wave-uniform
-          TopK tk;
-          wave_select_topk_reg(l[i], E, k, renorm, tk);
-          if (lane < k) {
-            const int q = t * k + lane;
-            sel_id[q] = tk.lid;
-            sel_w[q] = tk.lw;
-            if (ids_out != nullptr) ids_out[q] = tk.lid;
-            if (w_out != nullptr) w_out[q] = tk.lw;
-          }
-        }
-      }
+    for (int d = 1; d < kWave; d *= 2) {
+      const int v = __shfl_up(incl, d);
+      if (lane >= d) incl += v;
+    }
+    const int off = incl - tot;
+    const uint64_t act = __ballot(tot > 0);
+    if (lane < E) {
+      for (int w = 0; w < NW; ++w) base[w][lane] += off;
+      r.off[lane] = off;
+      if (tot > 0) r.active[__popcll(act & below)] = lane;
+    }
+    const int cls = __ballot(tot > kMaxTok) ? 2 : __ballot(tot > WR_TILE_SPLIT_M) ? 1 : 0;
+    if (lane == 0) {
+      r.off[E] = P;
+      r.n_active[0] = __popcll(act);
+      r.n_active[1] = min(max_cls, cls);
     }
   }
   __syncthreads();
-  group_pairs(P, E, k, sel_id, sel_w, s_cnt, s_off, r.off, r.active, r.n_active, r.pair_tok,
-              r.pair_w, r.tok_pair, r.n_active + 1, max_cls);
+  for (int c = c0; c < c1; ++c) {
+    const int q = c * kWave + lane;
+    const bool valid = q < P;
+    const int id = valid ? r.sel_id[q] : 0;
+    const uint64_t m = same(id, valid);
+    const int pos = mine[id] + __popcll(m & below);
+    if (valid) {
+      if ((m & below) == 0) mine[id] = pos + __popcll(m);
+      r.pair_tok[pos] = q / k;
+      r.pair_w[pos] = r.sel_w[q];
+      r.tok_pair[q] = pos;
+    }
+  }
+}
+
+// Few tokens and experts: k_router_logits, a block per logit, and the selection
+// in k_group; else k_router_topk.  Measured, us, router + grouping launches: E 16,
+// h 6144, B = 32 13.3 against 17.0; E 8, h 4096, B = 64 10.7 against 12.0; B = 512
+// 30 against 15; E 64, h 2048, B = 256 96 against 20.
+bool select_in_group(const Problem& p) { return p.E <= 16 && p.B <= 64; }
+
+hipError_t launch_group(const Problem& p, const BatchWs& w, int max_cls, hipStream_t s) {
+  hipLaunchKernelGGL(k_group, dim3(1), dim3(1024), 0, s, p.B * p.k, p.E, p.k, w.route, max_cls,
+                     select_in_group(p) ? w.logits : nullptr, p.renorm, p.topk_ids, p.topk_w);
+  return hipGetLastError();
 }
 
 // In-block routing for small batches (B <= WR_SMALL_TILE_MAX_B): every
 // gate/up block selects the B tokens' experts and groups the pairs itself,
-// in LDS, instead of waiting for a separate k_route launch.  The selection
+// in LDS, instead of waiting for separate launches.  The selection
 // is the same wave_select_topk_reg, so ids and weights are bit-identical.
 constexpr int kSmallPairs = WR_SMALL_TILE_MAX_B * WR_MAX_TOPK;
 struct SmallRoute {
@@ -1003,7 +1047,7 @@ constexpr int gu_min_blocks() {
 }
 
 // ROUTE: the block routes the batch itself (route_small) instead of reading
-// k_route's output; block (0, 0) publishes the routing for the later kernels.
+// k_group's output; block (0, 0) publishes the routing for the later kernels.
 template <typename WT, bool LO, int TOK, bool ROUTE, int KC, int WK, bool RAG, bool L2>
 __device__ __forceinline__ void gu_block(const WT* __restrict__ wbuf,
                                          const f16* __restrict__ x_hi,
@@ -2377,9 +2421,7 @@ hipError_t ragged_t(const Problem& p, const BatchWs& w, hipStream_t s) {
   const int tile = rag_tile(p);
   hipError_t err = hipSuccess;
   if (tile > 16) {
-    hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
-                       p.topk_ids, p.topk_w, w.route, 0);
-    if ((err = hipGetLastError()) != hipSuccess) return err;
+    if ((err = launch_group(p, w, 0, s)) != hipSuccess) return err;
   }
   const dim3 gg(g.Ip / kBM, slots), gd((p.h + kBM - 1) / kBM, BatchWs::kKSplit, slots);
   constexpr bool L2 = std::is_same<XT, float>::value;  // fp16 x: two terms hold all of it
@@ -2403,9 +2445,7 @@ hipError_t ragged_f32(const Problem& p, const BatchWs& w, hipStream_t s) {
   const int tile = rag_tile(p);
   hipError_t err = hipSuccess;
   if (tile > 16) {
-    hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
-                       p.topk_ids, p.topk_w, w.route, 0);
-    if ((err = hipGetLastError()) != hipSuccess) return err;
+    if ((err = launch_group(p, w, 0, s)) != hipSuccess) return err;
   }
   const dim3 gg(g.Ip / kBM, slots), gd((p.h + kBM - 1) / kBM, BatchWs::kKSplit, slots);
   auto gu = tile == 16 ? k_rag_gu_f32<16, true>
@@ -2431,9 +2471,7 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
   const bool many = p.B > kMaxTok && (int64_t)p.B * p.h * 4 < (int64_t{1} << 32);
   // Small batches route inside the gate/up kernel (one launch fewer).
   if (p.B > WR_SMALL_TILE_MAX_B) {
-    hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
-                       p.topk_ids, p.topk_w, w.route, many ? 2 : 1);
-    if ((err = hipGetLastError()) != hipSuccess) return err;
+    if ((err = launch_group(p, w, many ? 2 : 1, s)) != hipSuccess) return err;
   }
   // The lo term of x: fp32 x, or any x against bf16 (8-bit mantissa) terms.
   constexpr bool LO = std::is_same<XT, float>::value || bf16_ops<WT>();
@@ -2540,9 +2578,7 @@ hipError_t grouped_f32(const Problem& p, const BatchWs& w, hipStream_t s) {
   const XT* x = static_cast<const XT*>(p.x);
   hipError_t err = hipSuccess;
   if (p.B > WR_SMALL_TILE_MAX_B) {
-    hipLaunchKernelGGL(k_route, dim3(1), dim3(1024), 0, s, w.logits, p.B, p.E, p.k, p.renorm,
-                       p.topk_ids, p.topk_w, w.route, 0);
-    if ((err = hipGetLastError()) != hipSuccess) return err;
+    if ((err = launch_group(p, w, 0, s)) != hipSuccess) return err;
   }
   if (p.B <= WR_SMALL_TILE_MAX_B) {
     hipLaunchKernelGGL((k_gu_f32<XT, 16, true>), dim3(p.I / kBM, slots), dim3(kBlk), 0, s, wb, x,
@@ -2594,6 +2630,14 @@ bool grouped_ok(const Problem& p) {
   return 2 * pairs >= 3 * p.E && pairs * p.stride_b > tiny;
 }
 
+// The router launch: with the selection for larger batches (small ones select
+// in every gate/up block, one launch fewer).
+static hipError_t launch_router(const Problem& p, const BatchWs& w, const XSplit& xs, hipStream_t s) {
+  return p.B > WR_SMALL_TILE_MAX_B && !select_in_group(p)
+             ? launch_router_topk(p, w.route.sel_id, w.route.sel_w, xs, s)
+             : launch_logits_split(p, w.logits, xs, s);
+}
+
 hipError_t launch_grouped(const Problem& p, hipStream_t s) {
   const BatchWs w = BatchWs::carve(p.ws, p.E, p.h, p.I, p.k, p.B);
   const bool ragged = !aligned_ok(p);
@@ -2601,12 +2645,12 @@ hipError_t launch_grouped(const Problem& p, hipStream_t s) {
     XSplit xs = x_split(p);
     xs.f32 = w.x_f32();
     xs.ld = BatchWs::padded(p.h);
-    hipError_t err = launch_logits_split(p, w.logits, xs, s);
+    hipError_t err = launch_router(p, w, xs, s);
     if (err != hipSuccess) return err;
     return p.adt == WR_F16 ? ragged_f32<f16>(p, w, s) : ragged_f32<float>(p, w, s);
   }
   if (p.wdt == WR_F32) {  // exact fp32 products: x as it is, logits only
-    hipError_t err = launch_logits(p, w.logits, s);
+    hipError_t err = launch_router(p, w, x_split(p), s);
     if (err != hipSuccess) return err;
     return p.adt == WR_F16 ? grouped_f32<f16>(p, w, s) : grouped_f32<float>(p, w, s);
   }
@@ -2620,7 +2664,7 @@ hipError_t launch_grouped(const Problem& p, hipStream_t s) {
   xs.amax = bf ? nullptr : w.amax;
   xs.bf16 = bf ? 1 : 0;
   xs.ld = ragged ? BatchWs::padded(p.h) : p.h;
-  hipError_t err = launch_logits_split(p, w.logits, xs, s);
+  hipError_t err = launch_router(p, w, xs, s);
   if (err != hipSuccess) return err;
   if (ragged) {
     if (p.wdt == WR_FP8_E4M3)

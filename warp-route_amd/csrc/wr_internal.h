@@ -117,7 +117,7 @@ struct BatchRoute {
   int32_t* tok_pair;  // [P] by q: p
   int32_t* off;       // [E + 1]: expert e's pairs are [off[e], off[e + 1])
   int32_t* active;    // [E]: experts with pairs, ascending
-  int32_t* n_active;  // [2]: experts with pairs; the call's tile class (k_route)
+  int32_t* n_active;  // [2]: experts with pairs; the call's tile class (k_group)
 };
 
 struct BatchWs {
@@ -240,6 +240,10 @@ inline XSplit x_split(const Problem& p) {
 }
 // Logits and, with them, x as xs asks.
 hipError_t launch_logits_split(const Problem& p, float* logits, const XSplit& xs, hipStream_t s);
+// Router, top-K (to p.topk_ids / topk_w when set, and to sel_id / sel_w when set)
+// and x as xs asks, in one launch.
+hipError_t launch_router_topk(const Problem& p, int32_t* sel_id, float* sel_w, const XSplit& xs,
+                              hipStream_t s);
 // Grouped batched path: usable when grouped_ok(p).
 bool grouped_ok(const Problem& p);
 hipError_t launch_grouped(const Problem& p, hipStream_t s);

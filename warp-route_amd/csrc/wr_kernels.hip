@@ -202,6 +202,34 @@ __device__ __forceinline__ float router_combine(const float* p) {
   return (p[0] + p[1]) + (p[2] + p[3]);
 }
 
+// Elements i, i + step, ... < end of token b's row, written as xs asks; ex: the
+// row's exponent (fp16 terms).
+template <typename XT>
+__device__ __forceinline__ void write_x_split(const XSplit& xs, const XT* __restrict__ xb,
+                                              int64_t b, int h, int i, int end, int step, int ex) {
+  for (; i < end; i += step) {
+    const float v = i < h ? (float)xb[i] : 0.0f;
+    const int64_t o = b * xs.ld + i;
+    if (xs.bf16) {
+      const __bf16 bh = (__bf16)v;
+      const __bf16 bl = (__bf16)(v - (float)bh);
+      xs.hi[o] = __builtin_bit_cast(f16, bh);
+      xs.lo[o] = __builtin_bit_cast(f16, bl);
+      if (xs.l2 != nullptr)
+        xs.l2[o] = __builtin_bit_cast(f16, (__bf16)(v - (float)bh - (float)bl));
+    } else if (xs.f32 != nullptr) {
+      xs.f32[o] = v;
+    } else {
+      const float vs = ldexpf(v, ex);
+      const f16 vh = (f16)vs;
+      const f16 vl = (f16)(vs - (float)vh);
+      xs.hi[o] = vh;
+      xs.lo[o] = vl;
+      if (xs.l2 != nullptr) xs.l2[o] = (f16)(vs - (float)vh - (float)vl);
+    }
+  }
+}
+
 // grid (E, B), block 256.  Token b's logits go to logits[b * 64 + e] (padded
 // so that consumers can read all 64 with scalar loads).  Block (0, 0) also
 // zeroes the 8-byte words at zero + i * zstride, i < nzero <= kBlock (the
@@ -239,27 +267,7 @@ __global__ __launch_bounds__(kBlock) void k_router_logits(const float* __restric
                           : 0;
     const int cs = (xs.ld + E - 1) / E;
     const int end = min(xs.ld, (e + 1) * cs);
-    for (int i = e * cs + (int)threadIdx.x; i < end; i += kBlock) {
-      const float v = i < h ? (float)xb[i] : 0.0f;
-      const int64_t o = (int64_t)b * xs.ld + i;
-      if (xs.bf16) {
-        const __bf16 bh = (__bf16)v;
-        const __bf16 bl = (__bf16)(v - (float)bh);
-        xs.hi[o] = __builtin_bit_cast(f16, bh);
-        xs.lo[o] = __builtin_bit_cast(f16, bl);
-        if (xs.l2 != nullptr)
-          xs.l2[o] = __builtin_bit_cast(f16, (__bf16)(v - (float)bh - (float)bl));
-      } else if (xs.f32 != nullptr) {
-        xs.f32[o] = v;
-      } else {
-        const float vs = ldexpf(v, ex);
-        const f16 vh = (f16)vs;
-        const f16 vl = (f16)(vs - (float)vh);
-        xs.hi[o] = vh;
-        xs.lo[o] = vl;
-        if (xs.l2 != nullptr) xs.l2[o] = (f16)(vs - (float)vh - (float)vl);
-      }
-    }
+    write_x_split<XT>(xs, xb, b, h, e * cs + (int)threadIdx.x, end, kBlock, ex);
     if (e == 0) {
       if (threadIdx.x == 0 && xs.exp != nullptr) xs.exp[b] = ex;
       if (xs.amax != nullptr && (int)threadIdx.x < xs.k)
@@ -268,37 +276,196 @@ __global__ __launch_bounds__(kBlock) void k_router_logits(const float* __restric
   }
 }
 
-// Standalone gate: grid B, block 1024 (four 4-wave groups).  Group g handles
-// experts g, g+4, ...; wave 0 then selects and writes ids and weights.
-template <typename XT, int VEC>
-__global__ __launch_bounds__(1024) void k_gate_topk(const float* __restrict__ gate_w,
-                                                    const XT* __restrict__ x, int E, int h,
-                                                    int k, int renorm,
-                                                    int32_t* __restrict__ ids_out,
-                                                    float* __restrict__ w_out) {
-  __shared__ float part[WR_MAX_EXPERTS][4];
-  const int wave = threadIdx.x / kWave;
-  const int lane = threadIdx.x & (kWave - 1);
-  const int g = wave / 4, q = wave % 4;
-  const int b = blockIdx.x;
-  for (int e = g; e < E; e += 4) {
-    float unused;
-    const float p =
-        router_partial<XT, VEC>(gate_w + (int64_t)e * h, x + (int64_t)b * h, h, q, false, unused);
-    if (lane == 0) part[e][q] = p;
-  }
-  __syncthreads();
-  if (wave == 0) {
-    const float l = lane < E ? router_combine(part[lane]) : 0.0f;
-    TopK t;
-    wave_select_topk_reg(l, E, k, renorm, t);
+// The same for a whole row, eight elements per thread and round (h % 8 == 0, x
+// rows in 4-element loads): one element each took a dependent load per 1024
+// columns, 3 us of a launch at h = 6144.
+template <typename XT>
+__device__ __forceinline__ void write_x_split8(const XSplit& xs, const XT* __restrict__ xb,
+                                               int64_t b, int h, int ex) {
+  for (int i = 8 * (int)threadIdx.x; i < h; i += 8 * (int)blockDim.x) {
+    float v[8];
+    load_x<XT, 4>(xb + i, *reinterpret_cast<float(*)[4]>(v));
+    load_x<XT, 4>(xb + i + 4, *reinterpret_cast<float(*)[4]>(v + 4));
+    const int64_t o = b * xs.ld + i;
+    if (xs.f32 != nullptr) {
 #pragma unroll
-    for (int kk = 0; kk < WR_MAX_TOPK; ++kk) {
-      if (kk < k && lane == kk) {
-        ids_out[(int64_t)b * k + kk] = t.id[kk];
-        w_out[(int64_t)b * k + kk] = t.w[kk];
+      for (int q = 0; q < 2; ++q)
+        *reinterpret_cast<f32x4*>(xs.f32 + o + 4 * q) =
+            f32x4{v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]};
+      continue;
+    }
+    f16x8 hi, lo, l2;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if (xs.bf16) {
+        const __bf16 bh = (__bf16)v[e];
+        const __bf16 bl = (__bf16)(v[e] - (float)bh);
+        hi[e] = __builtin_bit_cast(f16, bh);
+        lo[e] = __builtin_bit_cast(f16, bl);
+        l2[e] = __builtin_bit_cast(f16, (__bf16)(v[e] - (float)bh - (float)bl));
+      } else {
+        const float vs = ldexpf(v[e], ex);
+        hi[e] = (f16)vs;
+        lo[e] = (f16)(vs - (float)hi[e]);
+        l2[e] = (f16)(vs - (float)hi[e] - (float)lo[e]);
       }
     }
+    *reinterpret_cast<f16x8*>(xs.hi + o) = hi;
+    *reinterpret_cast<f16x8*>(xs.lo + o) = lo;
+    if (xs.l2 != nullptr) *reinterpret_cast<f16x8*>(xs.l2 + o) = l2;
+  }
+}
+
+// Router and selection of T tokens per block: grid ceil(B / T), block 1024.
+// Wave 4 g + q computes quarter q of the logits of experts 4 g .. 4 g + 3, then
+// 16 more on, for all T tokens at once, so that a loaded piece of x serves four
+// experts and a piece of a router row T tokens.  Each dot product is summed
+// exactly as router_partial's (lane chunks of VEC columns, chunk j into sum j
+// mod 4), so the logits have the same bits.  Wave t then selects token t's
+// experts: ids and weights to ids_out / w_out (when set) and to sel_id / sel_w
+// (when set), [B][k].  Writes of x as in k_router_logits.  Bound by latency: a
+// load round per chunk, and the k selection rounds.  gate_topk, E 64, k 6, h
+// 2048, with one expert per four waves before, us: B = 4 14.7 -> 10.1, B = 256
+// 16.3 -> 11.7, B = 512 29.0 -> 15.6; in batched calls of more than 16 tokens, the
+// selection of all tokens was one block's work (B = 256: router 21 + k_route 75
+// -> 14 + k_group 5.4).
+template <typename XT, int VEC, int T>
+__global__ __launch_bounds__(1024) void k_router_topk(const float* __restrict__ gate_w,
+                                                      const XT* __restrict__ x, int B, int E,
+                                                      int h, int k, int renorm,
+                                                      int32_t* __restrict__ ids_out,
+                                                      float* __restrict__ w_out,
+                                                      int32_t* __restrict__ sel_id,
+                                                      float* __restrict__ sel_w, XSplit xs) {
+  constexpr int CH = kWave * VEC, NE = 4;
+  __shared__ float part[T][WR_MAX_EXPERTS][4];
+  __shared__ float pmax[T][4];
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kWave);
+  const int q = wave & 3, grp = wave >> 2;
+  const int b0 = blockIdx.x * T;
+  const int span = (h + 4 * CH - 1) / (4 * CH) * CH;
+  const int beg = q * span, end = min(h, beg + span);
+  const bool scaled = xs.hi != nullptr && !xs.bf16;
+  const XT* xr[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) xr[t] = x + (int64_t)min(b0 + t, B - 1) * h;
+#pragma unroll 1
+  for (int e0 = NE * grp; e0 < E; e0 += 4 * NE) {
+    const float* wr[NE];
+#pragma unroll
+    for (int i = 0; i < NE; ++i) wr[i] = gate_w + (int64_t)min(e0 + i, E - 1) * h;
+    float acc[NE][T][4];
+    float m[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      m[t] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < NE; ++i) acc[i][t][0] = acc[i][t][1] = acc[i][t][2] = acc[i][t][3] = 0.0f;
+    }
+    const bool want_max = scaled && e0 == 0;
+    // Chunk j adds to sum j mod 4: the sums rotate.  U chunks' loads at once.
+    constexpr int U = T == 1 ? 4 : 2;
+    const int chunks = end > beg ? (end - beg + CH - 1) / CH : 0;
+#pragma unroll 1
+    for (int j = 0; j < chunks; j += U) {
+      float wv[U][NE][VEC], xv[U][T][VEC];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        // Past the end: valid columns, as zeros below.
+        const int cc = min(beg + (j + u) * CH + lane * VEC, end - VEC);
+#pragma unroll
+        for (int i = 0; i < NE; ++i) load_x<float, VEC>(wr[i] + cc, wv[u][i]);
+#pragma unroll
+        for (int t = 0; t < T; ++t) load_x<XT, VEC>(xr[t] + cc, xv[u][t]);
+      }
+      __builtin_amdgcn_sched_barrier(0);  // all of them before the sums
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (j + u >= chunks) break;  // wave-uniform
+        const bool in = beg + (j + u) * CH + lane * VEC < end;
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+#pragma unroll
+          for (int v = 0; v < VEC; ++v) {
+            xv[u][t][v] = in ? xv[u][t][v] : 0.0f;
+            m[t] = fmaxf(m[t], fabsf(xv[u][t][v]));
+          }
+#pragma unroll
+          for (int i = 0; i < NE; ++i) {
+            float a = acc[i][t][0];
+#pragma unroll
+            for (int v = 0; v < VEC; ++v)
+              a = fmaf(in ? wv[u][i][v] : 0.0f, xv[u][t][v], a);
+            acc[i][t][0] = acc[i][t][1];
+            acc[i][t][1] = acc[i][t][2];
+            acc[i][t][2] = acc[i][t][3];
+            acc[i][t][3] = a;
+          }
+        }
+      }
+    }
+#pragma unroll 1
+    for (int j = chunks; j % 4 != 0; ++j) {  // back to their places
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int i = 0; i < NE; ++i) {
+          const float a = acc[i][t][0];
+          acc[i][t][0] = acc[i][t][1];
+          acc[i][t][1] = acc[i][t][2];
+          acc[i][t][2] = acc[i][t][3];
+          acc[i][t][3] = a;
+        }
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+#pragma unroll
+      for (int i = 0; i < NE; ++i) {
+        const float p =
+            wave_sum((acc[i][t][0] + acc[i][t][1]) + (acc[i][t][2] + acc[i][t][3]));
+        if (lane == 0 && e0 + i < E) part[t][e0 + i][q] = p;
+      }
+      if (want_max) {
+        const float mx = wave_max(m[t]);
+        if (lane == 0) pmax[t][q] = mx;
+      }
+    }
+  }
+  __syncthreads();
+  if (wave < T && b0 + wave < B) {
+    const int64_t b = b0 + wave;
+    const float l = lane < E ? router_combine(part[wave][lane]) : 0.0f;
+    TopK t;
+    wave_select_topk_reg(l, E, k, renorm, t);
+    if (lane < k) {
+      const int64_t o = b * k + lane;
+      if (ids_out != nullptr) ids_out[o] = t.lid;
+      if (w_out != nullptr) w_out[o] = t.lw;
+      if (sel_id != nullptr) sel_id[o] = t.lid;
+      if (sel_w != nullptr) sel_w[o] = t.lw;
+    }
+  }
+  if (xs.hi == nullptr && xs.f32 == nullptr) return;
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int64_t b = b0 + t;
+    if (b >= B) break;
+    const int ex = scaled ? split_exp(fmaxf(fmaxf(pmax[t][0], pmax[t][1]),
+                                            fmaxf(pmax[t][2], pmax[t][3])),
+                                      std::is_same<XT, f16>::value)
+                          : 0;
+    int rest = 0;  // columns not yet written
+    if constexpr (VEC == 4) {
+      if (h % 8 == 0) {
+        write_x_split8<XT>(xs, xr[t], b, h, ex);
+        rest = h;
+      }
+    }
+    write_x_split<XT>(xs, xr[t], b, h, rest + threadIdx.x, xs.ld, 1024, ex);
+    if (threadIdx.x == 0 && xs.exp != nullptr) xs.exp[b] = ex;
+    if (xs.amax != nullptr && (int)threadIdx.x < xs.k)
+      xs.amax[(b * xs.k + threadIdx.x) * BatchWs::kAmaxStride] = 0u;
   }
 }
 
@@ -2106,16 +2273,27 @@ hipError_t run_ffn(const Problem& p, hipStream_t s) {
   return run_ffn_only(p, nullptr, s);
 }
 
-template <typename XT>
-hipError_t gate_t(const Problem& p, hipStream_t s) {
+// Two tokens per block when one each would be more blocks than CUs.  gate_topk,
+// us, 1 / 2 / 4 tokens per block: E 64, h 2048, B = 256 11.7 / 14.5 / 23.5, B =
+// 512 18.4 / 15.6 / 24.1; E 16, h 6144 8.4 / 9.3 / 12.2 and 13.3 / 10.6 / 13.9.
+template <typename XT, int VEC>
+hipError_t router_topk_v(const Problem& p, int32_t* sel_id, float* sel_w, const XSplit& xs,
+                         hipStream_t s) {
   const XT* x = static_cast<const XT*>(p.x);
-  if (router_vec4(p))
-    hipLaunchKernelGGL((k_gate_topk<XT, 4>), dim3(p.B), dim3(1024), 0, s, p.gate_w, x, p.E, p.h,
-                       p.k, p.renorm, p.topk_ids, p.topk_w);
+  if (p.B > cu_count())
+    hipLaunchKernelGGL((k_router_topk<XT, VEC, 2>), dim3((p.B + 1) / 2), dim3(1024), 0, s,
+                       p.gate_w, x, p.B, p.E, p.h, p.k, p.renorm, p.topk_ids, p.topk_w, sel_id,
+                       sel_w, xs);
   else
-    hipLaunchKernelGGL((k_gate_topk<XT, 1>), dim3(p.B), dim3(1024), 0, s, p.gate_w, x, p.E, p.h,
-                       p.k, p.renorm, p.topk_ids, p.topk_w);
+    hipLaunchKernelGGL((k_router_topk<XT, VEC, 1>), dim3(p.B), dim3(1024), 0, s, p.gate_w, x, p.B,
+                       p.E, p.h, p.k, p.renorm, p.topk_ids, p.topk_w, sel_id, sel_w, xs);
   return hipGetLastError();
+}
+template <typename XT>
+hipError_t router_topk_t(const Problem& p, int32_t* sel_id, float* sel_w, const XSplit& xs,
+                         hipStream_t s) {
+  return router_vec4(p) ? router_topk_v<XT, 4>(p, sel_id, sel_w, xs, s)
+                        : router_topk_v<XT, 1>(p, sel_id, sel_w, xs, s);
 }
 
 }  // namespace
@@ -2125,8 +2303,14 @@ hipError_t launch_logits(const Problem& p, float* logits, hipStream_t s) {
                          : logits_t<float>(p, logits, nullptr, 0, 0, s);
 }
 
+hipError_t launch_router_topk(const Problem& p, int32_t* sel_id, float* sel_w, const XSplit& xs,
+                              hipStream_t s) {
+  return p.adt == WR_F16 ? router_topk_t<f16>(p, sel_id, sel_w, xs, s)
+                         : router_topk_t<float>(p, sel_id, sel_w, xs, s);
+}
+
 hipError_t launch_gate_topk(const Problem& p, hipStream_t s) {
-  return p.adt == WR_F16 ? gate_t<f16>(p, s) : gate_t<float>(p, s);
+  return launch_router_topk(p, nullptr, nullptr, x_split(p), s);
 }
 
 hipError_t launch_fused(const Problem& p, hipStream_t s) { return run_ffn(p, s); }
