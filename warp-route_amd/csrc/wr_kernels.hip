@@ -5,8 +5,10 @@
 // wave covers a quarter of the row, so one memory round trip covers it.
 // Every consumer then derives the top-K selection from the logits itself
 // (wave_select_topk: DPP max/sum and a 64-bit ballot).  For layers of many
-// gate/up blocks the single-token kernel computes the router rows itself
-// instead (route_and_select), one launch per layer as in the reference.
+// gate/up blocks, or of at most one block per CU, the single-token kernel
+// computes the router rows itself instead (route_and_select), one launch per
+// layer as in the reference.  Batches beyond 16 tokens and gate_topk take
+// k_router_topk: logits, selection and x's terms, a block per token.
 //
 // Single token (the decode hot path): k_fused_ffn, ONE launch whose first
 // blocks stream the selected experts' gate/up rows and write
@@ -1967,7 +1969,7 @@ uint64_t* tl_ptr() {
 #endif
 
 // Gate/up slots per CU from which the register-path kernel takes the router
-// inside (one launch per layer).
+// inside (one launch per layer); layers with at most one block per CU do too.
 constexpr int kFoldSlotsPerCu = 2;
 
 // fold == nullptr: the kernel reads the logits an earlier router launch left
@@ -2103,11 +2105,14 @@ hipError_t fused_rpw_t(const Problem& p, const FusedWs& w, bool* fold, hipStream
     if (fold != nullptr) {
       // The router inside the kernel (route_and_select) pays for layers of
       // at least kFoldSlotsPerCu gate/up slots per CU, whose gate/up phase
-      // spans rounds of resident blocks; smaller layers keep the router
-      // launch.  Measured (layer us): Mixtral 114.50 -> 113.54, DBRX 240.5 ->
-      // 239.4, Mixtral tp4 shard 42.96 -> 42.53 folded; tp8 shard 27.03 ->
-      // 27.74 and DeepSeek (claiming variant) 25.51 -> 26.37 would lose.
-      *fold = hs.n1 >= kFoldSlotsPerCu * cu_count();
+      // spans rounds of resident blocks.  Measured (layer us): Mixtral 114.50
+      // -> 113.54, DBRX 240.5 -> 239.4, Mixtral tp4 shard 42.96 -> 42.53
+      // folded; tp8 shard 27.03 -> 27.74 and DeepSeek (claiming variant) 25.51
+      // -> 26.37 would lose.  It also pays for layers of at most one block per
+      // CU, where no poll shares a CU with a router row or delays a weight
+      // load: fp32, E 8, h 256, I 512, k 2 (192 blocks) 8.84 -> 7.66 us.
+      // Layers between the two keep the router launch.
+      *fold = hs.n1 >= kFoldSlotsPerCu * cu_count() || hs.nb <= cu_count();
       if (!*fold) return hipSuccess;
       hipLaunchKernelGGL((k_fused_ffn<WT, XT, VEC, RPW, U1, RPD, U2, false, false, false, true>),
                          dim3(hs.n1 + n2), dim3(kBlock), 0, s, static_cast<const WT*>(p.wbuf),
