@@ -119,7 +119,6 @@ constexpr int kManyTok = 2 * kMaxTok;  // marks the many-token launch
 template <int TOK>
 __device__ __forceinline__ int tile_slot(const BatchRoute& r, int z) {
   static_assert(TOK == 16 || TOK == 32 || TOK == kMaxTok || TOK == kManyTok, "tile sizes");
-  static_assert(WR_MID_TILE_MAX_B <= WR_TILE_SPLIT_M, "32-token batches lead with no 64-token class");
   if constexpr (TOK == 16) {
     return z < r.n_active[0] ? z : -1;
   } else {
@@ -2469,14 +2468,18 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
   hipError_t err = hipSuccess;
   // The many-token kernels address x's two terms with 32-bit offsets.
   const bool many = p.B > kMaxTok && (int64_t)p.B * p.h * 4 < (int64_t{1} << 32);
-  // Small batches route inside the gate/up kernel (one launch fewer).
+  const bool mid = p.B <= WR_MID_TILE_MAX_B;
+  // Small batches route inside the gate/up kernel (one launch fewer).  The
+  // largest class is that of the kernels launched below, whatever the counts: a
+  // token without a finite logit selects expert 0 in all k slots, so an expert
+  // can have up to B k pairs (every kernel takes any number, in passes).
   if (p.B > WR_SMALL_TILE_MAX_B) {
-    if ((err = launch_group(p, w, many ? 2 : 1, s)) != hipSuccess) return err;
+    if ((err = launch_group(p, w, mid ? 0 : (many ? 2 : 1), s)) != hipSuccess) return err;
   }
   // The lo term of x: fp32 x, or any x against bf16 (8-bit mantissa) terms.
   constexpr bool LO = std::is_same<XT, float>::value || bf16_ops<WT>();
-  // An expert has at most B tokens (a token selects it at most once), so
-  // small batches take token tiles of 16 or 32.
+  // An expert has at most B tokens with finite logits (such a token selects it
+  // at most once), so small batches take token tiles of 16 or 32.
   if (p.B <= WR_SMALL_TILE_MAX_B) {
     // 16-token tiles: the wide K steps (kc_wide) where the K dimension (h for
     // gate/up, I for down) is a multiple of them.
@@ -2504,10 +2507,9 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
     // 168 us and bf16 161 -> 165 us (the launch costs more than the repeated
     // splits of 32-token tiles).
     constexpr bool kPre32 = wbits<WT>() < 16;
-    // The classes (tile_slot) that the call can be of: an expert has at most B
-    // tokens, and with more than n pairs per expert on average one has more
-    // than n.  One of the launches made runs.
-    const bool mid = p.B <= WR_MID_TILE_MAX_B;
+    // The classes (tile_slot) that the call can be of: up to WR_MID_TILE_MAX_B
+    // tokens only the 32-token one, and with more than n pairs per expert on
+    // average one has more than n.  One of the launches made runs.
     const bool run32 = P <= WR_TILE_SPLIT_M * p.E;
     const bool run64 = !mid && (!many || P <= kMaxTok * p.E);
     const dim3 gg(p.I / kBM, slots), gd(p.h / kBM, BatchWs::kKSplit, slots);
