@@ -157,17 +157,24 @@ def test_workspace_bytes():
     # grouped MFMA layout: logits, x as two fp16 terms and its per-token
     # exponents, one act-maximum word per pair on its own 256-byte line, five
     # [P] pair arrays, expert offsets / active list / count, act [P][I] and
-    # four K-slice partials [4][P][h] (P = B * k), each region rounded up to
-    # 256 bytes.
-    def up(n):
-        return (n + 255) // 256 * 256
-    B, E, h, I, k = 4, 8, 4096, 14336, 2
-    P = B * k
-    per_token = ctrl + B * 256 + P * I * 4
-    grouped = (up(B * 256) + 2 * up(B * h * 2) + up(B * 4) + P * 256 + 5 * up(P * 4)
-               + up((E + 1) * 4) + up(E * 4) + up(4) + up(P * I * 4) + up(4 * P * h * 4))
-    assert grouped == 1051648 + 256 + 8 * 256
-    assert lib.wr_workspace_bytes(capi.WR_KIND_BATCHED, E, h, I, k, B) == max(per_token, grouped)
+    # four K-slice partials [4][P][h] (P = B * k; rows of h and I rounded up to
+    # 128 columns), each region rounded up to 256 bytes.
+    def up(n, a=256):
+        return (n + a - 1) // a * a
+
+    def batched(B, E, h, I, k):
+        P = B * k
+        per_token = ctrl + B * 256 + up(P * I * 4)
+        h, I = up(h, 128), up(I, 128)
+        grouped = (up(B * 256) + 2 * up(B * h * 2) + up(B * 4) + P * 256 + 5 * up(P * 4)
+                   + up((E + 1) * 4) + up(E * 4) + up(4) + up(P * I * 4) + up(4 * P * h * 4))
+        return max(per_token, grouped)
+    assert batched(4, 8, 4096, 14336, 2) == 1051648 + 256 + 8 * 256
+    # Ragged rows, and rows whose padded length is no 32-bit integer.
+    for B, E, h, I, k in ((4, 8, 4096, 14336, 2), (7, 5, 101, 37, 3), (2, 8, 2**31 - 1, 16, 2),
+                          (2, 8, 16, 2**31 - 1, 2)):
+        assert (lib.wr_workspace_bytes(capi.WR_KIND_BATCHED, E, h, I, k, B)
+                == batched(B, E, h, I, k)), (B, E, h, I, k)
     assert lib.wr_workspace_bytes(capi.WR_KIND_NAIVE, 8, 100, 10, 1, 1) == 256 + 3 * 256 + 2 * 512
     assert lib.wr_workspace_bytes(7, 8, 64, 64, 2, 1) == 0
     assert lib.wr_workspace_bytes(capi.WR_KIND_FUSED, 65, 64, 64, 2, 1) == 0

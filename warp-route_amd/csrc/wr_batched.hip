@@ -2389,8 +2389,8 @@ GeomB make_geom_b(const Problem& p, int64_t es, bool ragged) {
   g.off_up = p.off_up_b / es;
   g.off_down = p.off_down_b / es;
   g.off_scale = p.off_scale_b;
-  g.hp = ragged ? BatchWs::padded(p.h) : p.h;
-  g.Ip = ragged ? BatchWs::padded(p.I) : p.I;
+  g.hp = ragged ? (int)BatchWs::padded(p.h) : p.h;
+  g.Ip = ragged ? (int)BatchWs::padded(p.I) : p.I;
   return g;
 }
 
@@ -2627,6 +2627,7 @@ bool grouped_ok(const Problem& p) {
                     : p.wdt == WR_MXFP4    ? 32
                                            : 8;
   if (p.h < piece || p.I < piece) return false;
+  if (BatchWs::padded(std::max(p.h, p.I)) > INT32_MAX) return false;  // padded rows are ints
   const int64_t pairs = (int64_t)p.B * p.k;
   const int64_t tiny = (int64_t)(p.wdt == WR_F32 ? 64 : piece == 8 ? 16 : 4) << 20;
   return 2 * pairs >= 3 * p.E && pairs * p.stride_b > tiny;
@@ -2646,7 +2647,7 @@ hipError_t launch_grouped(const Problem& p, hipStream_t s) {
   if (p.wdt == WR_F32 && ragged) {  // x in fp32 rows of whole K steps
     XSplit xs = x_split(p);
     xs.f32 = w.x_f32();
-    xs.ld = BatchWs::padded(p.h);
+    xs.ld = (int)BatchWs::padded(p.h);
     hipError_t err = launch_router(p, w, xs, s);
     if (err != hipSuccess) return err;
     return p.adt == WR_F16 ? ragged_f32<f16>(p, w, s) : ragged_f32<float>(p, w, s);
@@ -2665,7 +2666,7 @@ hipError_t launch_grouped(const Problem& p, hipStream_t s) {
   xs.exp = w.x_exp;
   xs.amax = bf ? nullptr : w.amax;
   xs.bf16 = bf ? 1 : 0;
-  xs.ld = ragged ? BatchWs::padded(p.h) : p.h;
+  xs.ld = ragged ? (int)BatchWs::padded(p.h) : p.h;
   hipError_t err = launch_router(p, w, xs, s);
   if (err != hipSuccess) return err;
   if (ragged) {

@@ -141,7 +141,7 @@ struct BatchWs {
   float* ypart;  // [kKSplit][P][h]: down partial sums
   // Row lengths of ragged layers (h or I not whole K steps): x and act rows are
   // zero past h and I, the partial sums' tails unused.
-  static constexpr int padded(int n) { return (n + 127) / 128 * 128; }
+  static constexpr int64_t padded(int n) { return ((int64_t)n + 127) / 128 * 128; }
   // Ragged layers: third bf16 terms of x, in the partial sums' bytes (which the
   // down kernel writes after the gate/up kernel has read them); x in fp32, in
   // the two terms' bytes (adjacent: padded rows are whole 256-byte units).
@@ -166,11 +166,10 @@ struct BatchWs {
       return p;
     };
     const size_t P = (size_t)B * k;
-    h = padded(h);
-    I = padded(I);
+    const size_t hp = padded(h), Ip = padded(I);
     w.logits = reinterpret_cast<float*>(take((size_t)B * WR_MAX_EXPERTS * 4));
-    w.x_hi = reinterpret_cast<_Float16*>(take((size_t)B * h * 2));
-    w.x_lo = reinterpret_cast<_Float16*>(take((size_t)B * h * 2));
+    w.x_hi = reinterpret_cast<_Float16*>(take((size_t)B * hp * 2));
+    w.x_lo = reinterpret_cast<_Float16*>(take((size_t)B * hp * 2));
     w.x_exp = reinterpret_cast<int32_t*>(take((size_t)B * 4));
     w.amax = reinterpret_cast<unsigned*>(take(P * kAmaxStride * 4));
     w.route.sel_id = reinterpret_cast<int32_t*>(take(P * 4));
@@ -181,8 +180,8 @@ struct BatchWs {
     w.route.off = reinterpret_cast<int32_t*>(take((size_t)(E + 1) * 4));
     w.route.active = reinterpret_cast<int32_t*>(take((size_t)E * 4));
     w.route.n_active = reinterpret_cast<int32_t*>(take(8));
-    w.act = reinterpret_cast<float*>(take(P * I * 4));
-    w.ypart = reinterpret_cast<float*>(take((size_t)kKSplit * P * h * 4));
+    w.act = reinterpret_cast<float*>(take(P * Ip * 4));
+    w.ypart = reinterpret_cast<float*>(take((size_t)kKSplit * P * hp * 4));
     if (total != nullptr) *total = off;
     return w;
   }
