@@ -826,10 +826,13 @@ struct GuScale {
   unsigned* s_amax;
 };
 
-// Ragged layers sum each K step apart and add it to a running sum, whose
-// length the step count then sets, instead of one chain through all MFMAs:
-// their error stays that of the per-token kernels' 64 lane sums (one chain,
-// h = 1500: 2.0 times it).
+// Ragged layers sum each K step apart, the lower terms of x and act first (where
+// the sum is small, and so is its rounding), and add it to a running sum: their
+// error is then at most that of the per-token kernels, whose 64 lane sums are
+// short.  Error against 64 bits over theirs, k = 1, fp32 x: bf16 weights 264 x
+// 520 0.91 (1.56 with the terms in turn), 1000 x 1400 0.85 (1.36); fp16 1.00
+// (1.39) and 0.9 (1.24); MXFP4 1504 x 2080 0.6 (1.14); one chain through all
+// steps, fp16 h = 1500, 2.0.
 template <int NT>
 __device__ __forceinline__ void ksum_open(f32x4 (&t)[NT], f32x4 (&a)[NT]) {
 #pragma unroll
@@ -928,30 +931,40 @@ __device__ __forceinline__ void gu_pass(TokTile<TOK, KC, L2>& xs,
         ksum_open(tg, ag);
         ksum_open(tu, au);
       }
+      // RAG: the lower terms first (ksum_open).
 #pragma unroll
-      for (int j = 0; j < KC / 32; ++j) {
-        const int c = 4 * j + (lane >> 4);
-        const int jw = hs * (KC / 32) + j;  // MFMA j of the token step within the weight step
-        const H8 ga = a_frag(wt, lane & 15, jw, lane >> 4);
-        const H8 ua = a_frag(wt, 16 + (lane & 15), jw, lane >> 4);
+      for (int ph = RAG && LO ? 0 : 1; ph < 2; ++ph) {
 #pragma unroll
-        for (int n = 0; n < NT; ++n) {
-          const int tn = n * 16 + (lane & 15);
-          constexpr bool BF = bf16_ops<WT>();
-          const H8 bh = xs.hi[tn][tslot<TOK, KC>(tn, c)];
-          ag[n] = mfma<BF>(ga, bh, ag[n]);
-          au[n] = mfma<BF>(ua, bh, au[n]);
-          if (LO) {
-            const H8 bl = xs.lo[tn][tslot<TOK, KC>(tn, c)];
-            ag[n] = mfma<BF>(ga, bl, ag[n]);
-            au[n] = mfma<BF>(ua, bl, au[n]);
-          }
-          if constexpr (L2) {
-            const H8 b2 = xs.l2[tn][tslot<TOK, KC>(tn, c)];
-            ag[n] = mfma<BF>(ga, b2, ag[n]);
-            au[n] = mfma<BF>(ua, b2, au[n]);
+        for (int j = 0; j < KC / 32; ++j) {
+          const int c = 4 * j + (lane >> 4);
+          const int jw = hs * (KC / 32) + j;  // MFMA j of the token step within the weight step
+          const H8 ga = a_frag(wt, lane & 15, jw, lane >> 4);
+          const H8 ua = a_frag(wt, 16 + (lane & 15), jw, lane >> 4);
+#pragma unroll
+          for (int n = 0; n < NT; ++n) {
+            const int tn = n * 16 + (lane & 15);
+            constexpr bool BF = bf16_ops<WT>();
+            if constexpr (L2) {
+              if (ph == 0) {
+                const H8 b2 = xs.l2[tn][tslot<TOK, KC>(tn, c)];
+                ag[n] = mfma<BF>(ga, b2, ag[n]);
+                au[n] = mfma<BF>(ua, b2, au[n]);
+              }
+            }
+            if (ph == 1) {
+              const H8 bh = xs.hi[tn][tslot<TOK, KC>(tn, c)];
+              ag[n] = mfma<BF>(ga, bh, ag[n]);
+              au[n] = mfma<BF>(ua, bh, au[n]);
+            }
+            if (LO && (ph == 0 || !RAG)) {
+              const H8 bl = xs.lo[tn][tslot<TOK, KC>(tn, c)];
+              ag[n] = mfma<BF>(ga, bl, ag[n]);
+              au[n] = mfma<BF>(ua, bl, au[n]);
+            }
           }
         }
+        // The second round reads the weights again: kept, they spill.
+        if constexpr (RAG) asm volatile("" ::: "memory");
       }
       if constexpr (RAG) {
         ksum_close(tg, ag);
@@ -1150,10 +1163,18 @@ __global__ __launch_bounds__(kBlk, (gu_min_blocks<WT, LO, TOK, KC, WK>())) void 
                                                      act, g, logits, ids_out, w_out);
 }
 
+// Blocks per CU that LDS allows and a VGPR bound then asks for.
+template <typename WT, bool L2, int TOK>
+constexpr int rag_gu_min_blocks() {
+  if (TOK == 16) return 3;
+  if (TOK == 32) return wbits<WT>() == 16 && L2 ? 2 : 3;
+  return wbits<WT>() == 4 ? 2 : 1;
+}
+
 // Ragged layers: any h and I of at least one 16-byte piece of weights, any
 // alignment of the pointers.
 template <typename WT, bool LO, bool L2, int TOK, bool ROUTE>
-__global__ __launch_bounds__(kBlk) void k_rag_gu(
+__global__ __launch_bounds__(kBlk, (rag_gu_min_blocks<WT, L2, TOK>())) void k_rag_gu(
     const WT* __restrict__ wbuf, const f16* __restrict__ x_hi, const f16* __restrict__ x_lo,
     const f16* __restrict__ x_l2, const int32_t* __restrict__ x_exp, unsigned* __restrict__ amax,
     BatchRoute r, float* __restrict__ act, GeomB g, const float* __restrict__ logits,
@@ -1269,17 +1290,24 @@ __device__ __forceinline__ void dn_pass(TokTile<TOK, KC, RAG>& xs,
         f32x4 ta[RAG ? NT : 1];
         if constexpr (RAG) ksum_open(ta, acc);
 #pragma unroll
-        for (int j = 0; j < KC / 32; ++j) {
-          const int c = 4 * j + (lane >> 4);
-          const H8 da = a_frag(wt, lane & 15, hs * (KC / 32) + j, lane >> 4);
+        for (int ph = RAG ? 0 : 1; ph < 2; ++ph) {  // as in gu_pass
 #pragma unroll
-          for (int n = 0; n < NT; ++n) {
-            const int tn = n * 16 + (lane & 15);
-            acc[n] = mfma<bf16_ops<WT>()>(da, xs.hi[tn][tslot<TOK, KC>(tn, c)], acc[n]);
-            acc[n] = mfma<bf16_ops<WT>()>(da, xs.lo[tn][tslot<TOK, KC>(tn, c)], acc[n]);
-            if constexpr (RAG)
-              acc[n] = mfma<bf16_ops<WT>()>(da, xs.l2[tn][tslot<TOK, KC>(tn, c)], acc[n]);
+          for (int j = 0; j < KC / 32; ++j) {
+            const int c = 4 * j + (lane >> 4);
+            const H8 da = a_frag(wt, lane & 15, hs * (KC / 32) + j, lane >> 4);
+#pragma unroll
+            for (int n = 0; n < NT; ++n) {
+              const int tn = n * 16 + (lane & 15);
+              constexpr bool BF = bf16_ops<WT>();
+              if constexpr (RAG) {
+                if (ph == 0) acc[n] = mfma<BF>(da, xs.l2[tn][tslot<TOK, KC>(tn, c)], acc[n]);
+              }
+              if (ph == 1) acc[n] = mfma<BF>(da, xs.hi[tn][tslot<TOK, KC>(tn, c)], acc[n]);
+              if (ph == 0 || !RAG)
+                acc[n] = mfma<BF>(da, xs.lo[tn][tslot<TOK, KC>(tn, c)], acc[n]);
+            }
           }
+          if constexpr (RAG) asm volatile("" ::: "memory");
         }
         if constexpr (RAG) ksum_close(ta, acc);
       }
@@ -2035,6 +2063,26 @@ __device__ __forceinline__ void f32_w_store(TileF<ROWS>& t, const WRegsF<ROWS>& 
     t.v[4 * i + lane / 16][fslot(4 * i + lane / 16, lane % 16)] = r.v[i];
 }
 
+// The 16 products of four MFMAs in two chains of 8; a step adds its four such
+// sums in pairs.  Ragged layers' error against 64 bits over the per-token
+// kernels' (k = 1): 264 x 520 1.02, 1000 x 1400 1.01, 2050 x 1500 1.03; with
+// chains of 16 1.18, 1.09 and 1.08, one chain through the step's 64 columns 1.8,
+// 1.6 and 1.4.  Calls of more than 32 tokens take 8% longer than with one chain,
+// smaller ones 0 to 3%.
+__device__ __forceinline__ f32x4 sum16_f32(const f32x4& a, const f32x4& b) {
+  const f32x4 z = {0.0f, 0.0f, 0.0f, 0.0f};
+  const f32x4 p = mfma_f32(a[1], b[1], mfma_f32(a[0], b[0], z));
+  const f32x4 q = mfma_f32(a[3], b[3], mfma_f32(a[2], b[2], z));
+  return p + q;
+}
+
+// Keeps one 16-column piece's LDS reads and MFMAs together: read ahead, or
+// with the sums of several pieces open, they spill.
+__device__ __forceinline__ void step_fence() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // Gate/up pass over up to TOK tokens (NT tiles of 16) of one expert, rows
 // row0 .. + 16 of its gate and up matrices (tile rows 0-15 and 16-31).
 template <typename XT, int NT, int TOK, bool RAG>
@@ -2071,11 +2119,7 @@ __device__ __forceinline__ void gu_pass_f32(TileF<TOK>& xs, TileF<32>& wt,
         f32_w_load<32>(wr, wbase, (s + 1) * kBKF);
       f32_tile_load(tv, x, off, (s + 1) * kBKF);
     }
-    f32x4 tg[RAG ? NT : 1], tu[RAG ? NT : 1];
-    if constexpr (RAG) {
-        ksum_open(tg, ag);
-        ksum_open(tu, au);
-      }
+    f32x4 tg[2][RAG ? NT : 1], tu[2][RAG ? NT : 1];  // RAG: the step's half sums
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       const f32x4 ga = wt.v[rl][fslot(rl, 4 * j + q)];
@@ -2083,17 +2127,27 @@ __device__ __forceinline__ void gu_pass_f32(TileF<TOK>& xs, TileF<32>& wt,
 #pragma unroll
       for (int n = 0; n < NT; ++n) {
         const f32x4 b = xs.v[n * 16 + rl][fslot(rl, 4 * j + q)];
+        if constexpr (RAG) {
+          const f32x4 pg = sum16_f32(ga, b), pu = sum16_f32(ua, b);
+          tg[j / 2][n] = j % 2 ? tg[j / 2][n] + pg : pg;
+          tu[j / 2][n] = j % 2 ? tu[j / 2][n] + pu : pu;
+          if (n % 2 == 1 || n == NT - 1) step_fence();
+        } else {
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-          ag[n] = mfma_f32(ga[m], b[m], ag[n]);
-          au[n] = mfma_f32(ua[m], b[m], au[n]);
+          for (int m = 0; m < 4; ++m) {
+            ag[n] = mfma_f32(ga[m], b[m], ag[n]);
+            au[n] = mfma_f32(ua[m], b[m], au[n]);
+          }
         }
       }
     }
     if constexpr (RAG) {
-        ksum_close(tg, ag);
-        ksum_close(tu, au);
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        ag[n] += tg[0][n] + tg[1][n];
+        au[n] += tu[0][n] + tu[1][n];
       }
+    }
   }
   // D layout: lane holds token n*16 + (lane % 16), rows 4 (lane / 16) .. +4.
   const int rq = row0 + q * 4;
@@ -2196,7 +2250,7 @@ __global__ __launch_bounds__(kBlk) void k_gu_f32(const float* __restrict__ wbuf,
 
 // Ragged layers, as k_rag_gu; x is the workspace's padded fp32 copy.
 template <int TOK, bool ROUTE>
-__global__ __launch_bounds__(kBlk) void k_rag_gu_f32(const float* __restrict__ wbuf,
+__global__ __launch_bounds__(kBlk, TOK == 16 ? 3 : 2) void k_rag_gu_f32(const float* __restrict__ wbuf,
                                                      const float* __restrict__ x, BatchRoute r,
                                                      float* __restrict__ act, GeomB g,
                                                      const float* __restrict__ logits,
@@ -2241,19 +2295,27 @@ __device__ __forceinline__ void dn_pass_f32(TileF<TOK>& xs, TileF<16>& wt,
           f32_w_load<16>(wr, wbase, (s + 1) * kBKF);
         f32_tile_load(tv, act, off, (s + 1) * kBKF);
       }
-      f32x4 ta[RAG ? NT : 1];
-      if constexpr (RAG) ksum_open(ta, acc);
+      f32x4 ta[2][RAG ? NT : 1];  // RAG: the step's half sums
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const f32x4 da = wt.v[rl][fslot(rl, 4 * j + q)];
 #pragma unroll
         for (int n = 0; n < NT; ++n) {
           const f32x4 b = xs.v[n * 16 + rl][fslot(rl, 4 * j + q)];
+          if constexpr (RAG) {
+            const f32x4 p = sum16_f32(da, b);
+            ta[j / 2][n] = j % 2 ? ta[j / 2][n] + p : p;
+            if (n % 2 == 1 || n == NT - 1) step_fence();
+          } else {
 #pragma unroll
-          for (int m = 0; m < 4; ++m) acc[n] = mfma_f32(da[m], b[m], acc[n]);
+            for (int m = 0; m < 4; ++m) acc[n] = mfma_f32(da[m], b[m], acc[n]);
+          }
         }
       }
-      if constexpr (RAG) ksum_close(ta, acc);
+      if constexpr (RAG) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n] += ta[0][n] + ta[1][n];
+      }
     }
   }
   const int rq = row0 + q * 4;
