@@ -319,8 +319,8 @@ __device__ __forceinline__ void write_x_split8(const XSplit& xs, const XT* __res
 }
 
 // Router and selection of T tokens per block: grid ceil(B / T), block 1024.
-// Wave 4 g + q computes quarter q of the logits of experts 4 g .. 4 g + 3, then
-// 16 more on, for all T tokens at once, so that a loaded piece of x serves four
+// Wave 4 g + q computes quarter q of the logits of NE experts from NE g on, then
+// 4 NE more on, for all T tokens at once, so that a loaded piece of x serves NE
 // experts and a piece of a router row T tokens.  Each dot product is summed
 // exactly as router_partial's (lane chunks of VEC columns, chunk j into sum j
 // mod 4), so the logits have the same bits.  Wave t then selects token t's
@@ -331,7 +331,7 @@ __device__ __forceinline__ void write_x_split8(const XSplit& xs, const XT* __res
 // 16.3 -> 11.7, B = 512 29.0 -> 15.6; in batched calls of more than 16 tokens, the
 // selection of all tokens was one block's work (B = 256: router 21 + k_route 75
 // -> 14 + k_group 5.4).
-template <typename XT, int VEC, int T>
+template <typename XT, int VEC, int T, int NE>
 __global__ __launch_bounds__(1024) void k_router_topk(const float* __restrict__ gate_w,
                                                       const XT* __restrict__ x, int B, int E,
                                                       int h, int k, int renorm,
@@ -339,7 +339,7 @@ __global__ __launch_bounds__(1024) void k_router_topk(const float* __restrict__ 
                                                       float* __restrict__ w_out,
                                                       int32_t* __restrict__ sel_id,
                                                       float* __restrict__ sel_w, XSplit xs) {
-  constexpr int CH = kWave * VEC, NE = 4;
+  constexpr int CH = kWave * VEC;
   __shared__ float part[T][WR_MAX_EXPERTS][4];
   __shared__ float pmax[T][4];
   const int lane = threadIdx.x & (kWave - 1);
@@ -354,6 +354,14 @@ __global__ __launch_bounds__(1024) void k_router_topk(const float* __restrict__ 
   for (int t = 0; t < T; ++t) xr[t] = x + (int64_t)min(b0 + t, B - 1) * h;
 #pragma unroll 1
   for (int e0 = NE * grp; e0 < E; e0 += 4 * NE) {
+    if constexpr (NE == 1 && T == 1) {  // one row, one token: nothing to share
+      float mx;
+      const float p = router_partial<XT, VEC>(gate_w + (int64_t)e0 * h, xr[0], h, q,
+                                              scaled && e0 == 0, mx);
+      if (lane == 0) part[0][e0][q] = p;
+      if (lane == 0 && e0 == 0) pmax[0][q] = mx;
+      continue;
+    }
     const float* wr[NE];
 #pragma unroll
     for (int i = 0; i < NE; ++i) wr[i] = gate_w + (int64_t)min(e0 + i, E - 1) * h;
@@ -366,7 +374,10 @@ __global__ __launch_bounds__(1024) void k_router_topk(const float* __restrict__ 
       for (int i = 0; i < NE; ++i) acc[i][t][0] = acc[i][t][1] = acc[i][t][2] = acc[i][t][3] = 0.0f;
     }
     const bool want_max = scaled && e0 == 0;
-    // Chunk j adds to sum j mod 4: the sums rotate.  U chunks' loads at once.
+    // Chunk j adds to sum j mod 4: the sums rotate.  U chunks per round; the
+    // break keeps the loads of all but the first behind its test, so each is a
+    // round trip, but without it a short row pays for the sums of chunks that it
+    // does not have (E 60, h 1000, B = 4: 7.6 us, without it 12.2).
     constexpr int U = T == 1 ? 4 : 2;
     const int chunks = end > beg ? (end - beg + CH - 1) / CH : 0;
 #pragma unroll 1
@@ -381,7 +392,7 @@ __global__ __launch_bounds__(1024) void k_router_topk(const float* __restrict__ 
 #pragma unroll
         for (int t = 0; t < T; ++t) load_x<XT, VEC>(xr[t] + cc, xv[u][t]);
       }
-      __builtin_amdgcn_sched_barrier(0);  // all of them before the sums
+      __builtin_amdgcn_sched_barrier(0);  // the first chunk's ahead of the sums
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         if (j + u >= chunks) break;  // wave-uniform
@@ -2284,24 +2295,34 @@ hipError_t run_ffn(const Problem& p, hipStream_t s) {
 // Two tokens per block when one each would be more blocks than CUs.  gate_topk,
 // us, 1 / 2 / 4 tokens per block: E 64, h 2048, B = 256 11.7 / 14.5 / 23.5, B =
 // 512 18.4 / 15.6 / 24.1; E 16, h 6144 8.4 / 9.3 / 12.2 and 13.3 / 10.6 / 13.9.
-template <typename XT, int VEC>
+template <typename XT, int VEC, int NE>
 hipError_t router_topk_v(const Problem& p, int32_t* sel_id, float* sel_w, const XSplit& xs,
                          hipStream_t s) {
   const XT* x = static_cast<const XT*>(p.x);
-  if (p.B > cu_count())
-    hipLaunchKernelGGL((k_router_topk<XT, VEC, 2>), dim3((p.B + 1) / 2), dim3(1024), 0, s,
-                       p.gate_w, x, p.B, p.E, p.h, p.k, p.renorm, p.topk_ids, p.topk_w, sel_id,
-                       sel_w, xs);
-  else
-    hipLaunchKernelGGL((k_router_topk<XT, VEC, 1>), dim3(p.B), dim3(1024), 0, s, p.gate_w, x, p.B,
-                       p.E, p.h, p.k, p.renorm, p.topk_ids, p.topk_w, sel_id, sel_w, xs);
+  const bool two = p.B > cu_count();
+  auto k = two ? k_router_topk<XT, VEC, 2, NE> : k_router_topk<XT, VEC, 1, NE>;
+  hipLaunchKernelGGL(k, dim3(two ? (p.B + 1) / 2 : p.B), dim3(1024), 0, s, p.gate_w, x, p.B, p.E,
+                     p.h, p.k, p.renorm, p.topk_ids, p.topk_w, sel_id, sel_w, xs);
   return hipGetLastError();
 }
+// Experts per wave and round: as few as the block's four groups of waves need,
+// since rows past the last are loaded and summed for nothing.  gate_topk, us,
+// 1 / 2 / 4 experts (mean over h from 37 to 7168 and B up to 256, in units of a
+// block of four single-expert groups): E = 1 0.99 / 1.09 / 1.25, 4 1.00 / 0.98 /
+// 1.09, 5 0.97 / 0.95 / 1.04, 8 0.94 / 0.87 / 0.90, 12 0.93 / 0.82 / 0.82, 64
+// 0.87 / 0.72 / 0.65.  E = 1, h 7168, B = 1024 7.0 us of such blocks, 4 experts
+// 13.7.
 template <typename XT>
 hipError_t router_topk_t(const Problem& p, int32_t* sel_id, float* sel_w, const XSplit& xs,
                          hipStream_t s) {
-  return router_vec4(p) ? router_topk_v<XT, 4>(p, sel_id, sel_w, xs, s)
-                        : router_topk_v<XT, 1>(p, sel_id, sel_w, xs, s);
+  if (p.E <= 4)
+    return router_vec4(p) ? router_topk_v<XT, 4, 1>(p, sel_id, sel_w, xs, s)
+                          : router_topk_v<XT, 1, 1>(p, sel_id, sel_w, xs, s);
+  if (p.E <= 8)
+    return router_vec4(p) ? router_topk_v<XT, 4, 2>(p, sel_id, sel_w, xs, s)
+                          : router_topk_v<XT, 1, 2>(p, sel_id, sel_w, xs, s);
+  return router_vec4(p) ? router_topk_v<XT, 4, 4>(p, sel_id, sel_w, xs, s)
+                        : router_topk_v<XT, 1, 4>(p, sel_id, sel_w, xs, s);
 }
 
 }  // namespace
