@@ -220,7 +220,7 @@ def test_exact_tie_known_answers(cuda, op):
 @pytest.mark.parametrize("B", [3, 20], ids=["B3-in-kernel-route", "B20-route-kernel"])
 def test_batched_exact_tie_known_answers(cuda, B, E):
     """The same ties through the grouped batched path (h and I multiples of
-    128).  B = 3 routes inside the gate/up kernel, B = 20 in k_route; E = 8
+    128).  B = 3 routes inside the gate/up kernel, B = 20 in k_group; E = 8
     selects four tokens per wave (one per 16-lane row), E = 24 one token per
     wave.  Every token must get the answers the single-token op gives."""
     h, I, k = 128, 128, 3

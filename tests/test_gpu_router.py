@@ -40,3 +40,21 @@ def test_gate_topk_variants(cuda, E, h, B):
             _, want, w = O.softmax_topk((f64(gw) @ f64(x[b])).astype("float32"), k, rn)
             assert ids[b].cpu().tolist() == want.tolist(), b
             assert abs(ws[b].cpu().double().numpy() - w).max() < 1e-5, b
+
+
+# Either side of the line between the selection in the grouping launch and in the
+# router launch: E <= 16 at 64 tokens, more experts at 24 + E h / 6144 (24, 32 and
+# 64 here) tokens.
+@pytest.mark.parametrize("E,h,B", [(16, 256, 64), (16, 256, 65), (17, 256, 24), (17, 256, 25),
+                                   (64, 768, 32), (64, 768, 33), (64, 4096, 64), (64, 4096, 65)])
+def test_batched_selection_is_gate_topk(cuda, E, h, B):
+    k, I = 6, 128
+    for xd in (torch.float32, torch.float16):
+        x, gw, buf = make_layer(E, h, I, torch.float16, router_std=h ** -0.5, seed=B, batch=B,
+                                device=cuda, gen_device=cuda, x_dtype=xd)
+        want_ids, want_ws = F.gate_topk(x, gw, E, h, k, True)
+        ids, ws = torch.empty_like(want_ids), torch.empty_like(want_ws)
+        print(f"[gpu] batched selection E={E} h={h} B={B} {xd}", flush=True)
+        F.batched_fused_moe(x, gw, buf, E, h, I, k, True, ids, ws)
+        torch.cuda.synchronize()
+        assert torch.equal(ids, want_ids) and torch.equal(ws, want_ws)

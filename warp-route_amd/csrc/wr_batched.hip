@@ -9,11 +9,11 @@
 //      x 2^e_b, with a power of two e_b per token that puts max|x 2^e_b| in
 //      [2^14, 2^15): hi stays finite and |x 2^e_b - (hi + lo)| <= 2^-22
 //      |x 2^e_b| + 2^-25 (split_exp)): k_router_topk (wr_kernels.hip), which
-//      selects every token's top-K as well; for B <= WR_SMALL_TILE_MAX_B
-//      k_router_logits, logits[B][64].
+//      selects every token's top-K as well, or k_router_logits, logits[B][64],
+//      for few tokens (select_in_group).
 //   2. k_group: one block groups the (token, expert) pairs by expert, tokens
-//      ascending, with ballot prefix sums (deterministic, no global atomics).
-//      For B <= WR_SMALL_TILE_MAX_B there is no such launch: every gate/up block
+//      ascending, with ballot prefix sums (deterministic, no global atomics);
+//      after k_router_logits it selects first.  For B <= WR_SMALL_TILE_MAX_B there is no such launch: every gate/up block
 //      of step 3 selects (the same wave_select_topk as every other path, so ids
 //      and weights are bit-identical to the single-token op) and groups in LDS
 //      (route_small), and block (0, 0) publishes it.
@@ -55,6 +55,7 @@
 // scaling leaves no range condition on x or act beyond fp32's own.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "wr_device.h"
@@ -212,16 +213,17 @@ __device__ __forceinline__ void group_pairs(int P, int E, int k, const int* sel_
   }
 }
 
-// Groups the P selections that k_router_topk left in r.sel_id / r.sel_w by
-// expert, as group_pairs does, and names the call's tile class (tile_slot).
+// Groups the P selections in r.sel_id / r.sel_w (from k_router_topk, or this
+// block's own, below) by expert, as group_pairs does, and names the call's tile
+// class (tile_slot).
 // One block of 16 waves, each with an equal run of 64-pair chunks in order.  A
 // lane finds the lanes of its chunk with its expert from one ballot per id bit,
 // so a chunk costs the same for any number of experts (one ballot per expert
 // and chunk before: B = 256, E = 64, k = 6 about 5 us).
 //
-// logits set (E <= 16): the block first selects from them, four tokens per wave
-// at once, one per 16-lane row (row_select_topk), also to ids_out / w_out when
-// set.
+// logits set: the block first selects from them, also to ids_out / w_out when
+// set: E <= 16 four tokens per wave at once, one per 16-lane row
+// (row_select_topk), else a wave per token.
 __global__ __launch_bounds__(1024) void k_group(int P, int E, int k, BatchRoute r, int max_cls,
                                                 const float* __restrict__ logits, int renorm,
                                                 int32_t* __restrict__ ids_out,
@@ -245,19 +247,29 @@ __global__ __launch_bounds__(1024) void k_group(int P, int E, int k, BatchRoute 
   };
   static_assert(WR_MAX_EXPERTS <= 64, "six id bits");
   if (logits != nullptr) {
-    const int row = lane >> 4, li = lane & 15, B = P / k;
-    for (int t0 = 4 * wave; t0 < B; t0 += 4 * NW) {  // wave-uniform bound
-      const int t = t0 + row;
-      const float l = t < B ? logits[(int64_t)t * WR_MAX_EXPERTS + li] : 0.0f;
-      int sid;
-      float sw;
-      row_select_topk(l, E, k, renorm, sid, sw);
-      if (t < B && li < k) {
-        const int q = t * k + li;
-        r.sel_id[q] = sid;
-        r.sel_w[q] = sw;
-        if (ids_out != nullptr) ids_out[q] = sid;
-        if (w_out != nullptr) w_out[q] = sw;
+    const int B = P / k;
+    auto put = [&](int t, int kk, int sid, float sw) {
+      const int q = t * k + kk;
+      r.sel_id[q] = sid;
+      r.sel_w[q] = sw;
+      if (ids_out != nullptr) ids_out[q] = sid;
+      if (w_out != nullptr) w_out[q] = sw;
+    };
+    if (E <= 16) {
+      const int row = lane >> 4, li = lane & 15;
+      for (int t0 = 4 * wave; t0 < B; t0 += 4 * NW) {  // wave-uniform bound
+        const int t = t0 + row;
+        const float l = t < B ? logits[(int64_t)t * WR_MAX_EXPERTS + li] : 0.0f;
+        int sid;
+        float sw;
+        row_select_topk(l, E, k, renorm, sid, sw);
+        if (t < B && li < k) put(t, li, sid, sw);
+      }
+    } else {
+      for (int t = wave; t < B; t += NW) {  // wave-uniform
+        TopK tk;
+        wave_select_topk_reg(logits[(int64_t)t * WR_MAX_EXPERTS + lane], E, k, renorm, tk);
+        if (lane < k) put(t, lane, tk.lid, tk.lw);
       }
     }
     __syncthreads();
@@ -316,11 +328,19 @@ __global__ __launch_bounds__(1024) void k_group(int P, int E, int k, BatchRoute 
   }
 }
 
-// Few tokens and experts: k_router_logits, a block per logit, and the selection
-// in k_group; else k_router_topk.  Measured, us, router + grouping launches: E 16,
-// h 6144, B = 32 13.3 against 17.0; E 8, h 4096, B = 64 10.7 against 12.0; B = 512
-// 30 against 15; E 64, h 2048, B = 256 96 against 20.
-bool select_in_group(const Problem& p) { return p.E <= 16 && p.B <= 64; }
+// Few tokens: k_router_logits, a block per logit, and the selection in k_group;
+// else k_router_topk, a block per token, which a few tokens spread over too few
+// CUs (the more so the longer a token's E h sums) and which overtakes as one
+// block's selections add up.  Measured, us, router + grouping launches, selection
+// in k_group against k_router_topk: E 16, h 6144, B = 32 13.3 against 17.0; E 8, h
+// 4096, B = 64 10.7 against 12.0; B = 512 30 against 15; E 64, h 2048, B = 256 96
+// against 20.  E > 16, difference of a call: E 17, h 1024, B = 24 -0.2 and B = 40
+// +2.5; E 32, h 4096, B = 40 -1.2 and 48 +1.2; E 64, h 1024, B = 32 -1.7 and 64
+// +2.9; h 4096, B = 17 -9.3, 48 -3.5 and 80 +0.7; h 7168, B = 17 -17.3, 64 -6.8
+// and 96 +3.6.
+bool select_in_group(const Problem& p) {
+  return p.B <= (p.E <= 16 ? 64 : std::min<int64_t>(64, 24 + (int64_t)p.E * p.h / 6144));
+}
 
 hipError_t launch_group(const Problem& p, const BatchWs& w, int max_cls, hipStream_t s) {
   hipLaunchKernelGGL(k_group, dim3(1), dim3(1024), 0, s, p.B * p.k, p.E, p.k, w.route, max_cls,
