@@ -58,3 +58,27 @@ def test_many_tokens_every_row(cuda, wd, E, B, x_dtype):
         if ref["robust"]:
             assert_parity(out[b], ids[b], ws[b], ref, rel_tol=2e-3 if x_dtype == F16 else 1e-4,
                           label=f"{wd} E={E} B={B} row {b}")
+
+
+def test_many_tokens_long_act_rows(cuda):
+    """A pass whose act rows end more than 4 GiB past its first: the many-token
+    kernels' 32-bit offsets do not reach, the 64-token kernels take the call."""
+    E, h, I, k, B = 1, 128, 52864 * 128, 1, 160
+    assert 160 * I * 4 > 159 * I * 4 > 1 << 32
+    gen = torch.Generator(device=cuda).manual_seed(5)
+    lay = F.weight_layout(E, h, I, MX4)
+    buf = F.zeros_weights(lay["expert_stride"], MX4, cuda)
+    raw = buf.view(torch.uint8)
+    for part in raw.split(1 << 26):
+        part.copy_(torch.randint(0, 256, (part.numel(),), generator=gen, device=cuda,
+                                 dtype=torch.uint8))
+    raw[lay["scale_offset"]:].fill_(122)  # 2^-5
+    x = torch.randn(B, h, generator=gen, device=cuda)
+    gw = torch.randn(E, h, generator=gen, device=cuda) * h ** -0.5
+    print("[gpu] many tokens, act rows of 26 MiB", flush=True)
+    out = F.batched_fused_moe(x, gw, buf, E, h, I, k)
+    for b in (0, 63, 64, 127, 158, 159):
+        single = F.fused_moe(x[b], gw, buf, E, h, I, k)
+        torch.cuda.synchronize()
+        # fp32 sums of 6.8 million columns, in other orders.
+        assert_same_up_to_order(out[b], single, f"row {b}", 1e-3)

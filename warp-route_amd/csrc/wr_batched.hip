@@ -1559,7 +1559,7 @@ __device__ __forceinline__ int many_slot(int n, int c) {
 // split ahead (k_act_split: 8 hi terms, then 8 lo terms).  Rows past the pass's
 // tokens repeat a valid one; their sums are not used.
 // at(n, c, t): bytes from base to piece c of term t of row n, 32 bits (the host
-// checks that x's two terms lie within 4 GiB); kCol: bytes per column.
+// checks that x's two terms, and a pass's act rows, lie within 4 GiB); kCol: bytes per column.
 struct RowsX {
   const char* base;  // the hi terms
   uint32_t lo;       // bytes from a hi term to its lo term
@@ -2548,8 +2548,11 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
   const WT* wb = static_cast<const WT*>(p.wbuf);
 
   hipError_t err = hipSuccess;
-  // The many-token kernels address x's two terms with 32-bit offsets.
-  const bool many = p.B > kMaxTok && (int64_t)p.B * p.h * 4 < (int64_t{1} << 32);
+  // The many-token kernels address x's two terms and a pass's act rows with 32-bit
+  // offsets.
+  const int64_t lim = int64_t{1} << 32;
+  const bool many =
+      p.B > kMaxTok && (int64_t)p.B * p.h * 4 < lim && (int64_t)kPassTok * p.I * 4 < lim;
   const bool mid = p.B <= WR_MID_TILE_MAX_B;
   // Small batches route inside the gate/up kernel (one launch fewer).  The
   // largest class is that of the kernels launched below, whatever the counts: a
