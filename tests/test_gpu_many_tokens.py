@@ -1,10 +1,11 @@
-"""GPU parity of batched calls with more than 64 tokens on an expert: the
+"""GPU parity of batched calls with more than 64 tokens on an expert.  With more
+than 32 (fp16, bf16), 48 (fp8) or 80 (MXFP4) pairs per expert on average the
 many-token kernels (k_many_gu, k_many_dn) take them in equal passes of up to 160
-tokens (fp8 and MXFP4 weights 128), five (four) 16-token tiles per wave.
+tokens, five 16-token tiles per wave; else the 64-token kernels do, 64 per pass.
 
 Batch sizes put an expert's count at, just below and just above each number of
 tiles, the 64-token kernels' limit and one pass, so that every instantiation
-and the second pass run.  Rows are checked against the oracle (a sample) and
+and the second pass run, and the average at and just above each of its bounds.  Rows are checked against the oracle (a sample) and
 against the single-token op (all: identical ids, outputs equal up to summation
 order, 1e-5 of max|out|; bf16 and MXFP4 weights, whose batched operands are two
 bf16 terms within 2^-18, at 5e-5, as for the smaller tiles); two calls agree
@@ -27,9 +28,10 @@ WTYPES = {"f16": F16, "bf16": BF16, "fp8": FP8, "mxfp4": MX4}
 
 @pytest.mark.parametrize("x_dtype", [F32, F16], ids=["xf32", "xf16"])
 # Clustered on one pair of experts: close to B tokens on each.  E = 2 with
-# k = 2: exactly B on both.
-@pytest.mark.parametrize("E,B", [(2, 65), (2, 96), (2, 97), (2, 128), (2, 129), (2, 160), (2, 161),
-                                 (2, 321), (8, 200)])
+# k = 2: exactly B on both.  E = 8, k = 2: the average is B / 4.
+@pytest.mark.parametrize("E,B", [(2, 65), (2, 81), (2, 96), (2, 97), (2, 128), (2, 129), (2, 160),
+                                 (2, 161), (2, 321), (8, 128), (8, 129), (8, 192), (8, 193),
+                                 (8, 200), (8, 320), (8, 321)])
 @pytest.mark.parametrize("wd", WTYPES)
 def test_many_tokens_every_row(cuda, wd, E, B, x_dtype):
     h, I, k, rn = (384, 640, 2, True) if B % 2 else (512, 256, 2, False)

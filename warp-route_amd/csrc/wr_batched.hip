@@ -2540,6 +2540,27 @@ hipError_t ragged_f32(const Problem& p, const BatchWs& w, hipStream_t s) {
   return launch_combine_k<OT>(w, p, g.hp, s);
 }
 
+// Whether the many-token kernels are launched: with more than many_avg pairs per
+// expert on average.  With fewer, few experts have more than 64 tokens: two
+// launches that run nothing cost 3.5 us (E 4, 1024 x 4096, k 1, B = 128: 46 -> 49
+// us), and a call with one such expert runs all others in these kernels too, at
+// fewer blocks per CU (fp8) and without the 256-column weight step (MXFP4).
+// Above 32 pairs the 32-token kernels are not launched, so no call makes more
+// than two launches per GEMM.  Clustered calls of Mixtral with more than 64
+// tokens on one expert, 64-token tiles against these, us: fp8 B = 192 (48 per
+// expert) 488 / 519; MXFP4 B = 96 339 / 399, B = 256 547 / 606, B = 320 (80 per
+// expert) 583 / 634.  Over 2600 calls of nine layers (B 72 to 768, even and
+// clustered), those above the bounds take 0.84 (fp16, bf16, fp8) and 0.92 (MXFP4)
+// of the 64-token kernels' time on average, at worst 1.09.
+// They address x's two terms and a pass's act rows with 32-bit offsets.
+template <typename WT>
+bool many_ok(const Problem& p) {
+  constexpr int many_avg = wbits<WT>() == 16 ? 32 : wbits<WT>() == 8 ? 48 : 80;
+  const int64_t lim = int64_t{1} << 32;
+  return p.B > kMaxTok && (int64_t)p.B * p.k > (int64_t)many_avg * p.E &&
+         (int64_t)p.B * p.h * 4 < lim && (int64_t)kPassTok * p.I * 4 < lim;
+}
+
 template <typename WT, typename XT>
 hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
   const GeomB g = make_geom_b(p, sizeof(WT), false);
@@ -2548,11 +2569,7 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
   const WT* wb = static_cast<const WT*>(p.wbuf);
 
   hipError_t err = hipSuccess;
-  // The many-token kernels address x's two terms and a pass's act rows with 32-bit
-  // offsets.
-  const int64_t lim = int64_t{1} << 32;
-  const bool many =
-      p.B > kMaxTok && (int64_t)p.B * p.h * 4 < lim && (int64_t)kPassTok * p.I * 4 < lim;
+  const bool many = many_ok<WT>(p);
   const bool mid = p.B <= WR_MID_TILE_MAX_B;
   // Small batches route inside the gate/up kernel (one launch fewer).  The
   // largest class is that of the kernels launched below, whatever the counts: a
