@@ -97,12 +97,13 @@ def test_ragged_batched_error(cuda, wd, hI):
 
 
 @pytest.mark.parametrize("x_dtype", [F32, F16], ids=["xf32", "xf16"])
-@pytest.mark.parametrize("hI", [(15, 40), (17, 33), (255, 257), (260, 1030), (1031, 261), (2049, 77),
-                                (3001, 1027)], ids=str)
+@pytest.mark.parametrize("hI", [(15, 40), (17, 33), (255, 257), (257, 515), (770, 255), (260, 1030),
+                                (1031, 261), (2049, 77), (77, 2049), (3001, 1027)], ids=str)
 @pytest.mark.parametrize("wd", WTYPES, ids=WIDS)
 def test_ragged_single_token(cuda, wd, hI, x_dtype):
-    """One token: rows shorter than one piece, around half a wave of pieces (the
-    bound between single elements and pieces), and of several rounds."""
+    """One token: rows shorter than one piece, around the bounds between single
+    elements and pieces (half a wave of pieces on average; fp8 a quarter for the
+    shorter row), and of several rounds."""
     E, h, I, k = of_type((6, *hI, 3), wd)
     for seed in range(50):
         x, gw, buf = make_layer(E, h, I, wd, router_std=h ** -0.5, expert_std=0.05, seed=seed,

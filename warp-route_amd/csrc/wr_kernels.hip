@@ -2228,13 +2228,29 @@ hipError_t ffn_t(const Problem& p, const FusedWs& w, bool* fold, hipStream_t s) 
   return per_token_t<WT, XT, VEC, RAG>(p, w, s);
 }
 
-// Rows of whole, aligned 16-byte pieces; else ragged rows (at least one piece
-// long, which MXFP4 rows always are) long enough that half of a wave's lanes
-// have a piece of the average one; shorter ones take one element per lane and
-// access.  Measured, one token, us, one element / ragged pieces: fp16 257 x 259
-// 11.8 / 10.9, 513 x 515 14.7 / 11.5, 1500 x 2050 57.8 / 16.3; fp8 101 x 37 10.7
-// / 14.0, 385 x 387 11.8 / 12.4, 513 x 515 13.9 / 12.4, 1500 x 2050 26.2 / 14.7;
-// fp32 1500 x 2050 24.1 / 22.3.
+// Ragged rows (at least one 16-byte piece long, which MXFP4 rows always are) in
+// unaligned pieces, where half of a wave's lanes have a piece of the average row,
+// or in one element per lane and access.  The latter also, of those:
+//   several tokens of fp8 rows (16 columns per piece, 16 conversions of x) with a
+//   piece for less than a quarter of the lanes: 100 x 1000, E 32, k 1, B = 40 27.5
+//   us / 44.4 in pieces, 3000 x 200 80.8 / 122.4, 513 x 515 0.89 in favour of pieces;
+//   one token whose rows are few rounds of 64 columns either way, a round or two
+//   of latency: E 8, k 2, 255 x 257 fp32 8.6 us / 10.2, fp16 9.2 / 10.6, k 1, 33 x
+//   1023 bf16 9.7 / 12.2; k 6, 255 x 257 fp16 13.7 / 11.2; fp8 k 1, 33 x 1023 9.5 /
+//   14.0, k 2, 250 x 900 12.9 / 11.8, k 6, 33 x 1023 22.6 / 13.7.
+// Long rows, one token, us, one element / pieces: fp16 513 x 515 14.7 / 11.5, 1500
+// x 2050 57.8 / 16.3; fp8 26.2 / 14.7; fp32 24.1 / 22.3.
+template <typename WT>
+bool rag_pieces(const Problem& p) {
+  constexpr int V = wvec_width<WT>();
+  if (p.h < V || p.I < V || (int64_t)p.h + p.I < kWave * V) return false;
+  const bool thin = std::is_same<WT, fp8w>::value && std::min(p.h, p.I) < 16 * V;
+  if (p.B > 1) return !thin;
+  const int64_t down = (int64_t)p.k * ((p.I - 1) / kWave + 1);  // rounds of all experts
+  return thin ? down > 32 : p.h > 5 * kWave || down > 16;
+}
+
+// Rows of whole, aligned 16-byte pieces, or ragged ones.
 template <typename WT, typename XT>
 hipError_t ffn_w(const Problem& p, const FusedWs& w, bool* fold, hipStream_t s) {
   constexpr int V = wvec_width<WT>();
@@ -2242,8 +2258,7 @@ hipError_t ffn_w(const Problem& p, const FusedWs& w, bool* fold, hipStream_t s) 
   if constexpr (std::is_same<WT, fp4x2>::value) {
     return ffn_t<WT, XT, V, true>(p, w, fold, s);
   } else {
-    if (p.h >= V && p.I >= V && p.h + p.I >= kWave * V)
-      return ffn_t<WT, XT, V, true>(p, w, fold, s);
+    if (rag_pieces<WT>(p)) return ffn_t<WT, XT, V, true>(p, w, fold, s);
     return ffn_t<WT, XT, 1, false>(p, w, fold, s);
   }
 }
