@@ -51,8 +51,8 @@ def check(x, gw, buf, E, h, I, k, rn, label):
 
 # h and I: around one 16-byte piece, one below / above whole K steps of 64 and
 # 128, odd, one of the two aligned; then layers large enough for the batched
-# kernels at every B (the small ones take them at the larger B and for the
-# narrower types only).
+# kernels from B = 16 on, and some at B = 2 (the small ones take them at the larger
+# B and for the narrower types only).
 SHAPES = [(8, 32, 96, 2), (5, 127, 129, 2), (20, 72, 40, 6), (8, 264, 520, 2),
           (2, 1151, 1025, 2), (3, 1025, 1151, 3), (2, 2047, 1536, 1), (2, 1536, 1990, 2),
           (12, 500, 1258, 3)]

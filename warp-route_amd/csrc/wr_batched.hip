@@ -56,6 +56,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 #include "wr_device.h"
@@ -2710,17 +2711,20 @@ hipError_t grouped_f32(const Problem& p, const BatchWs& w, hipStream_t s) {
 }  // namespace
 
 // Aligned layers always; ragged ones (rows of at least one 16-byte piece, which
-// MXFP4 rows always are) where tokens share experts and the layer is not tiny.
-// Measured, µs per call, per-token kernels against these:
-//   fewer than 1.5 pairs per expert: E 8, k 2, h 1000, I 1400, B = 4 fp16 22.1
-//   / 34.0, fp8 23.5 / 29.4; E 16, k 4, 1501 x 1003, B = 4 fp16 43.3 / 48.3,
-//   fp32 58.5 / 72.2; with more: B = 8 fp16 33.4 / 34.7 and 69.2 / 53.5, fp8
-//   37.9 / 30.1 and 73.0 / 42.9, fp32 53.3 / 50.9 and 105 / 80.0; B = 32 fp16
-//   72.0 / 39.3 and 211 / 60.6;
-//   few weight bytes over all pairs (four launches and their latency): 264 x
-//   520, fp16 B = 8 (13 MB) 17.9 / 21.7, B = 16 (26 MB) 23.1 / 21.8; fp32 B =
-//   16 (52 MB) 23.8 / 25.5; fp8 B = 8 (7 MB) 21.1 / 20.4; 101 x 37, fp16
-//   B = 32 (1 MB) 16.7 / 21.7.
+// MXFP4 rows always are) where the grouped kernels are faster.  The per-token
+// kernels read the weights of all P pairs (mostly from cache), the grouped ones
+// those of the D distinct experts, after two or three more launches and along a
+// chain of K steps (h / 128 of them) that few rows do not hide: grouped when
+//   P MB + p P > d D MB + q h / 1000 + c,    MB: an expert's weights,
+// D the expected number for even routing, with the constants fitted to both
+// kernels' times over 8015 calls of 31 shapes (101 x 37 to 4100 x 1100), E 2 to
+// 64, B 2 to 128.  Of the faster kernel's time the rule's choice takes 1.005 to
+// 1.009 on average by type (at worst 1.9, small layers), always grouped 1.02 to
+// 1.07 (at worst 3.0).  us per call, per-token / grouped: fp16 1000 x 1400, E 4, k 1,
+// B = 6 20.1 / 29.6; E 8, k 2, B = 8 31.9 / 31.9, B = 32 75.5 / 34.8; fp32 3000 x
+// 200, E 2, k 2, B = 5 24.6 / 74.0; fp8 1501 x 1003, E 8, k 2, B = 8 42.5 / 32.5.  Not measured and not
+// grouped: fewer than 1.5 pairs per expert, or less than `tiny` weight bytes over
+// all pairs.
 bool grouped_ok(const Problem& p) {
   if (p.B <= 1) return false;
   if (aligned_ok(p)) return true;
@@ -2732,7 +2736,18 @@ bool grouped_ok(const Problem& p) {
   if (BatchWs::padded(std::max(p.h, p.I)) > INT32_MAX) return false;  // padded rows are ints
   const int64_t pairs = (int64_t)p.B * p.k;
   const int64_t tiny = (int64_t)(p.wdt == WR_F32 ? 64 : piece == 8 ? 16 : 4) << 20;
-  return 2 * pairs >= 3 * p.E && pairs * p.stride_b > tiny;
+  if (2 * pairs < 3 * p.E || pairs * p.stride_b <= tiny) return false;
+  struct Fit {
+    double p, d, q, c;
+  };
+  const Fit f = p.wdt == WR_F32        ? Fit{0.3, 0.67, 147, 56}
+                : p.wdt == WR_FP8_E4M3 ? Fit{0.03, 0.06, 9.75, 6.7}
+                : p.wdt == WR_MXFP4    ? Fit{0.14, 0.92, 18, 0}
+                : p.vec == 8           ? Fit{0.2, 1.05, 48, 20}
+                                       : Fit{0.8, 0.65, 47, 16};
+  const double mb = (double)p.stride_b * 1e-6;
+  const double distinct = p.E * (1.0 - std::pow(1.0 - (double)p.k / p.E, p.B));
+  return pairs * (mb + f.p) > f.d * distinct * mb + f.q * 1e-3 * p.h + f.c;
 }
 
 // The router launch: with the selection for larger batches (small ones select
