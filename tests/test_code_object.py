@@ -108,6 +108,38 @@ def _waits_before_mfma(insns):
     return bad
 
 
+def _innermost_loops(insns):
+    """Bodies of the loops that hold no other loop: from a backward branch's
+    target to the branch."""
+    idx = {a: i for i, (a, _, _) in enumerate(insns)}
+    spans = set()
+    for b, (addr, op, args) in enumerate(insns):
+        t = idx.get(_branch_target(addr, op, args))
+        if t is not None and t <= b:
+            spans.add((t, b))
+    return [insns[s:e + 1] for s, e in spans
+            if not any(o != (s, e) and s <= o[0] and o[1] <= e for o in spans)]
+
+
+def _awaited_before_mfma(body):
+    """(weight loads of a loop body, how many of them are awaited before the
+    next MFMA, around the loop)."""
+    loads = [i for i, (_, op, args) in enumerate(body)
+             if op.startswith("global_load_dwordx4") and args.endswith(" nt")]
+    bad = 0
+    for i in loads:
+        after = 0
+        for _, op, args in body[i + 1:] + body[:i]:
+            if op.startswith("v_mfma"):
+                break
+            after += bool(re.match(r"(global|buffer)_(load|store|atomic)", op))
+            m = re.search(r"vmcnt\((\d+)\)", args) if op == "s_waitcnt" else None
+            if m and int(m.group(1)) <= after:
+                bad += 1
+                break
+    return len(loads), bad
+
+
 def _tool(name):
     path = os.path.join(LLVM, name)
     if not os.access(path, os.X_OK):
@@ -175,7 +207,8 @@ def batched_isa(kernels, tmp_path_factory):
         for line in text.splitlines():
             m = re.match(r"^[0-9a-f]+ <(\S+)>:$", line)
             if m:
-                name = m.group(1) if re.search(r"k_(gu|dn)_(mfma|f32)", m.group(1)) else None
+                name = m.group(1) if re.search(
+                    r"k_(gu|dn)_(mfma|f32)|k_(rag|many)_(gu|dn)", m.group(1)) else None
                 if name:
                     out[name] = []
                 continue
@@ -186,18 +219,32 @@ def batched_isa(kernels, tmp_path_factory):
 
 
 def test_batched_k_loops_keep_weight_loads_in_flight_over_mfmas(batched_isa):
-    assert len(batched_isa) >= 30, sorted(batched_isa)
+    isa = {n: i for n, i in batched_isa.items() if "k_many" not in n}
+    assert sum("k_rag" in n for n in isa) == 42 and len(isa) >= 72, sorted(isa)
     looped = 0
     bad = {}
-    for name, insns in batched_isa.items():
+    for name, insns in isa.items():
         idx = {a: i for i, (a, _, _) in enumerate(insns)}
         looped += any(op.startswith("global_load_dwordx4") and args.endswith(" nt")
                       and i in _walk(insns, idx, i) for i, (_, op, args) in enumerate(insns))
         b = _waits_before_mfma(insns)
         if b:
             bad[name] = b[:3]
-    assert looped == len(batched_isa), "a kernel's K loop was not found"
+    assert looped == len(isa), "a kernel's K loop was not found"
     assert not bad, f"K-loop weight loads awaited before the MFMAs: {bad}"
+
+
+def test_many_token_k_loops_keep_weight_loads_in_flight_over_mfmas(batched_isa):
+    # k_many_gu / k_many_dn: one K loop per pass size (3, 4 and 5 token tiles per
+    # wave) inside the loop over passes, whose prologue waits for the first weight
+    # step by design, so only the innermost loops are looked at.
+    isa = {n: i for n, i in batched_isa.items() if "k_many" in n}
+    assert len(isa) == 10, sorted(isa)
+    for name, insns in isa.items():
+        loops = [_awaited_before_mfma(b) for b in _innermost_loops(insns)
+                 if any(op.startswith("v_mfma") for _, op, _ in b)]
+        many = [(n, bad) for n, bad in loops if n]
+        assert len(many) == 3 and all(bad == 0 for _, bad in many), (name, loops)
 
 
 def test_no_kernel_uses_scratch_memory_or_spills(kernels):
@@ -224,6 +271,18 @@ def test_single_token_kernels_keep_four_waves_per_simd(kernels):
     assert all(n > 0 for n in fused.values()), "kernel descriptors not found"
     over = {k: n for k, n in fused.items() if n > 128}
     assert not over, f"single-token kernels allocating more than 128 VGPRs: {over}"
+
+
+def test_ragged_single_token_kernels_keep_three_waves_per_simd(kernels):
+    # k_fused_ffn<WT, Ragged<XT>, VEC, ...>: the masks and clamped columns of
+    # ragged pieces cost the 16-bit and MXFP4 kernels the fourth wave; fp32
+    # weights keep it.  2 x types x 2 RPW for four weight types, one RPW for MXFP4.
+    rag = {k: v["vgpr_alloc"] for k, v in kernels.items()
+           if "k_fused_ffn" in k and "RaggedI" in k}
+    assert len(rag) == 18, sorted(rag)
+    assert all(n > 0 for n in rag.values()), "kernel descriptors not found"
+    over = {k: n for k, n in rag.items() if n > (128 if "k_fused_ffnIf" in k else 168)}
+    assert not over, f"ragged single-token kernels over their VGPRs: {over}"
 
 
 # f16 / bf16 single-token kernels with x in LDS and half the column chunks in
@@ -316,3 +375,13 @@ def test_bounded_gateup_tiles_fit_their_blocks_per_cu(kernels):
         for k, v in ks.items():
             assert 0 < v["vgpr_alloc"] <= 512 // blocks // 8 * 8, (k, v["vgpr_alloc"])
             assert blocks * v.get("group_segment_fixed_size", 0) <= 160 * 1024, (k, v)
+
+
+def test_many_token_kernels_fit_two_blocks_per_cu(kernels):
+    # k_many_gu / k_many_dn: 4 waves per block, 2 blocks per CU (512 VGPRs per SIMD
+    # lane, 160 KB of LDS).
+    many = {k: v for k, v in kernels.items() if "k_many_" in k}
+    assert len(many) == 10, sorted(many)
+    for k, v in many.items():
+        assert 0 < v["vgpr_alloc"] <= 256, (k, v["vgpr_alloc"])
+        assert 2 * v.get("group_segment_fixed_size", 0) <= 160 * 1024, (k, v)
