@@ -95,9 +95,9 @@ LOWP = [
     (8, 4096, 1024, 2, FP8, True),    # 4 KB fp8 rows
     (8, 6144, 512, 2, FP8, False),    # fp8 rows longer than 4 KB
     (8, 6144, 512, 2, BF16, False),   # bf16 rows longer than 4 KB: 2 rows per wave
-    (5, 100, 36, 2, BF16, False),     # h % 8 != 0: scalar path
-    (5, 100, 36, 2, FP8, True),       # h % 16 != 0: scalar path
-    (3, 48, 40, 3, FP8, False),       # I % 16 != 0: scalar path, k == E
+    (5, 100, 36, 2, BF16, False),     # h % 8 != 0: short ragged rows
+    (5, 100, 36, 2, FP8, True),       # h % 16 != 0: short ragged rows
+    (3, 48, 40, 3, FP8, False),       # I % 16 != 0: short ragged rows, k == E
     (8, 256, 512, 2, MX4, True),      # MXFP4: blocks of 32 along rows
     (64, 256, 512, 6, MX4, False),
     (16, 512, 1024, 4, MX4, True),
@@ -217,7 +217,7 @@ def test_exact_tie_known_answers(cuda, op):
 
 
 @pytest.mark.parametrize("E", [8, 24], ids=["E8-rows", "E24-wave"])
-@pytest.mark.parametrize("B", [3, 20], ids=["B3-in-kernel-route", "B20-route-kernel"])
+@pytest.mark.parametrize("B", [3, 20], ids=["B3-in-kernel-route", "B20-group-kernel"])
 def test_batched_exact_tie_known_answers(cuda, B, E):
     """The same ties through the grouped batched path (h and I multiples of
     128).  B = 3 routes inside the gate/up kernel, B = 20 in k_group; E = 8

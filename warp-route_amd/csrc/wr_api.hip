@@ -97,8 +97,9 @@ size_t ws_bytes(int kind, int E, int h, int I, int k, int B) {
 
 // Elements per lane per weight access.  The 128-bit path needs every row and
 // every expert block 16-byte aligned (h and I multiples of the vector width,
-// 16-byte aligned weight and activation pointers); anything else takes the
-// scalar path.
+// 16-byte aligned weight and activation pointers); anything else is ragged
+// (vec 1, MXFP4 2): unaligned 16-byte pieces or single elements, as the launchers
+// choose.
 int choose_vec(const wr_moe_args* a) {
   if (a->weight_dtype == WR_MXFP4) {  // h, I multiples of 32: 32 elements per 16 bytes, else 2
     const bool al = reinterpret_cast<uintptr_t>(a->weight_buf) % 16 == 0 &&

@@ -13,17 +13,19 @@
 //      for few tokens (select_in_group).
 //   2. k_group: one block groups the (token, expert) pairs by expert, tokens
 //      ascending, with ballot prefix sums (deterministic, no global atomics);
-//      after k_router_logits it selects first.  For B <= WR_SMALL_TILE_MAX_B there is no such launch: every gate/up block
-//      of step 3 selects (the same wave_select_topk as every other path, so ids
-//      and weights are bit-identical to the single-token op) and groups in LDS
-//      (route_small), and block (0, 0) publishes it.
+//      after k_router_logits it selects first.  For B <= WR_SMALL_TILE_MAX_B
+//      there is no such launch: every gate/up block of step 3 selects (the same
+//      wave_select_topk as every other path, so ids and weights are bit-identical
+//      to the single-token op) and groups in LDS (route_small), and block (0, 0)
+//      publishes it.
 //   3. k_gu_mfma: block (row tile, expert slot): 4 waves x 16 gate rows and
 //      the same 16 up rows each, all of the expert's tokens (up to 64 per
 //      pass); the token tile is staged in LDS and shared by the 4 waves.
 //      Tiles of 16 tokens for B <= 16 and 32 for B <= 32; beyond that the 32-
-//      and 64-token kernels and, for B > 64, the many-token kernels (k_many_gu)
-//      are launched where the pair counts allow them, and one of them runs, as
-//      k_group's largest count says (tile_slot).
+//      and 64-token kernels, or with more pairs per expert the 64-token and the
+//      many-token kernels (k_many_gu, many_ok), are launched where the pair
+//      counts allow them, and one of them runs, as k_group's largest count says
+//      (tile_slot).
 //      v_mfma_f32_16x16x32_f16 with A = weight rows (fp16, or fp8 E4M3 codes
 //      staged as they are and converted exactly to fp16 per fragment) and
 //      B = the hi and lo terms of x; products are exact and accumulate in
@@ -72,8 +74,8 @@ namespace {
 #ifndef WR_MID_TILE_MAX_B
 #define WR_MID_TILE_MAX_B 32    // and up to this size 32-token tiles
 #endif
-// Larger batches launch both the 32- and the 64-token tile kernels (and the
-// many-token ones), and one of them runs (tile_slot): the 32-token one when no
+// Larger batches launch both the 32- and the 64-token tile kernels (or the 64- and
+// many-token ones, many_ok), and one of them runs (tile_slot): the 32-token one when no
 // expert has more than this many pairs, for every expert.  Mixtral, B = 64,
 // per call, in 32-token tiles against 64-token tiles: random routing (26
 // pairs per expert at most) fp16 486 against 527 us, fp8 316 against 346,
@@ -1510,7 +1512,9 @@ __global__ __launch_bounds__(kBlk) void k_act_split(float* __restrict__ act,
 // sub-steps before they are stored.  Experts of at most 64 tokens run gu_pass /
 // dn_pass.
 // ---------------------------------------------------------------------------
-constexpr int kPassTok = 160;  // tokens per pass
+// Tokens per pass: the most whose sums leave two blocks per CU (5 token tiles per
+// wave: 224 to 256 VGPRs, 74 KB of LDS).
+constexpr int kPassTok = 160;
 constexpr int kManyRows = 128;  // weight rows per block: 64 gate and 64 up, or 128 down
 constexpr int kManyP = 4;       // 16-byte pieces per token row and term of a sub-step
 
@@ -1784,8 +1788,9 @@ __device__ __forceinline__ void gu_pass_many(unsigned char* raw,
   }
 }
 
-// grid (I / 64, expert slots).  Two blocks per CU: 256 VGPRs.
-template <typename WT, bool LO, int WK = kBK>
+// grid (I / 64, expert slots).  Two blocks per CU: 256 VGPRs.  (A call's experts of
+// at most 64 tokens take kBK-column weight steps here, MXFP4 too.)
+template <typename WT, bool LO>
 __global__ __launch_bounds__(kBlk, 2) void k_many_gu(
     const WT* __restrict__ wbuf, const f16* __restrict__ x_hi, const f16* __restrict__ x_lo,
     const int32_t* __restrict__ x_exp, unsigned* __restrict__ amax, BatchRoute r,
@@ -1810,24 +1815,24 @@ __global__ __launch_bounds__(kBlk, 2) void k_many_gu(
   const int wrow = row0 + wave * 16;  // this wave's staged rows (gate; the same up rows)
   if (M <= kMaxTok) {
     const int lane = lane0;
-    const WT* G = w_lane_base<WT, WK>(blk, wrow, g.h, lane);
-    constexpr int N = WRegs<WT, 32, WK>::N, RP = WGeo<WT, WK>::kRowsPer;
+    const WT* G = w_lane_base<WT, kBK>(blk, wrow, g.h, lane);
+    constexpr int N = WRegs<WT, 32, kBK>::N, RP = WGeo<WT, kBK>::kRowsPer;
     const WT* wbase[N];
     const uint8_t* wsc[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) {  // as in gu_block
       wbase[i] = G + (i < N / 2 ? 0 : g.off_up) + eoff<WT>((int64_t)(RP * (i % (N / 2))) * g.h);
-      wsc[i] = w_lane_scale<WT, WK>(mxs + (i < N / 2 ? 0 : (int64_t)g.I * g.h / 32), wrow, g.h,
+      wsc[i] = w_lane_scale<WT, kBK>(mxs + (i < N / 2 ? 0 : (int64_t)g.I * g.h / 32), wrow, g.h,
                                     lane) +
                (int64_t)(RP * (i % (N / 2))) * (g.h / 32);
     }
     auto& xs = *reinterpret_cast<TokTile<kMaxTok, kBK>*>(raw);
-    auto& wt = reinterpret_cast<WTile<WT, 32, WK>*>(raw + sizeof(xs))[wave];
+    auto& wt = reinterpret_cast<WTile<WT, 32, kBK>*>(raw + sizeof(xs))[wave];
     switch ((M + 15) / 16) {
-      case 1: gu_pass<WT, LO, 1, kMaxTok, kBK, WK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
-      case 2: gu_pass<WT, LO, 2, kMaxTok, kBK, WK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
-      case 3: gu_pass<WT, LO, 3, kMaxTok, kBK, WK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
-      default: gu_pass<WT, LO, 4, kMaxTok, kBK, WK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
+      case 1: gu_pass<WT, LO, 1, kMaxTok, kBK, kBK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
+      case 2: gu_pass<WT, LO, 2, kMaxTok, kBK, kBK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
+      case 3: gu_pass<WT, LO, 3, kMaxTok, kBK, kBK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
+      default: gu_pass<WT, LO, 4, kMaxTok, kBK, kBK>(xs, wt, wbase, wsc, x_hi, x_lo, nullptr, r, pbeg, M, act, wrow, sc, xsc, g, lane); break;
     }
     return;
   }
@@ -1892,9 +1897,9 @@ __device__ __forceinline__ void dn_pass_many(unsigned char* raw,
   }
 }
 
-// grid (h / 128, kKSplit, expert slots), act split ahead; K slices of whole WK
+// grid (h / 128, kKSplit, expert slots), act split ahead; K slices of whole kBK
 // steps, as k_dn_mfma's.
-template <typename WT, int WK = kBK>
+template <typename WT>
 __global__ __launch_bounds__(kBlk, 2) void k_many_dn(const WT* __restrict__ wbuf, BatchRoute r,
                                                      const float* __restrict__ act,
                                                      const unsigned* __restrict__ amax,
@@ -1909,9 +1914,9 @@ __global__ __launch_bounds__(kBlk, 2) void k_many_dn(const WT* __restrict__ wbuf
   int bx = blockIdx.x, ks = blockIdx.y;
   dn_relabel(bx, ks);
   const int row0 = bx * kManyRows;
-  const int nsteps = g.I / WK;
-  const int kb = nsteps * ks / BatchWs::kKSplit * WK;
-  const int ke = nsteps * (ks + 1) / BatchWs::kKSplit * WK;
+  const int nsteps = g.I / kBK;
+  const int kb = nsteps * ks / BatchWs::kKSplit * kBK;
+  const int ke = nsteps * (ks + 1) / BatchWs::kKSplit * kBK;
   const WT* blk = wbuf + (int64_t)e * g.stride;
   const float* sdown = nullptr;
   if constexpr (std::is_same<WT, fp8w>::value) sdown = wscales(blk, g.off_scale) + 2 * g.I;
@@ -1921,25 +1926,25 @@ __global__ __launch_bounds__(kBlk, 2) void k_many_dn(const WT* __restrict__ wbuf
   if (M <= kMaxTok) {  // the block's rows in two halves of 4 x 16
     const int lane = lane0;
     auto& xs = *reinterpret_cast<TokTile<kMaxTok, kBK>*>(raw);
-    auto& wt = reinterpret_cast<WTile<WT, 16, WK>*>(raw + sizeof(xs))[wave];
-    constexpr int N = WRegs<WT, 16, WK>::N;
+    auto& wt = reinterpret_cast<WTile<WT, 16, kBK>*>(raw + sizeof(xs))[wave];
+    constexpr int N = WRegs<WT, 16, kBK>::N;
     for (int half = 0; half < 2; ++half) {
       const int wrow = row0 + half * kBM + wave * 16;
-      const WT* D = w_lane_base<WT, WK>(blk + g.off_down, wrow, g.I, lane);
+      const WT* D = w_lane_base<WT, kBK>(blk + g.off_down, wrow, g.I, lane);
       const WT* wbase[N];
       const uint8_t* wsc[N];
 #pragma unroll
       for (int i = 0; i < N; ++i) {  // as in dn_block
-        wbase[i] = D + eoff<WT>((int64_t)(WGeo<WT, WK>::kRowsPer * i) * g.I);
-        wsc[i] = w_lane_scale<WT, WK>(mxs, wrow, g.I, lane) +
-                 (int64_t)(WGeo<WT, WK>::kRowsPer * i) * (g.I / 32);
+        wbase[i] = D + eoff<WT>((int64_t)(WGeo<WT, kBK>::kRowsPer * i) * g.I);
+        wsc[i] = w_lane_scale<WT, kBK>(mxs, wrow, g.I, lane) +
+                 (int64_t)(WGeo<WT, kBK>::kRowsPer * i) * (g.I / 32);
       }
       const int sb = kb / kBK, se = ke / kBK;
       switch ((M + 15) / 16) {
-        case 1: dn_pass<WT, 1, kMaxTok, kBK, true, WK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
-        case 2: dn_pass<WT, 2, kMaxTok, kBK, true, WK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
-        case 3: dn_pass<WT, 3, kMaxTok, kBK, true, WK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
-        default: dn_pass<WT, 4, kMaxTok, kBK, true, WK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
+        case 1: dn_pass<WT, 1, kMaxTok, kBK, true, kBK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
+        case 2: dn_pass<WT, 2, kMaxTok, kBK, true, kBK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
+        case 3: dn_pass<WT, 3, kMaxTok, kBK, true, kBK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
+        default: dn_pass<WT, 4, kMaxTok, kBK, true, kBK>(xs, wt, wbase, wsc, act, amax, pbeg, M, sb, se, y, wrow, sdown, g, lane); break;
       }
     }
     return;
@@ -2488,7 +2493,10 @@ bool aligned_ok(const Problem& p) {
 
 // Token tile of a ragged layer: 16 and 32 as the aligned layers', then 64
 // when the average expert gets more than 24 tokens (an expert with more
-// than the tile takes several passes).
+// than the tile takes several passes).  Time in 64-token tiles over that in
+// 32-token ones, mean of four shapes (520 x 1190 to 2880 x 2880): at 18 to 25
+// tokens per expert fp32 1.02, fp16 1.24, bf16 1.08, fp8 1.14, MXFP4 1.17 (fewer:
+// up to 1.45), at 30 to 36 0.85, 0.92, 0.83, 0.89, 0.91.
 int rag_tile(const Problem& p) {
   if (p.B <= WR_SMALL_TILE_MAX_B) return 16;
   return p.B <= WR_MID_TILE_MAX_B || p.B * p.k <= 24 * p.E ? 32 : 64;
@@ -2621,7 +2629,7 @@ hipError_t grouped_t(const Problem& p, const BatchWs& w, hipStream_t s) {
     // B = 24 / 32: 115.1 / 119.6 -> 102.8 / 103.5 us per call (gate/up 176
     // VGPRs, 2 blocks per CU; a 3-block bound, 144 VGPRs, measured slower).
     constexpr int KM = (WR_MID_WIDE && std::is_same<WT, fp4x2>::value) ? kc_wide<WT>() : kBK;
-    // The weight step of 64-token and many-token tiles.
+    // The weight steps of 64-token tiles.
     constexpr int KG = (WR_W2 && std::is_same<WT, fp4x2>::value) ? kc_wide<WT>() : kBK;
     constexpr int KD = (WR_W2DN && std::is_same<WT, fp4x2>::value) ? kc_wide<WT>() : kBK;
     if (run32) {

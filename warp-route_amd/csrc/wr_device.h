@@ -371,7 +371,7 @@ __device__ __forceinline__ int topk_id_lanes(const TopK& t, int kk) {
 
 // ---------------------------------------------------------------------------
 // Vector loads.  VEC elements per lane: 16 x fp8, 8 x fp16 / bf16 or 4 x fp32
-// is one 128-bit access; VEC = 1 is the scalar path for unaligned shapes.
+// is one 128-bit access, at any address with load_wq_u; VEC = 1 is one element.
 // ---------------------------------------------------------------------------
 template <typename T, int VEC>
 struct WVec;

@@ -2122,10 +2122,11 @@ hipError_t fused_rpw_t(const Problem& p, const FusedWs& w, bool* fold, hipStream
       // -> 26.37 would lose.  It also pays for layers of at most one block per
       // CU, where no poll shares a CU with a router row or delays a weight
       // load: fp32, E 8, h 256, I 512, k 2 (192 blocks) 8.84 -> 7.66 us.
-      // Layers between the two keep the router launch, which loses at 1.5
-      // blocks per CU (fp32 1024 x 1024, k 1: 10.7 / 9.9 folded) and wins
-      // beyond (fp16 6144 x 1024, k 2: 24.8 / 25.7 folded; fp32 E 64, 2048 x
-      // 352, k 6: 18.7 / 19.1).
+      // Layers between the two keep the router launch, which wins from 2 blocks
+      // per CU on (fp16 6144 x 1024, k 2: 24.8 / 25.7 folded; fp32 E 64, 2048 x
+      // 352, k 6: 18.7 / 19.1).  It loses at 1.5 (fp32 1024 x 1024, k 1: 10.7 /
+      // 9.9), but there blocks do share CUs and no other shape was measured, so
+      // the line stays where the reason does.
       *fold = hs.n1 >= kFoldSlotsPerCu * cu_count() || hs.nb <= cu_count();
       if (!*fold) return hipSuccess;
       hipLaunchKernelGGL((k_fused_ffn<WT, XT, VEC, RPW, U1, RPD, U2, false, false, false, true>),
